@@ -8,16 +8,25 @@
 //   adc(code)   = four accumulators over j mod 4           pq.h:36-46
 //   depth       = rerank < 0 ? max(10 k, 100) : rerank     RerankDepth, ivf_pq.cc:16-19
 //   distance_computations = rows (+ the candidates reranked)
-// The tables are built on the device ([nq][m x 256] floats), the scan is the exact-score
-// scan of the flat path with the ADC as its score (row splits with a wave top-k each, then
-// a merge; a segmented sort beyond 240), the rerank the flat path's k_rerank.
+// The tables are built on the device ([nq][m x 256] floats).  Up to 240 results of at least
+// 1,024 rows, where the padded dim has a GEMM kernel, the scan is the flat path's ranking
+// GEMM over the rows the codes decode to (fp16 halves, gemm16.hip SPLIT 3: the ADC is the
+// distance to the decoded row up to its rounding, which the query's bound takes in); every
+// candidate it admits is then scored by ADC from the query's table, certified against the
+// admission threshold, and re-scanned code by code when that fails.  Otherwise every code is
+// scored (row splits with a wave top-k each, then a merge; a segmented sort beyond 240).
 //
-// Bound: HBM.  Each query streams the n x m code bytes (plus its 16 KB table, L2-resident).
+// Bound: MFMA (2 n pd flop per query; 890 TFLOP/s at 1M x 128, 2,000 queries).  Scoring every
+// code is bound by its m table reads a row instead: the batch of 2,000 queries over 1M codes
+// of 16 bytes took 26.1 ms that way and takes 0.74 ms ranked (the GEMM 0.57).  The decoded
+// rows cost 2 pd + 4 bytes a row of device memory.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <string>
 #include <vector>
 
+#include "gemm.h"
 #include "vdbg_device.h"
 #include "vdbg_internal.h"
 
@@ -25,6 +34,9 @@ namespace vdbg {
 namespace {
 
 constexpr int kKsub = 256;
+// the ranking GEMM path's limits (RunScan): results per query and rows
+constexpr size_t kRankK = 240;
+constexpr size_t kRankRows = 1024;
 
 // compute_table (pq.cc:63-73) for nq queries: one thread per (query, subspace, centroid).
 __global__ void k_pq_tables(const float* __restrict__ Q, int pd, int nq,
@@ -39,6 +51,42 @@ __global__ void k_pq_tables(const float* __restrict__ Q, int pd, int nq,
   const float* qs = Q + q * pd + size_t(j) * dsub;
   const float* cc = cen + size_t(e) * dsub;
   T[t] = l2 ? l2sq_any(qs, cc, dsub) : -dot_any(qs, cc, dsub);
+}
+
+// The rows the codes decode to, for the ranking GEMM (gemm16.hip SPLIT 3): fp16(v 2^e) of
+// each decoded value, zero in the padding, the row's fp32 norm and the largest norm (float
+// bits).  One wave per row; writes 2 pd bytes a row, once per index.
+__global__ __launch_bounds__(256) void k_pq_decode16(const uint8_t* __restrict__ codes,
+                                                     const float* __restrict__ cen, uint32_t n,
+                                                     int m, int dsub, int pd, int e,
+                                                     uint16_t* __restrict__ y,
+                                                     float* __restrict__ norm,
+                                                     uint32_t* __restrict__ max_norm) {
+  __shared__ float s_max[4];
+  const int wave = threadIdx.x >> 6, lane = lane_id();
+  const size_t r = size_t(blockIdx.x) * 4 + wave;
+  float sum = 0.f;
+  if (r < n) {
+    for (int i = lane; i < pd; i += kWave) {
+      float v = 0.f;
+      if (i < m * dsub) {
+        const int j = i / dsub;
+        v = cen[(size_t(j) * kKsub + codes[r * m + j]) * dsub + (i - j * dsub)];
+      }
+      y[r * pd + i] = __builtin_bit_cast(uint16_t, _Float16(ldexpf(v, e)));
+      sum = fmaf(v, v, sum);
+    }
+  }
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+  if (lane == 0) {
+    if (r < n) norm[r] = sum;
+    s_max[wave] = r < n ? sum : 0.f;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    atomicMax(max_norm, __float_as_uint(fmaxf(fmaxf(s_max[0], s_max[1]),
+                                              fmaxf(s_max[2], s_max[3]))));
 }
 
 // distance_computations of PqFlatIndex::search: every row, plus the candidates handed to
@@ -91,19 +139,30 @@ int PqFlatSearch(PqFlatIndex* x, const float* Q, size_t nq, size_t k, int rerank
         static_cast<float*>(tables.p));
     VDBG_HIP(hipGetLastError());
   }
+  const float* T = static_cast<const float*>(tables.p);
   ScanSource src;
   src.kind = 2;
   src.C = x->codes;
   src.pq_m = x->m;
   src.N = uint32_t(n);
-  src.pd = int(ts);
+  src.pd = int(ds->pd);
   src.metric = ds->metric;
-  const float* T = static_cast<const float*>(tables.p);
+  // the kk best by (ADC, id): the ranking GEMM over the decoded rows and the ADC of the few
+  // codes it admits, or the ADC of every code
+  auto scan = [&](size_t kk, uint32_t* ids, float* d) {
+    if (x->src.X16 != nullptr && x->src.N == n && c->fp16_gemm && kk <= kRankK) {
+      VDBG_RETURN_IF_ERROR(BuildSample(c, &x->src, s));
+      ScanSource ranked = x->src;
+      ranked.pq_tables = T;
+      return RunScan(c, &ranked, Q, nq, kk, allow, ids, d, s);
+    }
+    return ScoreScan(c, src, T, nq, kk, allow, ids, d, s);
+  };
   // the scan keeps at most n candidates, as a TopK of any capacity over n rows does (depth
   // may exceed vdb's largest k: max(10 k, 100) at k = 10,000)
   const size_t keep = std::min(kk, std::max<size_t>(n, k));
   if (depth == 0) {
-    VDBG_RETURN_IF_ERROR(ScoreScan(c, src, T, nq, k, allow, out_ids, out_d, s));
+    VDBG_RETURN_IF_ERROR(scan(k, out_ids, out_d));
     if (dc != nullptr)
       k_pqflat_dc<<<dim3(unsigned((nq + 255) / 256)), 256, 0, s>>>(out_ids, int(k), int(nq), n, 0,
                                                                    dc);
@@ -115,7 +174,7 @@ int PqFlatSearch(PqFlatIndex* x, const float* Q, size_t nq, size_t k, int rerank
   VDBG_HIP(hipMallocAsync(&ci.p, nq * keep * 4, s));
   VDBG_HIP(hipMallocAsync(&cd.p, nq * keep * 4, s));
   uint32_t* cand = static_cast<uint32_t*>(ci.p);
-  VDBG_RETURN_IF_ERROR(ScoreScan(c, src, T, nq, keep, allow, cand, static_cast<float*>(cd.p), s));
+  VDBG_RETURN_IF_ERROR(scan(keep, cand, static_cast<float*>(cd.p)));
   VDBG_RETURN_IF_ERROR(Rerank(c, ds->rows, int(ds->pd), ds->metric, Q, nq, cand, keep, k, out_ids,
                               out_d, s, &ds->src));
   if (dc != nullptr)
@@ -126,10 +185,85 @@ int PqFlatSearch(PqFlatIndex* x, const float* Q, size_t nq, size_t k, int rerank
 }
 
 void FreePqFlat(PqFlatIndex* x) {
+  FreeSample(&x->src);
+  x->src = ScanSource{};
+  (void)hipFree(x->dec16);
+  (void)hipFree(x->dec_norm);
+  x->dec16 = nullptr;
+  x->dec_norm = nullptr;
   (void)hipFree(x->cen);
   (void)hipFree(x->codes);
   x->cen = nullptr;
   x->codes = nullptr;
+}
+
+// Makes the decoded rows the ranking GEMM reads (the codes are in place).  Without them, for
+// padded dims with no GEMM kernel, segments below the GEMM path's 1,024 rows, non-finite
+// codebooks or when memory is short, searches score every code.
+int MakeDecoded(Ctx* c, PqFlatIndex* x, hipStream_t s) {
+  const size_t n = x->ds->n, pd = x->ds->pd;
+  if (n < kRankRows || !GemmSupported(pd)) return kOk;
+  float ma = 0.f;
+  for (const float v : x->cen_h) {
+    if (!(std::fabs(v) <= 3.0e38f)) return kOk;
+    ma = std::max(ma, std::fabs(v));
+  }
+  int e = 0;  // the largest magnitude in [2^14, 2^15)
+  if (ma > 0.f) {
+    int ex = 0;
+    (void)std::frexp(ma, &ex);
+    e = 15 - ex;
+  }
+  uint32_t* max_norm = nullptr;
+  const bool got =
+      hipMalloc(reinterpret_cast<void**>(&x->dec16), n * pd * sizeof(uint16_t)) == hipSuccess &&
+      hipMalloc(reinterpret_cast<void**>(&x->dec_norm), n * sizeof(float)) == hipSuccess &&
+      hipMalloc(reinterpret_cast<void**>(&max_norm), 256) == hipSuccess;
+  auto drop = [&]() {
+    (void)hipFree(x->dec16);
+    (void)hipFree(x->dec_norm);
+    (void)hipFree(max_norm);
+    x->dec16 = nullptr;
+    x->dec_norm = nullptr;
+  };
+  if (!got) {
+    (void)hipGetLastError();
+    drop();
+    return kOk;
+  }
+  uint32_t bits = 0;
+  int rc = Fill32(max_norm, 0, 1, s);
+  if (rc == kOk) {
+    k_pq_decode16<<<dim3(unsigned((n + 3) / 4)), 256, 0, s>>>(x->codes, x->cen, uint32_t(n), x->m,
+                                                               x->dsub, int(pd), e, x->dec16,
+                                                               x->dec_norm, max_norm);
+    if (hipGetLastError() != hipSuccess) rc = SetError(kInternal, "pq decode");
+  }
+  if (rc == kOk) rc = ReadWords(c, max_norm, 1, s, &bits);
+  float xn = 0.f;
+  std::memcpy(&xn, &bits, 4);
+  if (rc != kOk || !(xn <= 3.0e38f)) {
+    (void)hipStreamSynchronize(s);
+    drop();
+    return rc;
+  }
+  (void)hipFree(max_norm);
+  ScanSource& src = x->src;
+  src.kind = 2;
+  src.C = x->codes;
+  src.pq_m = x->m;
+  src.X16 = x->dec16;
+  src.x16_exp = e;
+  src.x16_approx = 1;
+  src.rn = x->dec_norm;
+  src.N = uint32_t(n);
+  src.pd = int(pd);
+  src.metric = x->ds->metric;
+  src.stats.max_abs = ma;
+  src.stats.xn_max = xn;
+  src.stats.all_int = 0;  // the ranking is never exact: ADC sums in its own order
+  src.rmag = xn;
+  return kOk;
 }
 
 // Uploads the codebook (and codes, when given on the host) of an index over ds.
@@ -191,6 +325,8 @@ int vdbg_pqflat_build(vdbg_dataset* ds, size_t pq_m, uint64_t seed,
                   x.dsub, x.codes, s);
     if (rc != kOk) return fail(rc);
     if (hipStreamSynchronize(s) != hipSuccess) return fail(SetError(kInternal, "pq encode"));
+    rc = MakeDecoded(c, &x, s);
+    if (rc != kOk) return fail(rc);
   }
   ++d.live_indexes;
   *out = h;
@@ -242,7 +378,8 @@ int vdbg_pqflat_load(vdbg_dataset* ds, const void* file, size_t len, vdbg_pqflat
   x.dsub = int(dsub);
   x.cen_h = std::move(cen);
   x.trained = true;
-  const int rc = InstallPqFlat(c, &x, codes, c->stream);
+  int rc = InstallPqFlat(c, &x, codes, c->stream);
+  if (rc == kOk) rc = MakeDecoded(c, &x, c->stream);
   if (rc != kOk) {
     FreePqFlat(&x);
     delete h;

@@ -652,6 +652,7 @@ struct PrepArgs {
   int c8;
   uint32_t* mb8;  // nullable: SQ8 on the int8 GEMM, the batch's max |B| (float bits, atomicMax)
   int single16;   // float rows held as their scaled h halves alone (gemm16.hip SPLIT 3)
+  int adc;        // the exact score is the ADC of a code whose decoded row the GEMM ranks
 };
 
 // One wave per query.
@@ -832,7 +833,14 @@ __device__ uint32_t query_prep_wave(const PrepArgs& a, int q) {
         bound16f + (a.metric != 0 ? drop * sqrt(double(qmag) * double(a.rmag))
                                   : drop * (double(qmag) + double(a.rmag)));
     const bool split = a.Q16 != nullptr && (a.kind == 1 || a.x16_parts == 2 || a.single16);
-    const double bsplit = a.kind == 1 ? bound16 : (a.single16 ? bound16h : bound16f);
+    double bsplit = a.kind == 1 ? bound16 : (a.single16 ? bound16h : bound16f);
+    // ADC of a code: table entries over dsub dims (each off by at most (dsub + 6) u of itself;
+    // inner product: of its sum |q_i x_i|), m of them added, so at most (pd + 16) u of the
+    // whole, which is at most 2 (|q|^2 + |x|^2) (L2) or |q||x|; doubled for margin.
+    if (a.adc)
+      bsplit += (4.0 * pd + 64.0) * u *
+                (a.metric != 0 ? sqrt(double(qmag) * double(a.rmag))
+                               : double(qmag) + double(a.rmag));
     a.exact[q] = ex && !half_norm ? 1 : 0;
     a.eb[q] = half_norm ? 1.f : ex ? 0.f : float((split ? bsplit : bound) * 1.001);
   }
@@ -1976,7 +1984,8 @@ static int ExactScanT(Ctx* c, Workspace& w, const ScanSource& src, const Scorer&
   VDBG_RETURN_IF_ERROR(w.reserve(need));
   uint2* part = w.take<uint2>(size_t(nslots) * nsplit * cap);
   uint32_t* pc = w.take<uint32_t>(size_t(nslots) * nsplit);
-  ScanArgs sa{Q, allow, src.pd, N, qlist, nslots, split_rows, nsplit, part, pc, nslots_dev};
+  const int spd = ScorePd(src);
+  ScanArgs sa{Q, allow, spd, N, qlist, nslots, split_rows, nsplit, part, pc, nslots_dev};
   {
     ProfScope ps(c, "exact_scan", s);
     VDBG_DISPATCH_ES(E, launch_scan, Scorer, s, sa, sc);
@@ -1991,7 +2000,7 @@ static int ExactScanT(Ctx* c, Workspace& w, const ScanSource& src, const Scorer&
   se.qlist = qlist;
   se.nslots = nslots;
   se.k = int(k);
-  se.pd = src.pd;
+  se.pd = spd;
   se.rescore = 0;
   se.out_ids = out_ids;
   se.out_d = out_d;
@@ -2997,6 +3006,9 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
   // rows wider than one K chunk keep each wave's query fragments resident (one 32-query
   // block per wave, gemm16.hip QRES); the sample pass keeps two blocks per wave
   const bool wide16 = single && Gemm16ResQueries(pd);
+  // PQ codes rank on the rows they decode to and are scored by ADC from the batch's tables
+  const bool adc = src->kind == 2;
+  const float* SQ = adc ? src->pq_tables : Q;  // what the exact scorer reads per query
   const bool try8f = c->fp16_gemm && c->int8_gemm && split == 2 &&
                      src->X8 != nullptr && src->x8_parts == 2 && Gemm8Supported(pd) &&
                      double(N) * double(nq) * double(pd) >= c->int8_float_min_work;
@@ -3133,10 +3145,10 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
     VDBG_HIP(hipGetLastError());
   }
 
-  PrepArgs pa{Q, Qb, int(nq), int(pd), src->kind, src->metric, src->stats, src->rmag,
+  PrepArgs pa{Q, Qb, int(nq), int(pd), adc ? 0 : src->kind, src->metric, src->stats, src->rmag,
               src->vmin, src->scale, shift, eb, exact, Q16, all16, Qf, src->x16_parts,
               src->x16_exp, try8 ? Q8 : nullptr, try8 ? Qd : nullptr, try8 ? all8 : nullptr,
-              fit8q, src->c8, mb8, single ? 1 : 0};
+              fit8q, src->c8, mb8, single ? 1 : 0, adc ? 1 : 0};
   {
     ProfScope ps(c, "query_prep", s);
     k_query_prep<<<dim3(unsigned((nq + 3) / 4)), 256, 0, s>>>(pa);
@@ -3163,8 +3175,8 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
     use16 = try16 && !use8 && (split != 0 || fl[0] != 0);
   }
   // a source reading its parent's rows through Xmap ranks on its fp16 copy (no fp32 GEMM)
-  if (src->Xmap != nullptr && !use8 && !use16)
-    return SetError(kInternal, "scan: remapped fp32 rows on the fp32 GEMM");
+  if ((src->Xmap != nullptr || adc) && !use8 && !use16)
+    return SetError(kInternal, "scan: remapped fp32 rows or PQ codes on the fp32 GEMM");
   // the bound of the GEMM the batch ranks on
   const float* ebx = use8 && try8op ? eb8 : eb;
   c->last_gemm_bits = use8 ? 8 : (use16 ? 16 : 32);
@@ -3262,7 +3274,7 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
   int blocks = 0;
   GemmGrid(ga, P.nqt, nchunks, &blocks);
   {
-    ProfScope ps(c, src->kind == 0 ? "flat_gemm" : "sq8_gemm", s);
+    ProfScope ps(c, src->kind == 0 ? "flat_gemm" : (adc ? "pq_gemm" : "sq8_gemm"), s);
     if (gated) {
       // the int8 pass when every query fits it, else the fp32 pass (one grid, one plan)
       GemmArgs g8 = ga;
@@ -3303,7 +3315,7 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
     VDBG_HIP(hipGetLastError());
   }
   SelectArgs se{};
-  se.Q = Q;
+  se.Q = SQ;
   se.cand = cand;
   se.counts = counts;
   se.nseg = nseg;
@@ -3314,85 +3326,69 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
   se.exact = exact;
   se.nslots = int(nq);
   se.k = int(kk);
-  se.pd = int(pd);
-  se.rescore = 1;
+  se.pd = ScorePd(*src);
+  // ADC scores are a few table reads each and sit closer together than the bound of the
+  // fp16 ranking (about 370 distance units against gaps of under 10 at depth 100 on 1M
+  // SIFT-like rows), so every buffered candidate of a PQ scan is scored at once.
+  se.rescore = adc ? 2 : 1;
   se.T = T;
   se.out_ids = out_ids;
   se.out_d = out_d;
   se.fb_list = fb_list;
   se.fb_count = fb_count;
   se.force_fallback = c->test_fallbacks;
-  {
-    ProfScope ps(c, "select", s);
-    if (UseFlat8(*src, nq, kk, 1)) {
-      VDBG_DISPATCH_ES(Esel, launch_select, FlatScorer8, s, se, Flat8Of(*src, c->kset));
+  auto select = [&](const SelectArgs& a, const char* name) -> int {
+    ProfScope ps(c, name, s);
+    if (adc) {
+      VDBG_DISPATCH_ES(Esel, launch_select, PqScorer, s, a, PqScorer{src->C, src->pq_m});
+    } else if (UseFlat8(*src, nq, kk, a.rescore)) {
+      VDBG_DISPATCH_ES(Esel, launch_select, FlatScorer8, s, a, Flat8Of(*src, c->kset));
     } else if (src->kind == 0) {
-      VDBG_DISPATCH_ES(Esel, launch_select, FlatScorer, s, se, FlatOf(*src, c->kset));
+      VDBG_DISPATCH_ES(Esel, launch_select, FlatScorer, s, a, FlatOf(*src, c->kset));
     } else {
-      VDBG_DISPATCH_ES(Esel, launch_select, Sq8Scorer, s, se, Sq8Of(*src, c->kset));
+      VDBG_DISPATCH_ES(Esel, launch_select, Sq8Scorer, s, a, Sq8Of(*src, c->kset));
     }
     VDBG_HIP(hipGetLastError());
+    return kOk;
+  };
+  VDBG_RETURN_IF_ERROR(select(se, "select"));
+  // Uncertified queries take a second chance (every buffered candidate re-scored; the first
+  // pass has done that already for PQ codes) and, if it fails too, the exact re-scan.  When
+  // the re-scan's scratch for every query of the batch is small, both passes are queued for
+  // every slot and run only for the slots the pass before listed (its count stays on the
+  // device): nothing waits on the host.  Otherwise the host reads each count and sizes the
+  // pass to it.
+  const bool second = !adc;
+  const bool gate_fb = c->gate_fallbacks && PlanExact(N, int(nq), kk).need <= kGatedExactBytes;
+  uint32_t nfb = 0;
+  if (!gate_fb) {
+    VDBG_RETURN_IF_ERROR(ReadWords(c, fb_count, 1, s, &nfb));
+    if (nfb == 0) return kOk;
   }
-  // Uncertified queries take a second chance (every buffered candidate re-scored) and, if it
-  // fails too, the exact re-scan.  When the re-scan's scratch for every query of the batch is
-  // small, both passes are queued for every slot and run only for the slots the pass before
-  // listed (its count stays on the device): nothing waits on the host.  Otherwise the host
-  // reads each count and sizes the pass to it.
-  if (c->gate_fallbacks && PlanExact(N, int(nq), kk).need <= kGatedExactBytes) {
+  if (second) {
     SelectArgs s2 = se;
     s2.qlist = fb_list;
-    s2.nslots = int(nq);
-    s2.nslots_dev = fb_count;
+    s2.nslots = gate_fb ? int(nq) : int(nfb);
+    s2.nslots_dev = gate_fb ? fb_count : nullptr;
     s2.by_query = 1;
     s2.rescore = 2;
-    s2.T = T;
     s2.fb_list = fb2_list;
     s2.fb_count = fb_count + 1;
-    {
-      ProfScope ps(c, "rescore", s);
-      if (UseFlat8(*src, nq, kk, 2)) {
-        VDBG_DISPATCH_ES(Esel, launch_select, FlatScorer8, s, s2, Flat8Of(*src, c->kset));
-      } else if (src->kind == 0) {
-        VDBG_DISPATCH_ES(Esel, launch_select, FlatScorer, s, s2, FlatOf(*src, c->kset));
-      } else {
-        VDBG_DISPATCH_ES(Esel, launch_select, Sq8Scorer, s, s2, Sq8Of(*src, c->kset));
-      }
-      VDBG_HIP(hipGetLastError());
-    }
-    VDBG_RETURN_IF_ERROR(ExactScan(c, W2, *src, Q, fb2_list, int(nq), kk, allow, out_ids, out_d,
-                                   s, fb_count + 1, c->fb_dev));
+    VDBG_RETURN_IF_ERROR(select(s2, "rescore"));
+  }
+  const uint32_t* list = second ? fb2_list : fb_list;
+  const uint32_t* count = second ? fb_count + 1 : fb_count;
+  if (gate_fb) {
+    VDBG_RETURN_IF_ERROR(ExactScan(c, W2, *src, SQ, list, int(nq), kk, allow, out_ids, out_d, s,
+                                   count, c->fb_dev));
     c->fb_dev_used = true;
     return kOk;
   }
-  uint32_t nfb = 0;
-  VDBG_RETURN_IF_ERROR(ReadWords(c, fb_count, 1, s, &nfb));
-  if (nfb == 0) return kOk;
-  // second chance: rescore every buffered candidate of the uncertified queries
-  SelectArgs s2 = se;
-  s2.qlist = fb_list;
-  s2.nslots = int(nfb);
-  s2.by_query = 1;
-  s2.rescore = 2;
-  s2.T = T;
-  s2.fb_list = fb2_list;
-  s2.fb_count = fb_count + 1;
-  {
-    ProfScope ps(c, "rescore", s);
-    if (UseFlat8(*src, nq, kk, 2)) {
-      VDBG_DISPATCH_ES(Esel, launch_select, FlatScorer8, s, s2, Flat8Of(*src, c->kset));
-    } else if (src->kind == 0) {
-      VDBG_DISPATCH_ES(Esel, launch_select, FlatScorer, s, s2, FlatOf(*src, c->kset));
-    } else {
-      VDBG_DISPATCH_ES(Esel, launch_select, Sq8Scorer, s, s2, Sq8Of(*src, c->kset));
-    }
-    VDBG_HIP(hipGetLastError());
-  }
-  uint32_t nfb2 = 0;
-  VDBG_RETURN_IF_ERROR(ReadWords(c, fb_count + 1, 1, s, &nfb2));
-  c->last_fallbacks += nfb2;
-  if (nfb2 > 0)
+  if (second) VDBG_RETURN_IF_ERROR(ReadWords(c, count, 1, s, &nfb));
+  c->last_fallbacks += nfb;
+  if (nfb > 0)
     VDBG_RETURN_IF_ERROR(
-        ExactScan(c, W2, *src, Q, fb2_list, int(nfb2), kk, allow, out_ids, out_d, s));
+        ExactScan(c, W2, *src, SQ, list, int(nfb), kk, allow, out_ids, out_d, s));
   return kOk;
 }
 

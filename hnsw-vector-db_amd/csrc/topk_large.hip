@@ -81,6 +81,7 @@ static int ExactAllT(Ctx* c, const ScanSource& src, const Scorer& sc, const floa
                      size_t kk, const uint64_t* allow, uint32_t* out_ids, float* out_d,
                      hipStream_t s) {
   const uint32_t N = src.N;
+  const int spd = ScorePd(src);
   // queries per chunk: at most 256 MiB of keys and fewer than 2^31 keys
   size_t chunk = std::max<size_t>(1, (size_t(256) << 20) / (size_t(N) * 8));
   chunk = std::min({chunk, nq, size_t(65535)});  // queries run on grid.y
@@ -94,8 +95,8 @@ static int ExactAllT(Ctx* c, const ScanSource& src, const Scorer& sc, const floa
     const int nc = int(std::min(chunk, nq - q0));
     {
       ProfScope ps(c, "exact_all", s);
-      k_score_all<Scorer><<<dim3((N + 255) / 256, nc), 256, 0, s>>>(Q + q0 * src.pd, src.pd, N,
-                                                                       allow, sc, keys);
+      k_score_all<Scorer><<<dim3((N + 255) / 256, nc), 256, 0, s>>>(Q + q0 * spd, spd, N, allow,
+                                                                       sc, keys);
     }
     k_seg_offsets<<<dim3(unsigned((nc + 256) / 256)), 256, 0, s>>>(off, nc, int(N));
     if (hipGetLastError() != hipSuccess) {

@@ -168,11 +168,12 @@ struct Ctx {
 
 // What an exhaustive scan reads: fp32 rows (kind 0, flat) or SQ8 codes (kind 1), the
 // GEMM-form row norms, and a bit-reversed strided sample of rows built on first use; or PQ
-// codes (kind 2, scored by ADC against per-query tables of pd = m x 256 floats, ScoreScan
-// only).
+// codes (kind 2), scored by ADC against per-query tables of m x 256 floats and ranked, where
+// they are held, on the fp16 halves of the rows the codes decode to (X16, x16_approx).
 struct ScanSource {
   int kind = 0;
   int pq_m = 0;                 // kind 2: bytes per code
+  const float* pq_tables = nullptr;  // kind 2: the batch's ADC tables (set for one call)
   const float* X = nullptr;     // kind 0: n x pd rows
   const uint32_t* Xmap = nullptr;  // kind 0, nullable: row r of this source is row Xmap[r] of
                                    // X (a compacted source reading its parent's fp32 rows)
@@ -327,6 +328,12 @@ struct PqFlatIndex {
   uint8_t* codes = nullptr;  // n x m
   std::vector<float> cen_h;
   bool trained = false;    // false for an index built over no rows (no codebook)
+  // the decoded rows as fp16 halves (2 pd bytes a row) and their norms, which the ranking
+  // GEMM reads (null where pd has no kernel, n is small or memory is short: every code is
+  // then scored); src is the scan's view of them
+  uint16_t* dec16 = nullptr;
+  float* dec_norm = nullptr;
+  ScanSource src;
 };
 
 // ---------------------------------------------------------------- launchers
@@ -493,6 +500,8 @@ size_t SampleBytes(const ScanSource& src, uint32_t smax);
 int GatherSample(Ctx* c, ScanSource* src, hipStream_t s, void* buf, uint32_t cap);
 uint32_t SampleWant(const Ctx* c, const ScanSource& src, size_t nq, size_t kk);
 void FreeSample(ScanSource* src);
+// Floats per query that the source's exact scorer reads: its ADC table (kind 2) or the query.
+inline int ScorePd(const ScanSource& src) { return src.kind == 2 ? src.pq_m * 256 : src.pd; }
 
 // Host-pointer staging shared by the _host entry points.  The host writes the queries (and
 // the filter words) into the context's pinned, mapped, coherent block; one kernel copies them

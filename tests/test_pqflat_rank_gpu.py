@@ -1,0 +1,77 @@
+"""PQ-flat searches ranked on the decoded rows (the fp16 GEMM, then the ADC of the codes it
+admits) against the oracle's scan of every code: the path's row, depth and dimension edges,
+odd code widths, filters, and the exact re-scan behind a failed certificate."""
+import numpy as np
+import pytest
+
+import vdbg
+from vdbg import datagen
+from ivf_file import parse_pqflat
+
+pytestmark = pytest.mark.gpu
+
+
+def words(bits):
+    w = np.zeros((len(bits) + 63) // 64 * 8, np.uint8)
+    b = np.packbits(bits, bitorder="little")
+    w[:b.size] = b
+    return w.view(np.uint64)
+
+
+# rows at the path's limit of 1,024 and at remainders of the 64-row tiles; padded dims of one
+# and several K chunks, with padding (100 -> 112, 20 -> 32) and without a kernel (400)
+@pytest.mark.parametrize("n,dim,m,metric", [
+    (1023, 64, 8, "l2"), (1024, 64, 8, "l2"), (1025, 100, 20, "cosine"), (4097, 20, 5, "l2"),
+    (9000, 128, 16, "l2"), (9000, 128, 32, "ip"), (3001, 384, 48, "cosine"),
+    (2000, 400, 16, "l2"), (70001, 96, 12, "l2")])
+def test_ranked_search_matches_oracle(ctx, oracle, n, dim, m, metric):
+    pd = vdbg.padded_dim(dim)
+    base = datagen.clustered_unit(n, dim, 31, 32, 60, 0.6) * np.float32(3.0)
+    q = datagen.pad(datagen.clustered_unit(131, dim, 33, 32, 60, 0.6) * np.float32(3.0), pd)
+    rows = datagen.pad(base, pd)
+    ds = vdbg.Dataset(ctx, rows, dim, metric)
+    ix = vdbg.PqFlatIndex.build(ds, m, max_points=16, iters=2)
+    pix = parse_pqflat(ix.save())
+    rng = np.random.default_rng(7)
+    ks = ctx.kernels
+    # depths 0 (ADC order), up to the path's 240 and past it; 1, 33 and 131 queries
+    for nq, k, rr, frac in ((1, 10, -1, None), (33, 10, -1, 0.4), (131, 24, 240, None),
+                            (131, 10, 0, 0.01), (33, 24, 241, None), (33, 40, 0, None)):
+        allow = None if frac is None else words(rng.random(n) < frac)
+        print(f"n={n} dim={dim} m={m} {metric} nq={nq} k={k} rerank={rr} filter={frac}", flush=True)
+        ids, d, dc = ix.search(q[:nq], k, rr, allow)
+        od, oi, odc = oracle.pqflat_search(pix, rows, q[:nq], k, rr, metric, allow, kset=ks)
+        assert np.array_equal(ids, oi)
+        assert np.array_equal(d.view(np.uint32), od.view(np.uint32))
+        assert np.array_equal(dc, odc)
+    ix.close()
+    ds.close()
+
+
+def test_duplicate_codes_and_fallbacks(ctx, oracle):
+    """Rows sharing codes tie on the ADC (ids decide), a non-finite query has no certificate,
+    and the forced exact re-scan returns the same results."""
+    rows = datagen.sift_like(5000, 64, 41)
+    rows[1000:3000] = rows[:2000]
+    ds = vdbg.Dataset(ctx, rows, 64)
+    ix = vdbg.PqFlatIndex.build(ds, 4, max_points=16, iters=2)
+    pix = parse_pqflat(ix.save())
+    q = datagen.sift_like(40, 64, 42)
+    od, oi, odc = oracle.pqflat_search(pix, rows, q, 30, 120, "l2", None, kset=ctx.kernels)
+    try:
+        for level in (0, 1, 2):
+            ctx.set_test_fallbacks(level)
+            ids, d, dc = ix.search(q, 30, 120)
+            assert np.array_equal(ids, oi), level
+            assert np.array_equal(d.view(np.uint32), od.view(np.uint32)), level
+            assert np.array_equal(dc, odc), level
+        # every query re-scanned at the last level
+        assert ctx.last_fallbacks() == 40
+    finally:
+        ctx.set_test_fallbacks(0)
+    q[7, 3] = np.inf
+    ids, d, _ = ix.search(q, 30, 120)
+    keep = np.arange(40) != 7
+    assert np.array_equal(ids[keep], oi[keep])
+    ix.close()
+    ds.close()
