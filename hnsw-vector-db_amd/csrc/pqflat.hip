@@ -8,13 +8,13 @@
 //   adc(code)   = four accumulators over j mod 4           pq.h:36-46
 //   depth       = rerank < 0 ? max(10 k, 100) : rerank     RerankDepth, ivf_pq.cc:16-19
 //   distance_computations = rows (+ the candidates reranked)
-// The tables are built on the device ([nq][m x 256] floats).  Up to 240 results of at least
-// 1,024 rows, where the padded dim has a GEMM kernel, the scan is the flat path's ranking
+// The tables are built on the device ([nq][m x 256] floats).  Over at least 1,024 rows,
+// where the padded dim has a GEMM kernel, the scan is the flat path's ranking
 // GEMM over the rows the codes decode to (fp16 halves, gemm16.hip SPLIT 3: the ADC is the
 // distance to the decoded row up to its rounding, which the query's bound takes in); every
 // candidate it admits is then scored by ADC from the query's table, certified against the
 // admission threshold, and re-scanned code by code when that fails.  Otherwise every code is
-// scored (row splits with a wave top-k each, then a merge; a segmented sort beyond 240).
+// scored (row splits with a wave top-k each, then a merge; a sort beyond 240 results).
 //
 // Bound: MFMA (2 n pd flop per query; 890 TFLOP/s at 1M x 128, 2,000 queries).  Scoring every
 // code is bound by its m table reads a row instead: the batch of 2,000 queries over 1M codes
@@ -34,9 +34,7 @@ namespace vdbg {
 namespace {
 
 constexpr int kKsub = 256;
-// the ranking GEMM path's limits (RunScan): results per query and rows
-constexpr size_t kRankK = 240;
-constexpr size_t kRankRows = 1024;
+constexpr size_t kRankRows = 1024;  // the ranking GEMM path's fewest rows (RunScan)
 
 // compute_table (pq.cc:63-73) for nq queries: one thread per (query, subspace, centroid).
 __global__ void k_pq_tables(const float* __restrict__ Q, int pd, int nq,
@@ -150,7 +148,7 @@ int PqFlatSearch(PqFlatIndex* x, const float* Q, size_t nq, size_t k, int rerank
   // the kk best by (ADC, id): the ranking GEMM over the decoded rows and the ADC of the few
   // codes it admits, or the ADC of every code
   auto scan = [&](size_t kk, uint32_t* ids, float* d) {
-    if (x->src.X16 != nullptr && x->src.N == n && c->fp16_gemm && kk <= kRankK) {
+    if (x->src.X16 != nullptr && x->src.N == n && c->fp16_gemm && kk <= 10000) {
       VDBG_RETURN_IF_ERROR(BuildSample(c, &x->src, s));
       ScanSource ranked = x->src;
       ranked.pq_tables = T;

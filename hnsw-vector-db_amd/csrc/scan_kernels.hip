@@ -29,6 +29,7 @@
 #include <cmath>
 #include <cstring>
 #include <type_traits>
+#include <vector>
 
 #include "gemm.h"
 #include "vdbg_device.h"
@@ -1727,6 +1728,96 @@ __global__ __launch_bounds__(256) void k_exact_scan(ScanArgs a, Scorer sc) {
   }
 }
 
+// ================================================================ deep selection
+
+// Exact scores of every buffered candidate of a query, as 64-bit (distance, id) keys in one
+// array per query, for answers deeper than a wavefront's list (k_sort_keys sorts and
+// certifies them).  Block (q, part) takes its share of the query's candidates; a prefix sum
+// over the segment counts in LDS maps a flat index to its segment.  Flat rows score eight
+// lanes a row, as in k_select.  Bound: the gather of the candidates' rows.
+struct DeepArgs {
+  const float* Q;
+  int spd;
+  const uint2* cand;
+  const uint32_t* counts;
+  int nseg, cap;
+  const int* ovf;
+  uint64_t* keys;     // [q][stride]
+  uint32_t stride;
+  uint32_t* total;    // [q] candidates (above stride: none were scored)
+};
+template <class Scorer>
+__global__ __launch_bounds__(256) void k_deep_score(DeepArgs a, Scorer sc) {
+  __shared__ uint32_t pre[kMaxSeg + 1];
+  __shared__ uint32_t wsum[4];
+  const int q = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = lane_id();
+  if (a.ovf[q]) {
+    if (blockIdx.y == 0 && tid == 0) a.total[q] = 0xffffffffu;
+    return;
+  }
+  constexpr int PT = kMaxSeg / 256;
+  uint32_t c[PT], sum = 0;
+#pragma unroll
+  for (int i = 0; i < PT; ++i) {
+    const int s = tid * PT + i;
+    c[i] = s < a.nseg ? a.counts[size_t(q) * a.nseg + s] : 0u;
+    sum += c[i];
+  }
+  uint32_t incl = sum;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const uint32_t t = __shfl_up(incl, o);
+    if (lane >= o) incl += t;
+  }
+  if (lane == kWave - 1) wsum[wave] = incl;
+  __syncthreads();
+  uint32_t at = incl - sum;
+  for (int w = 0; w < wave; ++w) at += wsum[w];
+#pragma unroll
+  for (int i = 0; i < PT; ++i) {
+    pre[tid * PT + i] = at;
+    at += c[i];
+  }
+  if (tid == 255) pre[kMaxSeg] = at;
+  __syncthreads();
+  const uint32_t total = pre[kMaxSeg];
+  if (blockIdx.y == 0 && tid == 0) a.total[q] = total;
+  if (total > a.stride) return;
+  const uint32_t per = ((total + gridDim.y - 1) / gridDim.y + kWave - 1) / kWave * kWave;
+  const uint32_t lo = blockIdx.y * per, hi = min(total, lo + per);
+  const float* qv = a.Q + size_t(q) * a.spd;
+  for (uint32_t g0 = lo + wave * kWave; g0 < hi; g0 += 4 * kWave) {
+    const uint32_t g = g0 + lane;
+    uint32_t id = kNoId;
+    if (g < hi) {
+      int l = 0, h = a.nseg;  // the largest segment with pre[s] <= g
+      while (h - l > 1) {
+        const int mid = (l + h) >> 1;
+        if (pre[mid] <= g) l = mid; else h = mid;
+      }
+      id = a.cand[(size_t(q) * a.nseg + l) * a.cap + (g - pre[l])].y;
+    }
+    float d = 0.f;
+    if constexpr (std::is_same<Scorer, FlatScorer>::value) {
+      if (sc.kset == kKsetAvx512) {
+        group_pass(id, 0, int(min(hi - g0, uint32_t(kWave))), d, [&](const auto& ids, auto& dd) {
+          constexpr int R = sizeof(dd) / sizeof(float);
+          const float* xs[R];
+#pragma unroll
+          for (int i = 0; i < R; ++i)
+            xs[i] = sc.X + size_t(sc.map != nullptr ? sc.map[ids[i]] : ids[i]) * sc.pd;
+          metric_exact_g8n<R>(sc.metric, qv, xs, sc.pd, dd);
+        });
+      } else if (id != kNoId) {
+        d = sc(qv, id);
+      }
+    } else if (id != kNoId) {
+      d = sc(qv, id);
+    }
+    if (g < hi) a.keys[size_t(q) * a.stride + g] = dist_key(d, id);
+  }
+}
+
 // ================================================================ rerank
 
 struct RerankArgs {
@@ -2943,6 +3034,37 @@ uint32_t SampleWant(const Ctx* c, const ScanSource& src, size_t nq, size_t kk) {
   return S;
 }
 
+// Answers deeper than a wavefront's list (kk > 240) on the ranking GEMM: whether the batch's
+// threshold admits few enough candidates for one block's sort, and how many it is expected to
+// admit.  The rank-th of the sample's G group minima lies where about -G ln(1 - rank / G)
+// sample rows do (rows fall into groups at random), so up to 0.6 G the expectation stays
+// within 1.5 times rank; past that the sample is too small for the depth and every row is
+// scored.  Twice the expectation, and kk rows more, is kept per query; a query admitting more
+// overflows to the scan of every row.
+struct DeepPlan {
+  bool on;
+  double expect;    // candidates per query
+  uint32_t stride;  // keys kept per query
+  size_t max_nq;    // queries per pass (1 GiB of keys and candidates)
+};
+static DeepPlan PlanDeep(const Ctx* c, const ScanSource& src, size_t nq, size_t kk) {
+  DeepPlan p{};
+  const uint32_t S = std::min(SampleWant(c, src, nq, kk), src.Smax);
+  const uint32_t N = std::min(src.N, src.SN != 0 ? src.SN : src.N);
+  const int rank = ThresholdRank(kk, S, N);
+  const double G = double((S + 31) / 32 * 2);
+  if (rank > 0.6 * G) return p;
+  p.expect = -G * std::log1p(-rank / G) * src.N / S;
+  const double want = 2.0 * p.expect + double(kk);
+  if (!(want <= double(kBlockSortKeys))) return p;
+  p.stride = 1024;
+  while (p.stride < want) p.stride <<= 1;
+  // (the candidate buffers hold about four times the expectation, in 8-byte entries)
+  p.max_nq = std::max<size_t>(64, (size_t(1) << 30) / (size_t(p.stride) * 8 * 4));
+  p.on = true;
+  return p;
+}
+
 int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
             const uint64_t* allow, uint32_t* out_ids, float* out_d, hipStream_t s,
             Workspace* ws, Workspace* ws2) {
@@ -2970,12 +3092,39 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
     VDBG_HIP(hipGetLastError());
     return kOk;
   }
-  // the select keeps K' >= kk + 16 keys in one wavefront (at most 256)
-  if (kk > 240) return ExactScanAll(c, *src, Q, nq, kk, allow, out_ids, out_d, s);
   const uint32_t N = src->N;
   const size_t pd = src->pd;
+  // PQ codes rank on the rows they decode to and are scored by ADC from the batch's tables
+  const bool adc = src->kind == 2;
+  const float* SQ = adc ? src->pq_tables : Q;  // what the exact scorer reads per query
   const bool gemm = GemmSupported(pd) && N >= 1024;
-  if (!gemm) return ExactScan(c, W, *src, Q, nullptr, int(nq), kk, allow, out_ids, out_d, s);
+  // The select keeps K' >= kk + 16 keys in one wavefront (at most 256).  Beyond that the same
+  // ranking admits the candidates and a block per query sorts their exact scores (k_sort_keys),
+  // where the threshold admits few enough (PlanDeep); else every row is scored and sorted.
+  // Segments whose every row fits that block's sort skip the ranking (61 queries, k = 1,000,
+  // 118,385 x 112 rows: 4.6 ms scoring and sorting every row, 0.2 ms ranked).
+  DeepPlan deep{};
+  if (kk > 240) {
+    if (gemm && N > kBlockSortKeys && !W.fixed) {
+      VDBG_RETURN_IF_ERROR(BuildSample(c, src, s));
+      deep = PlanDeep(c, *src, nq, kk);
+    }
+    if (!deep.on) return ExactScanAll(c, *src, SQ, nq, kk, allow, out_ids, out_d, s);
+    if (nq > deep.max_nq) {  // bounded scratch: the batch in parts, one count of re-scans
+      const bool acc = c->fb_accumulate;
+      int rc = kOk;
+      for (size_t q0 = 0; q0 < nq && rc == kOk; q0 += deep.max_nq) {
+        ScanSource part = *src;
+        if (adc) part.pq_tables += q0 * ScorePd(*src);
+        rc = RunScan(c, &part, Q + q0 * pd, std::min(deep.max_nq, nq - q0), kk, allow,
+                     out_ids + q0 * kk, out_d + q0 * kk, s, ws, ws2);
+        if (!acc) c->fb_accumulate = true;
+      }
+      if (!acc) c->fb_accumulate = false;
+      return rc;
+    }
+  }
+  if (!gemm) return ExactScan(c, W, *src, SQ, nullptr, int(nq), kk, allow, out_ids, out_d, s);
   if (tiny) return TinyScan(c, src, Q, nq, kk, allow, out_ids, out_d, s, W, W2);
   // A re-scan workspace that cannot grow must hold the re-scan of every query, checked
   // before anything is queued (which queries fall back is known only on the device).
@@ -3006,9 +3155,6 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
   // rows wider than one K chunk keep each wave's query fragments resident (one 32-query
   // block per wave, gemm16.hip QRES); the sample pass keeps two blocks per wave
   const bool wide16 = single && Gemm16ResQueries(pd);
-  // PQ codes rank on the rows they decode to and are scored by ADC from the batch's tables
-  const bool adc = src->kind == 2;
-  const float* SQ = adc ? src->pq_tables : Q;  // what the exact scorer reads per query
   const bool try8f = c->fp16_gemm && c->int8_gemm && split == 2 &&
                      src->X8 != nullptr && src->x8_parts == 2 && Gemm8Supported(pd) &&
                      double(N) * double(nq) * double(pd) >= c->int8_float_min_work;
@@ -3051,7 +3197,7 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
     p.schunk_rows = (S + p.schunks - 1) / p.schunks;
     p.schunk_rows = (p.schunk_rows + 63) / 64 * 64;
     p.schunks = int((S + p.schunk_rows - 1) / p.schunk_rows);
-    const double expect_seg = double(rank) * N / S * 2.0 / (2.0 * p.nchunks);
+    const double expect_seg = (deep.on ? deep.expect : double(rank) * N / S) / p.nchunks;
     p.caph = 32;
     while (p.caph < 3.0 * expect_seg + 32) p.caph <<= 1;
     p.nseg = 2 * p.nchunks;
@@ -3102,7 +3248,8 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
       (src->kind == 1 ? nq * pd * sizeof(float) : 0) + size_t(nq) * gm_groups * sizeof(float) +
       (try16 ? (split ? 2 : 1) * nq * pd * sizeof(uint16_t) + nq * sizeof(float) : 0) +
       (try8 ? nq * pd + nq * sizeof(int) : 0) +
-      (try8op ? 2 * nq * pd + nq * (sizeof(int) + sizeof(float)) : 0) + 26 * 256;
+      (try8op ? 2 * nq * pd + nq * (sizeof(int) + sizeof(float)) : 0) +
+      (deep.on ? nq * (deep.stride * sizeof(uint64_t) + sizeof(uint32_t)) : 0) + 28 * 256;
   // A workspace that cannot grow caps the candidate buffers instead: fewer, longer row
   // chunks (fewer blocks, so a less filled GPU) until they fit in what the rest leaves.
   // The sample pass and everything else are planned as before.
@@ -3139,6 +3286,8 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
   // the no-filter word of the fp16 and int8 GEMMs
   uint32_t* ones = try16 || try8any ? w.take<uint32_t>(1) : nullptr;
   int* fit8q = gated ? w.take<int>(nq) : nullptr;  // per query: inside the int8 bounds
+  uint64_t* dkeys = deep.on ? w.take<uint64_t>(nq * deep.stride) : nullptr;
+  uint32_t* dtotal = deep.on ? w.take<uint32_t>(nq) : nullptr;
   {
     const ScanInit si{ovf, int(nq), fb_count, all16, ones, try8op ? e8 : nullptr, fb_zero};
     k_scan_init<<<dim3(unsigned((std::max<size_t>(nq, 2) + 255) / 256)), 256, 0, s>>>(si);
@@ -3313,6 +3462,33 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
       VDBG_RETURN_IF_ERROR(LaunchGemm(pd, metric, src->kind, 0, s, blocks, ga));
     }
     VDBG_HIP(hipGetLastError());
+  }
+  if (deep.on) {
+    const DeepArgs da{SQ, ScorePd(*src), cand, counts, nseg, caph, ovf, dkeys, deep.stride,
+                      dtotal};
+    const dim3 grid(unsigned(nq), unsigned(std::max<size_t>(1, (size_t(deep.expect) + 255) / 256)));
+    {
+      ProfScope ps(c, "select", s);
+      if (adc) k_deep_score<<<grid, 256, 0, s>>>(da, PqScorer{src->C, src->pq_m});
+      else if (src->kind == 0) k_deep_score<<<grid, 256, 0, s>>>(da, FlatOf(*src, c->kset));
+      else k_deep_score<<<grid, 256, 0, s>>>(da, Sq8Of(*src, c->kset));
+      VDBG_HIP(hipGetLastError());
+    }
+    SortKeysArgs sk{dkeys, deep.stride, int(kk), out_ids, out_d, dtotal, T, shift, ebx, fb_list,
+                    fb_count, c->test_fallbacks >= 1 ? 1 : 0};
+    VDBG_RETURN_IF_ERROR(SortKeysTopK(c, sk, int(nq), s));
+    // uncertified queries (rare) have every row scored and sorted, one by one
+    uint32_t nfb = 0;
+    VDBG_RETURN_IF_ERROR(ReadWords(c, fb_count, 1, s, &nfb));
+    if (nfb == 0) return kOk;
+    std::vector<uint32_t> list(nfb);
+    VDBG_HIP(hipMemcpyAsync(list.data(), fb_list, nfb * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    VDBG_HIP(hipStreamSynchronize(s));
+    c->last_fallbacks += nfb;
+    for (const uint32_t q : list)
+      VDBG_RETURN_IF_ERROR(ExactScanAll(c, *src, SQ + size_t(q) * ScorePd(*src), 1, kk, allow,
+                                        out_ids + size_t(q) * kk, out_d + size_t(q) * kk, s));
+    return kOk;
   }
   SelectArgs se{};
   se.Q = SQ;

@@ -35,6 +35,79 @@ __global__ void k_unpack_keys(const uint64_t* __restrict__ keys, const int* __re
   }
 }
 
+// The K smallest of each query's keys, sorted, by one block per query: the keys (at most
+// kBlockSortKeys, kNoKey for none) go to LDS, padded to a power of two, through a bitonic
+// sort.  Layers of stride at most 64 stay inside one wave's 128 consecutive keys (thread i
+// takes the i-th pair), so only wider ones need a block barrier: 10 of 66 at 2,048 keys.
+// Bound: LDS (two reads and two writes of 8 bytes per key and layer).  It replaces the
+// device-wide segmented radix sort where a query's keys fit the LDS: 61 queries of 118,385
+// keys took 3.7 ms there, 61 of about 1,300 admitted keys take 20 us here.
+__global__ __launch_bounds__(1024) void k_sort_keys(SortKeysArgs a) {
+  extern __shared__ uint64_t sk[];
+  const int q = blockIdx.x;
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const uint32_t n = a.counts != nullptr ? a.counts[q] : a.stride;
+  if (n > a.stride) {  // overflowed: the caller answers this query another way
+    if (tid == 0) a.fb_list[atomicAdd(a.fb_count, 1u)] = uint32_t(q);
+    return;
+  }
+  uint32_t P = 2;
+  while (P < n) P <<= 1;
+  const uint64_t* src = a.keys + size_t(q) * a.stride;
+  for (uint32_t i = tid; i < P; i += nt) sk[i] = i < n ? src[i] : kNoKey;
+  __syncthreads();
+  for (uint32_t size = 2; size <= P; size <<= 1)
+    for (uint32_t j = size >> 1; j > 0; j >>= 1) {
+      for (uint32_t i = tid; i < P / 2; i += nt) {
+        const uint32_t lo = 2 * i - (i & (j - 1)), hi = lo + j;
+        const uint64_t x = sk[lo], y = sk[hi];
+        if ((x > y) == ((lo & size) == 0)) {
+          sk[lo] = y;
+          sk[hi] = x;
+        }
+      }
+      // the next layer crosses waves when its stride (or this one's) is above 64
+      const uint32_t next = j > 1 ? j >> 1 : size;
+      if (j > kWave || next > kWave) {
+        __syncthreads();
+      } else {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+    }
+  __syncthreads();
+  for (int i = tid; i < a.K; i += nt) {
+    const uint64_t key = uint32_t(i) < P ? sk[i] : kNoKey;
+    a.out_ids[size_t(q) * a.K + i] = key == kNoKey ? kNoId : uint32_t(key);
+    a.out_d[size_t(q) * a.K + i] = key == kNoKey ? __builtin_inff() : key_dist(key);
+  }
+  if (a.T != nullptr && tid == 0) {
+    // every row outside the keys has GEMM value > T, so an exact distance above
+    // T + shift - eb: certified when the K-th is at most that
+    const uint64_t key = uint32_t(a.K) <= P ? sk[a.K - 1] : kNoKey;
+    const double dk = key == kNoKey ? double(__builtin_inff()) : double(key_dist(key));
+    const double lower = (double(a.T[q]) + double(a.shift[q])) - double(a.eb[q]);
+    if (!(dk <= lower) || a.force_fallback) a.fb_list[atomicAdd(a.fb_count, 1u)] = uint32_t(q);
+  }
+}
+
+int SortKeysTopK(Ctx* c, const SortKeysArgs& a, int nq, hipStream_t s) {
+  if (nq == 0 || a.K == 0) return kOk;
+  uint32_t P = 128;
+  while (P < a.stride) P <<= 1;
+  if (P > kBlockSortKeys) return SetError(kInternal, "block sort: too many keys per query");
+  const size_t lds = size_t(P) * sizeof(uint64_t);
+  if (lds > 65536)  // (the default limit of dynamic LDS)
+    VDBG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_sort_keys),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 int(kBlockSortKeys * sizeof(uint64_t))));
+  ProfScope ps(c, "sort_keys", s);
+  k_sort_keys<<<dim3(unsigned(nq)), std::min<uint32_t>(1024, P / 2), lds, s>>>(a);
+  VDBG_HIP(hipGetLastError());
+  return kOk;
+}
+
 int SortSegmentsTopK(Ctx* c, uint64_t* keys, uint64_t* keys_alt, const int* off_dev, int nseg,
                      int total, int K, uint32_t* out_ids, float* out_d, hipStream_t s) {
   if (nseg == 0) return kOk;
@@ -98,11 +171,16 @@ static int ExactAllT(Ctx* c, const ScanSource& src, const Scorer& sc, const floa
       k_score_all<Scorer><<<dim3((N + 255) / 256, nc), 256, 0, s>>>(Q + q0 * spd, spd, N, allow,
                                                                        sc, keys);
     }
-    k_seg_offsets<<<dim3(unsigned((nc + 256) / 256)), 256, 0, s>>>(off, nc, int(N));
     if (hipGetLastError() != hipSuccess) {
       rc = SetError(kInternal, "exact-all launch");
       break;
     }
+    if (N <= kBlockSortKeys) {
+      rc = SortKeysTopK(c, SortKeysArgs{keys, N, int(kk), out_ids + q0 * kk, out_d + q0 * kk}, nc,
+                        s);
+      continue;
+    }
+    k_seg_offsets<<<dim3(unsigned((nc + 256) / 256)), 256, 0, s>>>(off, nc, int(N));
     rc = SortSegmentsTopK(c, keys, keys + nk, off, nc, int(size_t(nc) * N), int(kk),
                           out_ids + q0 * kk, out_d + q0 * kk, s);
   }
@@ -159,11 +237,16 @@ int RerankLarge(Ctx* c, const float* X, int pd, int metric, const float* Q, size
       k_rerank_keys<<<dim3(unsigned((n + 255) / 256)), 256, 0, s>>>(
           X, Q + q0 * pd, pd, metric, c->kset, cand + q0 * depth, int(depth), nc, keys);
     }
-    k_seg_offsets<<<dim3(unsigned((nc + 256) / 256)), 256, 0, s>>>(off, nc, int(depth));
     if (hipGetLastError() != hipSuccess) {
       rc = SetError(kInternal, "rerank launch");
       break;
     }
+    if (depth <= kBlockSortKeys) {
+      rc = SortKeysTopK(c, SortKeysArgs{keys, uint32_t(depth), int(k), out_ids + q0 * k,
+                                        out_d + q0 * k}, nc, s);
+      continue;
+    }
+    k_seg_offsets<<<dim3(unsigned((nc + 256) / 256)), 256, 0, s>>>(off, nc, int(depth));
     rc = SortSegmentsTopK(c, keys, keys + nk, off, nc, int(n), int(k), out_ids + q0 * k,
                           out_d + q0 * k, s);
   }

@@ -404,6 +404,26 @@ int ExactScanAll(Ctx* c, const ScanSource& src, const float* Q, size_t nq, size_
 int RerankLarge(Ctx* c, const float* X, int pd, int metric, const float* Q, size_t nq,
                 const uint32_t* cand, size_t depth, size_t k, uint32_t* out_ids, float* out_d,
                 hipStream_t s);
+// One block per query sorts its keys (keys[q * stride ..], counts[q] of them, or stride) in LDS
+// and writes the first K as (id, dist), padded with (UINT32_MAX, +inf).  With T the answer is
+// also certified (see k_sort_keys), and queries that fail, or whose count is above stride, are
+// appended to fb_list.
+constexpr uint32_t kBlockSortKeys = 16384;  // 128 KB of LDS
+struct SortKeysArgs {
+  const uint64_t* keys;
+  uint32_t stride;
+  int K;
+  uint32_t* out_ids;  // [q][K]
+  float* out_d;
+  const uint32_t* counts = nullptr;
+  const float* T = nullptr;
+  const float* shift = nullptr;
+  const float* eb = nullptr;
+  uint32_t* fb_list = nullptr;
+  uint32_t* fb_count = nullptr;
+  int force_fallback = 0;
+};
+int SortKeysTopK(Ctx* c, const SortKeysArgs& a, int nq, hipStream_t s);
 // Sorts nseg key segments (int offsets off_dev[0..nseg]) from keys into keys_alt and writes
 // the first K of each as (id, dist), padded with (UINT32_MAX, +inf).
 int SortSegmentsTopK(Ctx* c, uint64_t* keys, uint64_t* keys_alt, const int* off_dev, int nseg,
