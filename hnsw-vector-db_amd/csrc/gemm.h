@@ -10,6 +10,7 @@
 namespace vdbg {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // 16-byte vector (plain loads)
 
 struct GemmArgs {
   const float* X;      // fp32 rows (KIND 0)

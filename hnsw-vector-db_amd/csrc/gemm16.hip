@@ -24,7 +24,6 @@
 namespace vdbg {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // 16-byte vector (plain loads)
 
 // Block = 4 waves x (32 QB) queries each x one chunk of rows; block b takes work item
 // (b % 8) * per_xcd + b / 8 so the items of one XCD are consecutive and share row chunks in

@@ -30,7 +30,6 @@ namespace vdbg {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kDead8 = -(1 << 29);   // accumulator start of rows that take no part
 constexpr int kLive8 = -(1 << 28);   // every live row's u is above this

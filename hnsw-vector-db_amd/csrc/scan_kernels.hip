@@ -2234,6 +2234,9 @@ constexpr int kTinyQ = 2;       // queries
 constexpr int kTinyK = 48;      // k (kp = k + 16 <= 64 keys per chunk)
 constexpr int kTinyMaxPd = 256; // |key| < 2^23 stays exact in fp32
 constexpr int kTinyWaves = 4;   // waves per scan block
+constexpr int kRowQ = 8;        // queries of k_row_scan
+constexpr int kRowMaxQ = 4096;  // query floats it stages (nq * pd)
+constexpr int kRowTile = 1024;  // rows a block lists at a time
 
 struct TinyArgs {
   const float* Q;
@@ -2401,6 +2404,224 @@ __global__ __launch_bounds__(kTinyWaves * 64) void k_tiny_scan(TinyArgs a) {
   for (int q = 0; q < NQ; ++q) {
     if (q >= a.nq) break;
     for (int w = 0; w < kTinyWaves - 1; ++w) top[q].insert(md[w][q][lane], mi[w][q][lane]);
+    const size_t o = size_t(q) * a.nchunks + blockIdx.x;
+    if (lane < a.kp) a.part[o * a.kp + lane] = make_uint2(__float_as_uint(top[q].k.d[0]), top[q].k.id[0]);
+    const float kth = __shfl(top[q].k.d[0], rl);
+    const uint32_t kid = __shfl(top[q].k.id[0], rl);
+    if (lane == 0) a.bound[o] = kid == kNoId ? __builtin_inff() : kth;
+  }
+}
+
+// ================================================================ small batches of any rows
+//
+// At most kRowQ queries over one or several row sets (the segments of a collection) of any
+// values: k_row_scan scores every allowed row once, from its fp16 copy where it has one (half
+// the bytes) or its fp32 rows, and k_tiny_merge re-scores and certifies as it does for
+// k_tiny_scan's keys.  The key is the GEMM value fma(f, x.q, ||x||^2) (f = -2 2^-e for rows held
+// as fp16(x 2^e); -2^-e and no norm for inner product) accumulated in fp32 against the fp32
+// query: its error is inside the bound query_prep_wave states for the h-half GEMM (the rows'
+// rounding alone where that one drops both operands' low halves), or for the fp32 one.
+//
+// A block takes a chunk of a set's rows, kRowTile at a time.  Under a filter the block first
+// lists the tile's allowed rows in LDS, so a row that is not allowed costs one bit, and a
+// selective filter needs no compaction pass over the segment.  Eight lanes share a row (its
+// bytes read in 128-byte runs), four rows to a group, so a wave has 32 rows' loads in flight;
+// the groups' sums reduce by DPP and each wave keeps the kp best keys as k_tiny_scan does.
+//
+// Bound: the rows' bytes (200,000 x 384 fp16 rows, one query: 33 us, 4.6 TB/s, the rate of a
+// large copy on this card).
+struct RowSetArgs {
+  const void* X;          // fp16 or fp32 rows
+  const float* rn;
+  const uint64_t* allow;  // nullable
+  uint32_t N, chunk_rows; // chunk_rows: a multiple of 64
+  int chunk0;             // the set's first chunk
+  float f;
+};
+struct RowScanArgs {
+  RowSetArgs set[kRowSets];
+  int nsets;
+  const float* Q;
+  int nq, pd, metric, kp;
+  uint2* part;            // [q][chunk][kp] (key bits, row)
+  float* bound;           // [q][chunk]
+  int nchunks;
+  uint32_t* fb_count;     // [2] zeroed by block 0
+  uint32_t* fb_zero;      // nullable: zeroed by block 0
+};
+
+template <int NQ, bool F16>
+__global__ __launch_bounds__(256) void k_row_scan(RowScanArgs a) {
+  constexpr int W = kTinyWaves, R = 4;
+  constexpr int U = F16 ? 4 : 2;  // 64-dim runs loaded at a time
+  __shared__ float sd[W][NQ][2 * kWave];
+  __shared__ uint32_t si[W][NQ][2 * kWave];
+  __shared__ float md[W][NQ][kWave];
+  __shared__ uint32_t mi[W][NQ][kWave];
+  __shared__ uint64_t s_word[kRowTile / 64];
+  __shared__ uint16_t s_row[kRowTile];
+  extern __shared__ float s_q[];  // [NQ][pd]
+  const int tid = threadIdx.x, wave = tid >> 6, lane = lane_id();
+  const int g = lane >> 3, j = lane & 7;
+  if (blockIdx.x == 0 && tid < 2) a.fb_count[tid] = 0;
+  if (blockIdx.x == 0 && tid == 0 && a.fb_zero != nullptr) *a.fb_zero = 0;
+  int p = 0;
+  while (p + 1 < a.nsets && int(blockIdx.x) >= a.set[p + 1].chunk0) ++p;
+  const RowSetArgs& st = a.set[p];
+  for (int e = tid; e < NQ * a.pd; e += W * kWave) s_q[e] = e < a.nq * a.pd ? a.Q[e] : 0.f;
+  const uint32_t r0 = (blockIdx.x - uint32_t(st.chunk0)) * st.chunk_rows;
+  const uint32_t r1 = min(st.N, r0 + st.chunk_rows);
+  WaveTopK<1> top[NQ];
+  int staged[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    top[q].init();
+    staged[q] = 0;
+  }
+  const int rl = (a.kp - 1) & (kWave - 1);
+  for (uint32_t base = r0; base < r1; base += kRowTile) {
+    const uint32_t rows = min(uint32_t(kRowTile), r1 - base);
+    uint32_t n = rows;
+    __syncthreads();  // the query is staged; the last tile's list has been read
+    if (st.allow != nullptr) {
+      if (tid < kRowTile / 64) {
+        const uint32_t lo = tid * 64;
+        uint64_t v = lo < rows ? st.allow[(base >> 6) + tid] : 0ull;
+        if (lo < rows && rows - lo < 64) v &= (1ull << (rows - lo)) - 1ull;
+        s_word[tid] = v;
+      }
+      __syncthreads();
+      n = 0;
+      for (int t = 0; t < kRowTile / 64; ++t) {
+        const uint64_t v = s_word[t];
+        if ((t & (W - 1)) == wave && ((v >> lane) & 1ull))
+          s_row[n + __popcll(v & ((1ull << lane) - 1ull))] = uint16_t(t * 64 + lane);
+        n += uint32_t(__popcll(v));
+      }
+      __syncthreads();
+    }
+    for (uint32_t i0 = wave * 32; i0 < n; i0 += W * 32) {
+      uint32_t row[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const uint32_t i = min(i0 + g * R + r, n - 1);
+        row[r] = base + (st.allow != nullptr ? uint32_t(s_row[i]) : i);
+      }
+      float acc[NQ][R] = {};
+      for (int t0 = 0; t0 < a.pd; t0 += 64 * U) {
+        u32x4 v[R][U][F16 ? 1 : 2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int col = min(t0 + 64 * u + 8 * j, a.pd - 8);  // past the row: repeats, unused
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            const size_t at = size_t(row[r]) * a.pd + col;
+            if constexpr (F16) {
+              v[r][u][0] = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(st.X) + at);
+            } else {
+              const float* x = static_cast<const float*>(st.X) + at;
+              v[r][u][0] = *reinterpret_cast<const u32x4*>(x);
+              v[r][u][1] = *reinterpret_cast<const u32x4*>(x + 4);
+            }
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int col = t0 + 64 * u + 8 * j;
+          if (col >= a.pd) break;
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) {
+            const float4 q0 = *reinterpret_cast<const float4*>(&s_q[q * a.pd + col]);
+            const float4 q1 = *reinterpret_cast<const float4*>(&s_q[q * a.pd + col + 4]);
+            const float qs[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+              for (int e = 0; e < 8; ++e) {
+                float x;
+                if constexpr (F16)
+                  x = float(__builtin_bit_cast(_Float16, uint16_t(v[r][u][0][e / 2] >> (16 * (e & 1)))));
+                else
+                  x = __uint_as_float(v[r][u][e / 4][e & 3]);
+                acc[q][r] = fmaf(x, qs[e], acc[q][r]);
+              }
+          }
+        }
+      }
+      // lane j < 4 of a group takes its row j
+      const uint32_t item = i0 + g * R + (j & (R - 1));
+      const bool live = j < R && item < n;
+      uint32_t rid = row[0];
+#pragma unroll
+      for (int r = 1; r < R; ++r) rid = (j & (R - 1)) == r ? row[r] : rid;
+      const float xn = a.metric == 0 ? st.rn[rid] : 0.f;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        if (q >= a.nq) break;
+        float dot = 0.f;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          float x = acc[q][r];
+          x += lane_mirror8(x);
+          x += lane_xor(x, 2);
+          x += lane_xor(x, 1);
+          dot = (j & (R - 1)) == r ? x : dot;
+        }
+        const float key = fmaf(st.f, dot, xn);
+        const float td = __shfl(top[q].k.d[0], rl);
+        const uint32_t ti = __shfl(top[q].k.id[0], rl);
+        const bool want = live && nb_less(key, rid, td, ti);
+        const uint64_t bal = __ballot(want);
+        if (bal == 0) continue;
+        const int pos = staged[q] + __popcll(bal & ((1ull << lane) - 1ull));
+        if (want) {
+          sd[wave][q][pos] = key;
+          si[wave][q][pos] = rid;
+        }
+        staged[q] += __popcll(bal);
+        if (staged[q] >= kWave) {
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          const float d0 = sd[wave][q][lane];
+          const uint32_t i1 = si[wave][q][lane];
+          const bool more = lane + kWave < staged[q];
+          const float d2 = more ? sd[wave][q][lane + kWave] : 0.f;
+          const uint32_t i2 = more ? si[wave][q][lane + kWave] : 0u;
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          if (more) {
+            sd[wave][q][lane] = d2;
+            si[wave][q][lane] = i2;
+          }
+          staged[q] -= kWave;
+          top[q].insert(d0, i1);
+        }
+      }
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if (q >= a.nq) break;
+    if (staged[q] > 0) {
+      const bool have = lane < staged[q];
+      top[q].insert(have ? sd[wave][q][lane] : __builtin_inff(), have ? si[wave][q][lane] : kNoId);
+    }
+    md[wave][q][lane] = top[q].k.d[0];
+    mi[wave][q][lane] = top[q].k.id[0];
+  }
+  __syncthreads();
+  // the four lists of query q merge in wave q % 4
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if (q >= a.nq) break;
+    if ((q & (W - 1)) != wave) continue;
+    for (int w = 1; w < W; ++w)
+      top[q].insert(md[(wave + w) & (W - 1)][q][lane], mi[(wave + w) & (W - 1)][q][lane]);
     const size_t o = size_t(q) * a.nchunks + blockIdx.x;
     if (lane < a.kp) a.part[o * a.kp + lane] = make_uint2(__float_as_uint(top[q].k.d[0]), top[q].k.id[0]);
     const float kth = __shfl(top[q].k.d[0], rl);
@@ -2681,27 +2902,54 @@ __global__ __launch_bounds__(kSmallWaves * 64, SmallOccupancy(NKB * 32)) void k_
 
 constexpr int kMergeWaves = 8;  // key-merging waves of k_tiny_merge (plus one preparing)
 
+// One row set of a merge: its chunks among the scan's, what bounds its keys, its rows.
+struct MergeSet {
+  RowStats xs;
+  float rmag;
+  int x16_exp, single16;
+  int chunk0, nchunks;
+  FlatScorer8 sc;         // the rows and their int8 copy (the int8 re-scoring reads the copy)
+};
 struct TinyMergeArgs {
-  PrepArgs pa;            // the query's operands and bound (fit8q set)
-  const uint2* part;
-  const float* bound;
-  int nchunks, kp, k;
-  FlatScorer8 sc;         // the rows and their int8 copy (the re-scoring reads the copy)
-  uint32_t* out_ids;
+  PrepArgs pa;            // the query's operands and bound (fit8q set on int8 keys)
+  MergeSet set[kRowSets];
+  const uint2* part;      // [q][chunk][kp]
+  const float* bound;     // [q][chunk]
+  int nchunks, kp, k;     // nchunks: of all sets
+  uint32_t* out_ids;      // [set][q][k]
   float* out_d;
-  uint32_t* fb_list;
-  uint32_t* fb_count;     // [0] fallbacks, [1] finished merges
-  uint32_t* host_flag;    // nullable: pinned host words ([0] sequence, [1] fallback count)
-                          // the last merge publishes the count into
-  uint32_t seq;
+  uint32_t* fb_list;      // set * nq + q of every uncertified answer (null: only counted)
+  uint32_t* fb_count;
   int force_fallback;
 };
 
-// One block of 8 + 1 waves per query.  Each of 8 waves loads its share of the chunks' keys
+// The wave's 64 values sorted ascending across the lanes.
+__device__ __forceinline__ float wave_sort(float v) {
+  const int lane = lane_id();
+#pragma unroll
+  for (int size = 2; size <= kWave; size <<= 1)
+#pragma unroll
+    for (int j = size >> 1; j > 0; j >>= 1) {
+      const float o = lane_xor(v, j);
+      const bool lo = ((lane & size) == 0) == ((lane & j) == 0);
+      v = lo ? fminf(v, o) : fmaxf(v, o);
+    }
+  return v;
+}
+
+// One block of 8 + 1 waves per query and row set.  Each of 8 waves loads its share of the chunks' keys
 // with all loads in flight (up to 32 per lane at a time) and keeps the 64 best (staged, then
 // inserted 64 at a time); the ninth prepares the query's operands and bound meanwhile.  The
 // 8 sorted lists merge in a three-level tree of bitonic merges into wave 0, which then
-// re-scores and certifies.
+// re-scores and certifies.  I8: the keys are k_tiny_scan's or k_small_scan's (integer rows, one
+// row set), else k_row_scan's.
+//
+// Bound: latency (one block per query).  Keys above B, the (k + 9)-th smallest of 64 lanes'
+// minima over the chunks' first keys, are dropped before any insertion: k + 9 keys of
+// different chunks lie at or below B, so the best k + 9 of all do.  About 30 of 9,700 keys
+// pass at k = 10 over 512 chunks, where the smallest chunk bound alone passed some 300 (22.4
+// -> 17.2 us, one query over 1M rows).
+template <bool I8>
 __global__ __launch_bounds__(kMergeWaves * 64 + 64) void k_tiny_merge(TinyMergeArgs a) {
   constexpr int W = kMergeWaves;  // waves that merge keys; wave W prepares the query
   constexpr int B = 8;   // keys per lane of a group
@@ -2713,15 +2961,32 @@ __global__ __launch_bounds__(kMergeWaves * 64 + 64) void k_tiny_merge(TinyMergeA
   __shared__ uint32_t si[W][(B + 1) * kWave];
   __shared__ uint32_t ys[256];  // the query packed into int8 (Int8Query)
   const int q = blockIdx.x;
+  const MergeSet& ms = a.set[I8 ? 0 : blockIdx.y];
+  const int nch = ms.nchunks;
   const int tid = threadIdx.x, wave = tid >> 6, lane = lane_id();
   WaveTopK<1> top;
   top.init();
   float lb = __builtin_inff();
   const bool keys = wave < W;
-  const int per = (a.nchunks + W - 1) / W;
-  const int c0 = keys ? min(a.nchunks, wave * per) : a.nchunks, c1 = min(a.nchunks, c0 + per);
+  const int per = (nch + W - 1) / W;
+  const int c0 = keys ? min(nch, wave * per) : nch, c1 = min(nch, c0 + per);
   const size_t total = size_t(c1 - c0) * a.kp;
-  const uint2* src = a.part + (size_t(q) * a.nchunks + c0) * a.kp;
+  const size_t qc = size_t(q) * a.nchunks + ms.chunk0;  // the set's first chunk
+  const uint2* src = a.part + (qc + c0) * a.kp;
+  // this query's and set's words of the preparation
+  PrepArgs pa = a.pa;
+  if constexpr (!I8) {
+    pa.xs = ms.xs;
+    pa.rmag = ms.rmag;
+    pa.x16_exp = ms.x16_exp;
+    pa.single16 = ms.single16;
+    const size_t o = size_t(blockIdx.y) * pa.nq;
+    pa.shift += o;
+    pa.eb += o;
+    pa.exact += o;
+    pa.Qf += o;
+    pa.Q16 += o * 2 * pa.pd;
+  }
   constexpr size_t kGroup = size_t(B) * kWave;
   auto load_keys = [&](size_t g0, uint2 (&v)[B]) __attribute__((always_inline)) {
 #pragma unroll
@@ -2740,21 +3005,31 @@ __global__ __launch_bounds__(kMergeWaves * 64 + 64) void k_tiny_merge(TinyMergeA
   // fallback's inputs) while the others merge keys; wave 0 reads them after the merge's
   // barriers.  Wave 0 also packs the query for the re-scoring now: its loads go out behind
   // the keys, so the round trip overlaps theirs.
-  if (wave == W) (void)query_prep_wave(a.pa, q);
-  const float* qv = a.pa.Q + size_t(q) * a.pa.pd;
+  if (wave == W) (void)query_prep_wave(pa, q);
+  const float* qv = pa.Q + size_t(q) * pa.pd;
   Int8Query p8{0, 0, ys};
-  if (wave == 0)
-    p8 = int8_query(a.sc.X8, a.sc.c8, a.sc.xlo, a.sc.xhi, a.sc.xmax, a.sc.xint, a.sc.metric,
-                    a.sc.pd, qv, ys);
-  // Every chunk holds kp keys at or below its bound, so the best kp keys of all lie at or
-  // below the smallest bound LB: keys above it are skipped.
+  if constexpr (I8) {
+    if (wave == 0)
+      p8 = int8_query(ms.sc.X8, ms.sc.c8, ms.sc.xlo, ms.sc.xhi, ms.sc.xmax, ms.sc.xint,
+                      ms.sc.metric, ms.sc.pd, qv, ys);
+  }
+  // B (every wave for itself), and the smallest chunk bound: every chunk holds kp keys at or
+  // below its bound, so the best kp keys of all lie at or below the smallest one too.  Keys
+  // above LB, the smaller of the two, are skipped.
+  float B0 = __builtin_inff();
 #pragma unroll 4
-  for (int ch = c0 + lane; ch < c1; ch += kWave) lb = fminf(lb, a.bound[size_t(q) * a.nchunks + ch]);
+  for (int ch = lane; ch < nch; ch += kWave) {
+    const uint2 f = a.part[(qc + ch) * a.kp];
+    B0 = fminf(B0, f.y != kNoId ? __uint_as_float(f.x) : __builtin_inff());
+  }
+#pragma unroll 4
+  for (int ch = c0 + lane; ch < c1; ch += kWave) lb = fminf(lb, a.bound[qc + ch]);
+  B0 = __shfl(wave_sort(B0), (a.k + 9 - 1) & (kWave - 1));
   lb = wave_min(lb);
   if (lane == 0 && keys) s_lb[wave] = lb;
   __syncthreads();
-  float LB = s_lb[0];
-  for (int w = 1; w < W; ++w) LB = fminf(LB, s_lb[w]);
+  float LB = B0;
+  for (int w = 0; w < W; ++w) LB = fminf(LB, s_lb[w]);
   // the key to beat: the (k + 9)-th (the certificate reads the key after the k + 8 scored).
   // A group stages its keys below LB and below the list's current (k + 9)-th key (read once
   // per group: it only tightens, so a stale one admits more keys, never fewer); the staged
@@ -2835,20 +3110,33 @@ __global__ __launch_bounds__(kMergeWaves * 64 + 64) void k_tiny_merge(TinyMergeA
     }
   }
   if (wave != 0) return;
-  const float shift = a.pa.shift[q], eb = a.pa.eb[q];
-  const float Qd = float(a.pa.Qd[q]);
-  const bool fits = a.pa.fit8q[q] != 0;
+  const float shift = pa.shift[q], eb = pa.eb[q];
+  // int8 keys carry the query's constant, and only queries inside the int8 bounds count;
+  // float keys need a finite bound (a non-finite query or overflowing rows have none)
+  const float Qd = I8 ? float(pa.Qd[q]) : 0.f;
+  const bool fits = I8 ? pa.fit8q[q] != 0 : eb < __builtin_inff();
   lb = __builtin_inff();
   for (int w = 0; w < W; ++w) lb = fminf(lb, s_lb[w]);
   // exact re-scoring of the best n1 keys, certificate against every unscored row
   // (rows of 128 bytes from the int8 copy: their loads issue together, where the fp32
-  // rows' 512 bytes per lane form a chain of dependent load rounds)
+  // rows' 512 bytes per lane form a chain of dependent load rounds; float rows score eight
+  // lanes a row where the order has that form)
   const int n1 = min(kWave - 1, a.k + 8);
   float d = __builtin_inff();
-  uint32_t id = kNoId;
-  if (lane < n1 && top.k.id[0] != kNoId) {
-    id = top.k.id[0];
-    d = p8.on ? int8_distance(a.sc.X8, a.sc.c8, a.sc.metric, a.sc.pd, p8, id) : a.sc(qv, id);
+  uint32_t id = lane < n1 ? top.k.id[0] : kNoId;
+  if (!I8 && ms.sc.kset == kKsetAvx512) {
+    float got = __builtin_inff();
+    group_pass(id, 0, n1, got, [&](const auto& ids, auto& dd) {
+      constexpr int R = sizeof(dd) / sizeof(float);
+      const float* xs[R];
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+        xs[i] = ms.sc.X + size_t(ms.sc.map != nullptr ? ms.sc.map[ids[i]] : ids[i]) * ms.sc.pd;
+      metric_exact_g8n<R>(ms.sc.metric, qv, xs, ms.sc.pd, dd);
+    });
+    d = got;
+  } else if (id != kNoId) {
+    d = p8.on ? int8_distance(ms.sc.X8, ms.sc.c8, ms.sc.metric, ms.sc.pd, p8, id) : ms.sc(qv, id);
   }
   WaveKeys<1> r;
   r.d[0] = d;
@@ -2860,20 +3148,14 @@ __global__ __launch_bounds__(kMergeWaves * 64 + 64) void k_tiny_merge(TinyMergeA
   // every row scored (fewer keys than n1 + 1 and no full chunk): the answer is complete
   const bool all_scored = next == __builtin_inff() && lb == __builtin_inff();
   const bool certified = fits && a.force_fallback == 0 && (dk < lower || all_scored);
+  const size_t slot = (I8 ? 0 : size_t(blockIdx.y) * pa.nq) + q;
   if (lane < a.k) {
-    a.out_ids[size_t(q) * a.k + lane] = r.id[0];
-    a.out_d[size_t(q) * a.k + lane] = r.d[0];
+    a.out_ids[slot * a.k + lane] = r.id[0];
+    a.out_d[slot * a.k + lane] = r.d[0];
   }
-  if (lane == 0) {
-    if (!certified) a.fb_list[atomicAdd(a.fb_count, 1u)] = uint32_t(q);
-    if (a.host_flag == nullptr) return;  // the re-scan is gated on the device count
-    __threadfence();
-    if (atomicAdd(a.fb_count + 1, 1u) == uint32_t(gridDim.x - 1)) {
-      // the last merge: publish the fallback count (seq written last, with release)
-      a.host_flag[1] = __hip_atomic_load(a.fb_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __threadfence_system();
-      __hip_atomic_store(a.host_flag, a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+  if (lane == 0 && !certified) {
+    const uint32_t at = atomicAdd(a.fb_count, 1u);
+    if (a.fb_list != nullptr) a.fb_list[at] = uint32_t(slot);
   }
 }
 
@@ -2927,6 +3209,26 @@ static void launch_small(hipStream_t s, int blocks, const TinyArgs& a) {
     case 128: k_small_scan<4><<<dim3(blocks), kSmallWaves * 64, 0, s>>>(a); break;
     default: k_small_scan<8><<<dim3(blocks), kSmallWaves * 64, 0, s>>>(a); break;
   }
+}
+
+// The exact re-scan of a small batch's uncertified queries: queued for every query and gated on
+// the device count, or sized from a host read of it.
+static int SmallFallback(Ctx* c, const ScanSource& src, const float* Q, size_t nq, size_t kk,
+                         const uint64_t* allow, uint32_t* out_ids, float* out_d, hipStream_t s,
+                         Workspace& W2, const uint32_t* fb_list, const uint32_t* fb_count,
+                         bool gated) {
+  // a host call reads the count with its results and runs again when it is not zero
+  if (c->opt_count != nullptr) return kOk;
+  if (gated) {
+    VDBG_RETURN_IF_ERROR(ExactScan(c, W2, src, Q, fb_list, int(nq), kk, allow, out_ids, out_d, s,
+                                   fb_count, c->fb_dev));
+    c->fb_dev_used = true;
+    return kOk;
+  }
+  uint32_t nfb = 0;
+  VDBG_RETURN_IF_ERROR(ReadWords(c, fb_count, 1, s, &nfb));
+  c->last_fallbacks += nfb;
+  return ExactScan(c, W2, src, Q, fb_list, int(nfb), kk, allow, out_ids, out_d, s);
 }
 
 static int TinyScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
@@ -2986,36 +3288,164 @@ static int TinyScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t k
     else launch_tiny<2>(s, nchunks, ta);
     VDBG_HIP(hipGetLastError());
   }
-  if (gated) {
-    TinyMergeArgs ma{pa, part, bound, nchunks, kp, int(kk), Flat8Of(*src, c->kset), out_ids,
-                     out_d, fb_list, fb_count, nullptr, 0u, c->test_fallbacks};
-    {
-      ProfScope ps(c, "select", s);
-      k_tiny_merge<<<dim3(unsigned(nq)), kMergeWaves * 64 + 64, 0, s>>>(ma);
-      VDBG_HIP(hipGetLastError());
-    }
-    VDBG_RETURN_IF_ERROR(ExactScan(c, W2, *src, Q, fb_list, int(nq), kk, allow, out_ids, out_d,
-                                   s, fb_count, c->fb_dev));
-    c->fb_dev_used = true;
-    return kOk;
+  TinyMergeArgs ma{};
+  ma.pa = pa;
+  ma.set[0].nchunks = nchunks;
+  ma.set[0].sc = Flat8Of(*src, c->kset);
+  ma.part = part;
+  ma.bound = bound;
+  ma.nchunks = nchunks;
+  ma.kp = kp;
+  ma.k = int(kk);
+  ma.out_ids = out_ids;
+  ma.out_d = out_d;
+  ma.fb_list = c->opt_count != nullptr ? nullptr : fb_list;
+  ma.fb_count = c->opt_count != nullptr ? c->opt_count : fb_count;
+  ma.force_fallback = c->test_fallbacks;
+  {
+    ProfScope ps(c, "select", s);
+    k_tiny_merge<true><<<dim3(unsigned(nq)), kMergeWaves * 64 + 64, 0, s>>>(ma);
+    VDBG_HIP(hipGetLastError());
   }
-  uint32_t nfb = 0;
-  {  // the merge publishes the fallback count through the context's host flag
-    std::lock_guard<std::mutex> g(c->flag_mu);
-    const uint32_t seq = NextFlagSeq(c);
-    TinyMergeArgs ma{pa, part, bound, nchunks, kp, int(kk), Flat8Of(*src, c->kset), out_ids,
-                     out_d, fb_list, fb_count, c->host_flag_dev, seq, c->test_fallbacks};
-    {
-      ProfScope ps(c, "select", s);
-      k_tiny_merge<<<dim3(unsigned(nq)), kMergeWaves * 64 + 64, 0, s>>>(ma);
-      VDBG_HIP(hipGetLastError());
-    }
-    VDBG_RETURN_IF_ERROR(WaitWords(c, seq, fb_count, 1, s));
-    nfb = c->host_pinned[0];
+  return SmallFallback(c, *src, Q, nq, kk, allow, out_ids, out_d, s, W2, fb_list, fb_count, gated);
+}
+
+template <int NQ>
+static void launch_rows(bool f16, unsigned blocks, size_t lds, hipStream_t s,
+                        const RowScanArgs& a) {
+  if (f16) k_row_scan<NQ, true><<<dim3(blocks), kTinyWaves * 64, lds, s>>>(a);
+  else k_row_scan<NQ, false><<<dim3(blocks), kTinyWaves * 64, lds, s>>>(a);
+}
+
+// Whether k_row_scan reads a source's fp16 copy (one part per value) instead of its fp32 rows.
+static bool RowScanF16(const Ctx* c, const ScanSource& src) {
+  return c->fp16_gemm && src.X16 != nullptr && src.x16_parts == 1;
+}
+
+// Up to 8 queries; a source the ranking GEMM serves goes there from 3 on (its cost does not
+// grow with a few queries: 200,000 x 384 rows, 1 / 2 / 3 queries take 64 / 72 / 81 us here and
+// 79 / 80 / 80 us there, 20,000 x 100 rows 35 / 39 / 45 and 47 / 47 / 48, 50,000 x 848 rows,
+// which no GEMM kernel serves, 107 us for 2 queries against 205 scored exactly).
+static bool RowScanBeatsGemm(const ScanSource& src, size_t nq) {
+  return nq <= 2 || !GemmSupported(src.pd) || src.N < 1024;
+}
+
+bool RowScanEligible(const Ctx* c, const ScanSource& src, size_t nq, size_t kk) {
+  return nq >= 1 && nq <= size_t(kRowQ) && nq * size_t(src.pd) <= size_t(kRowMaxQ) && kk >= 1 &&
+         kk <= size_t(kTinyK) && src.kind == 0 && src.N >= 1 &&
+         (RowScanF16(c, src) || (src.Xmap == nullptr && src.X != nullptr));
+}
+
+bool RowScanLike(const Ctx* c, const ScanSource& a, const ScanSource& b) {
+  return a.pd == b.pd && a.metric == b.metric && RowScanF16(c, a) == RowScanF16(c, b);
+}
+
+bool SmallBatch(const Ctx* c, const ScanSource& src, size_t nq, size_t kk) {
+  return src.N > 0 && !c->ws.fixed &&
+         ((GemmSupported(src.pd) && TinyEligible(c, src, nq, kk, c->ws)) ||
+          (RowScanEligible(c, src, nq, kk) && RowScanBeatsGemm(src, nq)));
+}
+
+int RowScan(Ctx* c, const RowSet* sets, int nsets, const float* Q, size_t nq, size_t kk,
+            uint32_t* out_ids, float* out_d, hipStream_t s, Workspace& W, uint32_t* fb_zero,
+            uint32_t** fb_list, uint32_t** fb_count) {
+  if (nsets < 1 || nsets > kRowSets) return SetError(kInternal, "row scan: 1..16 row sets");
+  const ScanSource& s0 = *sets[0].src;
+  const int pd = s0.pd;
+  const bool f16 = RowScanF16(c, s0);
+  const int kp = int(kk) + 9;
+  uint64_t total = 0;
+  for (int i = 0; i < nsets; ++i) total += sets[i].src->N;
+  RowScanArgs ra{};
+  TinyMergeArgs ma{};
+  int chunks = 0;
+  for (int i = 0; i < nsets; ++i) {
+    const ScanSource& src = *sets[i].src;
+    if (!RowScanLike(c, s0, src)) return SetError(kInternal, "row scan: unlike row sets");
+    // two blocks per CU over all sets, by their rows
+    const uint64_t want = std::max<uint64_t>(1, uint64_t(2 * c->cu_count) * src.N / total);
+    uint32_t rows = uint32_t((src.N + want - 1) / want);
+    rows = (rows + 63) / 64 * 64;
+    RowSetArgs& st = ra.set[i];
+    st.X = f16 ? static_cast<const void*>(src.X16) : static_cast<const void*>(src.X);
+    st.rn = src.rn;
+    st.allow = sets[i].allow;
+    st.N = src.N;
+    st.chunk_rows = rows;
+    st.chunk0 = chunks;
+    const int e = f16 && src.x16_approx ? src.x16_exp : 0;
+    st.f = std::ldexp(src.metric == 0 ? -2.f : -1.f, -e);
+    MergeSet& ms = ma.set[i];
+    ms.xs = src.stats;
+    ms.rmag = src.rmag;
+    ms.x16_exp = src.x16_exp;
+    ms.single16 = f16 && src.x16_approx ? 1 : 0;
+    ms.chunk0 = chunks;
+    ms.nchunks = int((src.N + rows - 1) / rows);
+    static_cast<FlatScorer&>(ms.sc) = FlatOf(src, c->kset);
+    chunks += ms.nchunks;
   }
-  c->last_fallbacks += nfb;
-  if (nfb > 0)
-    VDBG_RETURN_IF_ERROR(ExactScan(c, W2, *src, Q, fb_list, int(nfb), kk, allow, out_ids, out_d, s));
+  W.used = 0;
+  const size_t slots = nq * size_t(nsets);
+  VDBG_RETURN_IF_ERROR(W.reserve(nq * size_t(chunks) * (size_t(kp) * sizeof(uint2) + sizeof(float)) +
+                                 slots * (4 * sizeof(float) + sizeof(int) + sizeof(uint32_t) +
+                                          2 * size_t(pd) * sizeof(uint16_t)) + 16 * 256));
+  ra.part = W.take<uint2>(nq * size_t(chunks) * kp);
+  ra.bound = W.take<float>(nq * size_t(chunks));
+  float* shift = W.take<float>(slots);
+  float* eb = W.take<float>(slots);
+  int* exact = W.take<int>(slots);
+  float* Qf = W.take<float>(slots);
+  uint16_t* Q16 = W.take<uint16_t>(slots * 2 * pd);
+  int* all16 = W.take<int>(2);
+  *fb_list = W.take<uint32_t>(slots);
+  *fb_count = W.take<uint32_t>(2);
+  ra.nsets = nsets;
+  ra.Q = Q;
+  ra.nq = int(nq);
+  ra.pd = pd;
+  ra.metric = s0.metric == 0 ? 0 : 1;
+  ra.kp = kp;
+  ra.nchunks = chunks;
+  ra.fb_count = *fb_count;
+  ra.fb_zero = fb_zero;
+  c->last_gemm_bits = f16 ? 16 : 32;
+  {
+    ProfScope ps(c, "flat_gemm", s);
+    const size_t one = size_t(pd) * sizeof(float);
+    if (nq == 1) launch_rows<1>(f16, unsigned(chunks), one, s, ra);
+    else if (nq == 2) launch_rows<2>(f16, unsigned(chunks), 2 * one, s, ra);
+    else if (nq <= 4) launch_rows<4>(f16, unsigned(chunks), 4 * one, s, ra);
+    else launch_rows<8>(f16, unsigned(chunks), 8 * one, s, ra);
+    VDBG_HIP(hipGetLastError());
+  }
+  PrepArgs& pa = ma.pa;
+  pa.Q = Q;
+  pa.nq = int(nq);
+  pa.pd = pd;
+  pa.metric = s0.metric;
+  pa.shift = shift;
+  pa.eb = eb;
+  pa.exact = exact;
+  pa.Q16 = Q16;
+  pa.all16 = all16;
+  pa.Qf = Qf;
+  pa.x16_parts = 1;
+  ma.part = ra.part;
+  ma.bound = ra.bound;
+  ma.nchunks = chunks;
+  ma.kp = kp;
+  ma.k = int(kk);
+  ma.out_ids = out_ids;
+  ma.out_d = out_d;
+  ma.fb_list = c->opt_count != nullptr ? nullptr : *fb_list;
+  ma.fb_count = c->opt_count != nullptr ? c->opt_count : *fb_count;
+  ma.force_fallback = c->test_fallbacks;
+  {
+    ProfScope ps(c, "select", s);
+    k_tiny_merge<false><<<dim3(unsigned(nq), unsigned(nsets)), kMergeWaves * 64 + 64, 0, s>>>(ma);
+    VDBG_HIP(hipGetLastError());
+  }
   return kOk;
 }
 
@@ -3070,9 +3500,26 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
             Workspace* ws, Workspace* ws2) {
   Workspace& W = ws != nullptr ? *ws : c->ws;
   Workspace& W2 = ws2 != nullptr ? *ws2 : c->ws2;
-  // (the tiny path clears the call's fallback count itself, in its scan kernel)
+  // (the tiny paths clear the call's fallback count themselves, in their scan kernels)
   const bool tiny = nq > 0 && kk > 0 && kk <= 10000 && src->N > 0 &&
                     GemmSupported(src->pd) && TinyEligible(c, *src, nq, kk, W);
+  if (!tiny && !W.fixed && RowScanEligible(c, *src, nq, kk) && RowScanBeatsGemm(*src, nq)) {
+    const bool gated = c->gate_fallbacks && PlanExact(src->N, int(nq), kk).need <= kGatedExactBytes;
+    if (!gated) VDBG_RETURN_IF_ERROR(ResetFallbacks(c, s));
+    uint32_t* zero = nullptr;
+    if (gated && !c->fb_accumulate) {
+      c->last_fallbacks = 0;
+      zero = c->fb_dev;
+    }
+    c->last_gemm_gate = nullptr;
+    WsUse wuse(&W, s);
+    VDBG_RETURN_IF_ERROR(wuse.status());
+    const RowSet set{src, allow};
+    uint32_t *fb_list = nullptr, *fb_count = nullptr;
+    VDBG_RETURN_IF_ERROR(RowScan(c, &set, 1, Q, nq, kk, out_ids, out_d, s, W, zero, &fb_list,
+                                 &fb_count));
+    return SmallFallback(c, *src, Q, nq, kk, allow, out_ids, out_d, s, W2, fb_list, fb_count, gated);
+  }
   // the GEMM path clears the device count in its init kernel (no launch of its own)
   const bool main_path = !tiny && nq > 0 && kk > 0 && kk <= 240 && src->N >= 1024 &&
                          GemmSupported(src->pd);

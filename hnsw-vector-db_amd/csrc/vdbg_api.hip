@@ -70,8 +70,11 @@ int WaitWords(Ctx* c, uint32_t seq, const uint32_t* dev, int n, hipStream_t s) {
 
 // ------------------------------------------------------------ host staging
 
-// Inputs: the device reads the mapped pinned block (16-byte vectors, grid-strided).
-__global__ void k_stage_in(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t n16) {
+// Inputs: the device reads the mapped pinned block (16-byte vectors, grid-strided); the call's
+// count of uncertified answers (Ctx::opt_count) starts at zero.
+__global__ void k_stage_in(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t n16,
+                           uint32_t* __restrict__ zero) {
+  if (blockIdx.x == 0 && threadIdx.x < 4) zero[threadIdx.x] = 0;
   const size_t step = size_t(gridDim.x) * blockDim.x;
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n16; i += step)
     dst[i] = src[i];
@@ -80,9 +83,9 @@ __global__ void k_stage_in(const uint4* __restrict__ src, uint4* __restrict__ ds
 // Results: every block writes its share into the mapped pinned block and fences at system
 // scope; the last block to finish (a device counter, reset by that block) raises the flag.
 struct StageOutArgs {
-  const uint4* src[3];
-  uint4* dst[3];
-  size_t n16[3];
+  const uint4* src[4];
+  uint4* dst[4];
+  size_t n16[4];
   int n;
   uint32_t* counter;
   uint32_t* flag;
@@ -164,7 +167,8 @@ int StageIn(Ctx* c, const void* const* src, const size_t* bytes, int nin, size_t
   const size_t n16 = in / 16;
   const unsigned blocks = unsigned(std::min<size_t>(256, (n16 + 255) / 256));
   k_stage_in<<<blocks, 256, 0, s>>>(reinterpret_cast<const uint4*>(c->stage_h_dev),
-                                    reinterpret_cast<uint4*>(base), n16);
+                                    reinterpret_cast<uint4*>(base), n16,
+                                    reinterpret_cast<uint32_t*>(c->stage_d + kStageOptWord));
   VDBG_HIP(hipGetLastError());
   *dev = base;
   return kOk;
@@ -172,7 +176,7 @@ int StageIn(Ctx* c, const void* const* src, const size_t* bytes, int nin, size_t
 
 int StageOut(Ctx* c, const uint8_t* const* src, const size_t* bytes, void* const* dst, int nout,
              hipStream_t s) {
-  if (nout < 1 || nout > 3) return SetError(kInternal, "StageOut: 1 to 3 regions");
+  if (nout < 1 || nout > 4) return SetError(kInternal, "StageOut: 1 to 4 regions");
   // the results land at the start of the pinned block (the inputs there have been read: the
   // copy-in kernel ran before everything queued after it)
   StageOutArgs a{};

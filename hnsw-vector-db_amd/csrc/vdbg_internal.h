@@ -128,6 +128,11 @@ struct Ctx {
   std::vector<uint8_t*> stage_h_retired;
   uint8_t* stage_d = nullptr;
   size_t stage_d_cap = 0;
+  // set while a host call runs a small batch (StageRegions): its merges only count uncertified
+  // answers here (a word of the device block, zeroed by the copy-in kernel), no re-scan is
+  // queued, and the host, which reads the word with the results, runs the call again without
+  // it when it is not zero
+  uint32_t* opt_count = nullptr;
   std::mutex flag_mu;  // one readback through host_flag at a time (scan lanes may run on
                        // worker threads of one call)
   std::mutex prof_mu;  // guards pending / free_events against those threads
@@ -378,6 +383,23 @@ int MakeRows8Split(Ctx* c, hipStream_t s, const float* rows, size_t n, size_t pd
 int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
             const uint64_t* allow, uint32_t* out_ids, float* out_d, hipStream_t s,
             Workspace* ws = nullptr, Workspace* ws2 = nullptr);
+// At most 8 queries, kk <= 48, over up to kRowSets row sets at once (k_row_scan and its merge):
+// out [set][nq][kk]; *fb_list / *fb_count (in W) receive the uncertified answers, set * nq + q
+// each, which the caller re-scans.  Sets share pd, metric and the form their rows are read in.
+constexpr int kRowSets = 16;
+struct RowSet {
+  const ScanSource* src;
+  const uint64_t* allow;  // nullable, device words
+};
+bool RowScanEligible(const Ctx* c, const ScanSource& src, size_t nq, size_t kk);
+// Whether two sources can be sets of one RowScan.
+bool RowScanLike(const Ctx* c, const ScanSource& a, const ScanSource& b);
+// Whether RunScan answers the batch from one pass over the rows (k_tiny_scan, k_small_scan,
+// k_row_scan), testing a filter row by row.
+bool SmallBatch(const Ctx* c, const ScanSource& src, size_t nq, size_t kk);
+int RowScan(Ctx* c, const RowSet* sets, int nsets, const float* Q, size_t nq, size_t kk,
+            uint32_t* out_ids, float* out_d, hipStream_t s, Workspace& W, uint32_t* fb_zero,
+            uint32_t** fb_list, uint32_t** fb_count);
 // Top-kk by the source's exact score without a ranking GEMM: every allowed row scored, wave
 // top-k per row split then a merge (kk <= 240), or a segmented sort (kk up to 10,000).
 int ScoreScan(Ctx* c, const ScanSource& src, const float* Q, size_t nq, size_t kk,
@@ -459,6 +481,10 @@ struct PrepPending {
   PrepPending& operator=(const PrepPending&) = delete;
   ~PrepPending();
 };
+// (status: nq device words of the caller's, 0 ok, 1 non-finite, 2 a zero query under cosine)
+int LaunchPrepare(Ctx* c, const float* raw, size_t nq, size_t dim, size_t pd, int metric,
+                  float* out, int* status, hipStream_t s);
+int PrepareStatusError(const int* status, size_t nq);
 int PrepareQueriesLaunch(Ctx* c, const float* raw, size_t nq, size_t dim, size_t pd, int metric,
                          float* out, hipStream_t s, PrepPending* pp);
 int PrepareQueriesCheck(PrepPending* pp);
@@ -529,6 +555,18 @@ inline int ScorePd(const ScanSource& src) { return src.kind == 2 ? src.pq_m * 25
 // the pinned block and then raises host_flag, which the host polls (no allocation, no
 // pageable copy and no stream synchronisation per call).  Regions start on 256-byte bounds.
 constexpr size_t kStageAlign = 256;
+constexpr size_t kStageOptWord = 128;  // Ctx::opt_count's place in the device block's header
+// Host calls of at most this many queries go without queued re-scans (the two gated launches
+// cost a lone query 9 of its 82 us; one uncertified query of the batch costs it a second run).
+constexpr size_t kOptQueries = 32;
+// Arms Ctx::opt_count for one host call's queued work.
+struct OptCount {
+  Ctx* c;
+  explicit OptCount(Ctx* ctx) : c(ctx) {
+    c->opt_count = reinterpret_cast<uint32_t*>(c->stage_d + kStageOptWord);
+  }
+  ~OptCount() { c->opt_count = nullptr; }
+};
 inline size_t StageRound(size_t b) { return (b + kStageAlign - 1) & ~(kStageAlign - 1); }
 // The bytes an input region of b bytes takes: at least one zero word past its end.
 inline size_t StageSpan(size_t b) { return StageRound(b + 8); }
@@ -537,7 +575,7 @@ inline size_t StageSpan(size_t b) { return StageRound(b + 8); }
 // *dev receives the device block's base.
 int StageIn(Ctx* c, const void* const* src, const size_t* bytes, int nin, size_t out,
             hipStream_t s, uint8_t** dev);
-// Copies the nout <= 3 device regions src[i] (inside the device block) to the host pointers
+// Copies the nout <= 4 device regions src[i] (inside the device block) to the host pointers
 // dst[i] after the work queued on s, through the pinned block.
 int StageOut(Ctx* c, const uint8_t* const* src, const size_t* bytes, void* const* dst, int nout,
              hipStream_t s);
@@ -565,13 +603,26 @@ inline int StageRegions(Ctx* c, const float* queries, size_t qb, const void* ext
   float* dd = reinterpret_cast<float*>(base + in_end + StageRound(ob));
   uint64_t* ddc = dist_comps ? reinterpret_cast<uint64_t*>(base + in_end + 2 * StageRound(ob))
                              : nullptr;
-  VDBG_RETURN_IF_ERROR(fn(dq, dx, di, dd, ddc, s));
-  const uint8_t* osrc[3] = {reinterpret_cast<const uint8_t*>(di),
+  const uint8_t* osrc[4] = {reinterpret_cast<const uint8_t*>(di),
                             reinterpret_cast<const uint8_t*>(dd),
                             reinterpret_cast<const uint8_t*>(ddc)};
-  const size_t obytes[3] = {ob, ob, cb};
-  void* const odst[3] = {out_ids, out_dists, dist_comps};
-  return StageOut(c, osrc, obytes, odst, dist_comps ? 3 : 2, s);
+  size_t obytes[4] = {ob, ob, cb};
+  void* odst[4] = {out_ids, out_dists, dist_comps};
+  int nout = dist_comps ? 3 : 2;
+  if (nq <= kOptQueries && c->gate_fallbacks) {
+    uint32_t uncertified[4] = {};
+    {
+      OptCount armed(c);
+      VDBG_RETURN_IF_ERROR(fn(dq, dx, di, dd, ddc, s));
+    }
+    osrc[nout] = c->stage_d + kStageOptWord;
+    obytes[nout] = sizeof(uncertified);
+    odst[nout] = uncertified;
+    VDBG_RETURN_IF_ERROR(StageOut(c, osrc, obytes, odst, nout + 1, s));
+    if (uncertified[0] == 0) return kOk;
+  }
+  VDBG_RETURN_IF_ERROR(fn(dq, dx, di, dd, ddc, s));
+  return StageOut(c, osrc, obytes, odst, nout, s);
 }
 
 // Queries of pd floats over an n_rows source with optional dense allow words (ceil(n/64)
