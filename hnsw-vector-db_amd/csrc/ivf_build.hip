@@ -183,9 +183,10 @@ __global__ __launch_bounds__(256) void k_assign_wide(const float* __restrict__ x
   if (dist != nullptr) dist[p] = best;
 }
 
-__global__ void k_iota(uint32_t* v, uint32_t n) {
+// v[i] = i mod per (per: the points of one set)
+__global__ void k_iota(uint32_t* v, uint32_t n, uint32_t per) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) v[i] = i;
+  if (i < n) v[i] = i % per;
 }
 
 __global__ void k_histogram(const uint32_t* __restrict__ a, uint32_t n, uint32_t* __restrict__ counts) {
@@ -193,18 +194,372 @@ __global__ void k_histogram(const uint32_t* __restrict__ a, uint32_t n, uint32_t
   if (i < n) atomicAdd(&counts[a[i]], 1u);
 }
 
+// off[c] = the first place of a cluster id >= c among the sorted ids (c in [0, k]).
+__global__ void k_offsets(const uint32_t* __restrict__ sorted, uint32_t n, uint32_t k,
+                          uint32_t* __restrict__ off) {
+  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c > k) return;
+  uint32_t lo = 0, hi = n;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (sorted[mid] < c) lo = mid + 1; else hi = mid;
+  }
+  off[c] = lo;
+}
+
+// AssignNearest with L2SqAny of several point sets at once (grid.y), one thread per point, a
+// set's centroids in LDS: key = set * k + the first centroid with the smallest distance.
+template <int D>
+__global__ __launch_bounds__(256) void k_assign_sets(const float* __restrict__ x, uint32_t n,
+                                                     int d, const float* __restrict__ cen, int k,
+                                                     uint32_t* __restrict__ key) {
+  extern __shared__ float cs[];
+  const size_t set = blockIdx.y;
+  for (int i = threadIdx.x; i < k * d; i += blockDim.x) cs[i] = cen[set * k * d + i];
+  __syncthreads();
+  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  const float* xp = x + (set * n + p) * d;
+  float xr[D > 0 ? D : 64];
+  const int dd = D > 0 ? D : d;
+  for (int i = 0; i < dd; ++i) xr[i] = xp[i];
+  float best = __builtin_inff();
+  uint32_t arg = 0;
+#pragma unroll 2
+  for (int c = 0; c < k; ++c) {
+    const float v = l2any_fixed<D>(xr, cs + c * dd, dd);
+    if (v < best) {
+      best = v;
+      arg = uint32_t(c);
+    }
+  }
+  key[set * n + p] = uint32_t(set * k) + arg;
+}
+
+// k-means++ (kmeans.cc:92-120) of several point sets of n points at once, two launches a pick:
+// k_pp_dist lowers every point's distance to its nearest pick, k_pp_pick (one block a set)
+// finds the next pick as the reference's loop does.  The host has drawn each set's first pick
+// and its canonical variates r (t = r total is what uniform_real_distribution(0, total) gives).
+//
+// That loop adds the n floats into one double in index order, and both the total and the pick
+// depend on every rounding of it.  While the sum stays in one binade [2^e, 2^(e+1)) its quantum
+// is u = 2^(e-52) and adding x adds exactly u rint(x / u), whatever the sum is, unless x / u
+// lies halfway between integers (the even neighbour then depends on the sum) or the sum
+// leaves the binade.  So a tile of points is summed in parallel in units of u (integers below
+// 2^53, exact in double and associative); at the first point that ties or leaves the binade
+// the block adds that point as the reference does and goes on behind it with the new quantum.
+// A sum of 65,536 squares crosses about 16 binades, six of them in the first 64 points, which
+// every thread adds one by one.  Every tile start and every point added by itself is a mark
+// (position, sum), so the pick is searched in one stretch between marks.
+//
+// fail: a set with a non-finite distance, a total that is not positive, or more marks than
+// are kept; the host then runs the reference's loop itself.
+// Bound: one block a set, the latency of about 27 block scans a pick (66 us; 132 us with 1,024
+// threads of four points, whose scans cross 16 waves).  16 sets of 65,536 points of 8 dims, 255
+// picks each: 18.6 ms, where the host's loop took 700 ms.
+constexpr int kPpThreads = 256, kPpPer = 16, kPpTile = kPpThreads * kPpPer, kPpMarks = 512;
+constexpr int kPpHead = 64;
+struct PpArgs {
+  const float* x;         // set j's points at x + j xset, `stride` floats apart
+  size_t xset;
+  uint32_t n, n4;         // n4: mind's set stride (a multiple of 4)
+  int d, stride, k, q, simd, kset;
+  const uint32_t* first;  // [sets]
+  const double* r;        // [sets][k - 1]
+  float* mind;            // [sets][n4]
+  float* cen;             // [sets][k][d]
+  int* fail;              // [sets]
+};
+
+// Distances to pick q - 1 (the first pick itself is written here, q = 1); grid.y the set.
+template <int D>
+__global__ __launch_bounds__(256) void k_pp_dist(PpArgs a) {
+  const int d = D > 0 ? D : a.d;
+  const size_t set = blockIdx.y;
+  const float* x = a.x + set * a.xset;
+  const float* last =
+      a.q == 1 ? x + size_t(a.first[set]) * a.stride : a.cen + (set * a.k + a.q - 1) * d;
+  if (a.q == 1 && blockIdx.x == 0)
+    for (int i = threadIdx.x; i < d; i += blockDim.x) a.cen[set * a.k * d + i] = last[i];
+  float* mind = a.mind + set * a.n4;
+  auto put = [&](uint32_t p, float dist) {
+    const float old = a.q == 1 ? __builtin_inff() : mind[p];
+    const float v = dist < old ? dist : old;
+    mind[p] = v;
+    if (!(v < __builtin_inff())) a.fail[set] = 1;
+  };
+  if (D == 0 && a.simd && a.kset == kKsetAvx512) {  // eight lanes a point, two points a group
+    const uint32_t p = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16 + (lane_id() >> 3) * 2;
+    const float* const xs[2] = {x + size_t(min(p, a.n - 1)) * a.stride,
+                                x + size_t(min(p + 1, a.n - 1)) * a.stride};
+    float v[2];
+    metric_exact_g8n<2>(0, last, xs, d, v);
+    if ((lane_id() & 7) < 2) {
+      const uint32_t pp = p + (lane_id() & 1);
+      if (pp < a.n) put(pp, (lane_id() & 1) ? v[1] : v[0]);
+    }
+    return;
+  }
+  const uint32_t p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= a.n) return;
+  float c[D > 0 ? D : 1], xr[D > 0 ? D : 1];
+  if constexpr (D > 0) {
+    for (int i = 0; i < D; ++i) {
+      c[i] = last[i];
+      xr[i] = x[size_t(p) * a.stride + i];
+    }
+    put(p, l2any_fixed<D>(xr, c, D));
+  } else {
+    put(p, a.simd ? metric_exact_k(a.kset, 0, x + size_t(p) * a.stride, last, d)
+                  : l2sq_any(x + size_t(p) * a.stride, last, d));
+  }
+}
+
+// v of lane - n (0 below it) for n = 1, 2, 4, 8 inside the lane's row of 16 (DPP row_shr).
+template <int N>
+__device__ __forceinline__ double row_shr(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const int lo = __builtin_amdgcn_update_dpp(0, int(uint32_t(b)), 0x110 + N, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, int(uint32_t(b >> 32)), 0x110 + N, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, uint64_t(uint32_t(lo)) | (uint64_t(uint32_t(hi)) << 32));
+}
+__device__ __forceinline__ double lane_of(double v, int l) {  // v of lane l (a constant)
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(
+      double, uint64_t(uint32_t(__builtin_amdgcn_readlane(int(uint32_t(b)), l))) |
+                  (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(uint32_t(b >> 32)), l))) << 32));
+}
+
+__global__ __launch_bounds__(kPpThreads) void k_pp_pick(PpArgs a) {
+  constexpr int W = kPpThreads / 64;
+  __shared__ double s_wave[W];
+  __shared__ int s_alone[W];
+  __shared__ float s_head[kPpHead];
+  __shared__ uint32_t s_hit;         // first point of the tile that ties or leaves the binade
+  __shared__ double s_before, s_at;  // the sum (in u) before it, and its value
+  __shared__ uint32_t s_pos[kPpMarks];
+  __shared__ double s_acc[kPpMarks];
+  __shared__ uint32_t s_pick;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = lane_id();
+  const size_t set = blockIdx.x;
+  if (a.fail[set] != 0) return;  // (block-uniform: written by earlier launches only)
+  const float* mind = a.mind + set * a.n4;
+  const double kTop = 9007199254740992.0;  // 2^53
+  // the units of value v under scale = 1 / u, and whether it must be added by itself
+  auto units = [&](float v, double scale, bool zero, bool& alone) {
+    const double y = double(v) * scale, r = rint(y);
+    alone = zero ? v != 0.f : fabs(y - r) == 0.5;
+    return zero ? 0.0 : r;
+  };
+  // exclusive block prefix of v, and the block's sum (each exact up to the first point that
+  // leaves the binade, and at least 2^53 behind it)
+  // (any: whether some thread passed alone)
+  auto block_scan = [&](double v, bool alone, double& sum, bool& any) {
+    double incl = v;  // inside each row of 16 lanes
+    incl += row_shr<1>(incl);
+    incl += row_shr<2>(incl);
+    incl += row_shr<4>(incl);
+    incl += row_shr<8>(incl);
+    const double t0 = lane_of(incl, 15), t1 = t0 + lane_of(incl, 31), t2 = t1 + lane_of(incl, 47);
+    const double before = lane < 16 ? 0.0 : lane < 32 ? t0 : lane < 48 ? t1 : t2;
+    const double excl = before + row_shr<1>(incl);
+    __syncthreads();  // (s_wave's last readers are done)
+    const bool one = __ballot(alone) != 0;
+    if (lane == kWave - 1) {
+      s_wave[wave] = before + incl;
+      s_alone[wave] = one ? 1 : 0;
+    }
+    __syncthreads();
+    double base = 0.0;
+    sum = 0.0;
+    any = false;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const double x = s_wave[w];
+      base += w < wave ? x : 0.0;
+      sum += x;
+      any |= s_alone[w] != 0;
+    }
+    return base + excl;
+  };
+  double acc = 0.0;
+  int marks = 0;
+  auto mark = [&](uint32_t pos) {
+    if (tid == 0 && marks < kPpMarks) {
+      s_pos[marks] = pos;
+      s_acc[marks] = acc;
+    }
+    ++marks;
+  };
+  auto load = [&](uint32_t p0, float (&v)[kPpPer]) {
+#pragma unroll
+    for (int e = 0; e < kPpPer; e += 4) {
+      float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (p0 + e < a.n4) f = *reinterpret_cast<const float4*>(mind + p0 + e);
+      v[e] = f.x;
+      v[e + 1] = f.y;
+      v[e + 2] = f.z;
+      v[e + 3] = f.w;
+    }
+  };
+  // the scale of the binade sum `from` lies in (1 / u), and u
+  auto quantum = [&](double from, double& scale, double& u) {
+    int ex = 0;
+    (void)frexp(from, &ex);
+    scale = ldexp(1.0, 53 - ex);
+    u = ldexp(1.0, ex - 53);
+  };
+  // the head's points one by one (the sum would leave its binade at every second of them)
+  if (tid < kPpHead) s_head[tid] = mind[tid];
+  float nxt[kPpPer];
+  load(tid * kPpPer, nxt);
+  mark(0);
+  __syncthreads();
+#pragma unroll 16
+  for (int i = 0; i < kPpHead; ++i) acc += double(s_head[i]);
+  for (uint32_t base = 0; base < a.n; base += kPpTile) {
+    const uint32_t p0 = base + tid * kPpPer;
+    float v[kPpPer];
+#pragma unroll
+    for (int e = 0; e < kPpPer; ++e) v[e] = nxt[e];  // (zero past the set's points)
+    load(p0 + kPpTile, nxt);  // the next tile's, while this one is summed
+    uint32_t pos = max(base, uint32_t(kPpHead));  // points before it are in acc
+    mark(pos);
+    for (;;) {  // (pos grows every round: at most kPpTile rounds)
+      const bool zero = acc == 0.0;
+      double scale, u;
+      quantum(acc, scale, u);
+      const double A = acc * scale;
+      double mine = 0.0;
+      bool alone = false;
+#pragma unroll
+      for (int e = 0; e < kPpPer; ++e) {
+        bool al;
+        const double y = units(v[e], scale, zero, al);
+        const bool in = p0 + e >= pos;
+        mine += in ? y : 0.0;
+        alone |= al && in;
+      }
+      if (tid == 0) s_hit = 0xffffffffu;
+      double sum;
+      bool any;
+      double run = A + block_scan(mine, alone, sum, any);
+      if (!any && A + sum < kTop) {  // (block-uniform)
+        acc = (A + sum) * u;
+        break;
+      }
+      if (alone || run + mine >= kTop) {
+#pragma unroll
+        for (int e = 0; e < kPpPer; ++e) {
+          if (p0 + e < pos) continue;
+          bool al;
+          const double y = units(v[e], scale, zero, al);
+          if (al || run + y >= kTop) {
+            atomicMin(&s_hit, p0 + e);
+            break;
+          }
+          run += y;
+        }
+      }
+      __syncthreads();
+      const uint32_t hit = s_hit;
+      if (hit >= p0 && hit < p0 + kPpPer) {  // (run stopped in front of it)
+        s_before = run;
+#pragma unroll
+        for (int e = 0; e < kPpPer; ++e)
+          if (hit == p0 + e) s_at = double(v[e]);
+      }
+      __syncthreads();
+      acc = s_before * u + s_at;
+      pos = hit + 1;
+      mark(pos);
+      if (marks > kPpMarks) break;
+    }
+    if (marks > kPpMarks) break;
+  }
+  __syncthreads();
+  if (marks > kPpMarks || !(acc > 0.0) || !(acc < double(__builtin_inff()))) {
+    if (tid == 0) a.fail[set] = 1;
+    return;  // (block-uniform)
+  }
+  // the first point whose sum reaches t, in the stretch behind the last mark below t
+  const double t = a.r[set * (a.k - 1) + (a.q - 1)] * acc;
+  if (tid == 0) s_pick = 0xffffffffu;
+  int mk = 0;
+  while (mk + 1 < marks && s_acc[mk + 1] < t) ++mk;
+  const uint32_t lo = s_pos[mk], hi = mk + 1 < marks ? s_pos[mk + 1] : a.n;
+  if (mk == 0) {  // in the head
+    double run = 0.0;
+    uint32_t at = kPpHead - 1;
+    for (int i = 0; i < kPpHead; ++i) {
+      run += double(s_head[i]);
+      if (run >= t) {
+        at = uint32_t(i);
+        break;
+      }
+    }
+    __syncthreads();
+    if (tid == 0) s_pick = at;
+  } else {
+    const double from = s_acc[mk];
+    const bool zero = from == 0.0;
+    double scale, u;
+    quantum(from, scale, u);
+    // (a stretch lies inside one tile; one that a point by itself ends holds that point last)
+    const uint32_t p0 = lo / kPpTile * kPpTile + tid * kPpPer;
+    float v[kPpPer];
+    load(p0, v);
+    double mine = 0.0;
+    bool al;
+#pragma unroll
+    for (int e = 0; e < kPpPer; ++e) {
+      if (p0 + e < lo || p0 + e >= hi) v[e] = 0.f;
+      mine += units(v[e], scale, zero, al);
+    }
+    double sum;
+    bool any;
+    double run = from * scale + block_scan(mine, false, sum, any);
+#pragma unroll
+    for (int e = 0; e < kPpPer; ++e) {
+      run += units(v[e], scale, zero, al);
+      if (p0 + e >= lo && p0 + e < hi && run * u >= t) {
+        atomicMin(&s_pick, p0 + e);
+        break;
+      }
+    }
+  }
+  __syncthreads();
+  // none inside: the point by itself that ends the stretch reached t (behind the last mark
+  // the reference's loop ends on the last point)
+  const uint32_t pick = s_pick != 0xffffffffu ? s_pick : hi - 1;
+  const float* xp = a.x + set * a.xset + size_t(pick) * a.stride;
+  for (int i = tid; i < a.d; i += kPpThreads) a.cen[(set * a.k + a.q) * a.d + i] = xp[i];
+}
+
 // Centroid update (kmeans.cc:146-158): fp64 sums of each cluster's members in row order,
-// float(sum * (1.0 / count)) for non-empty clusters.  grid = clusters, threads over dims.
-__global__ void k_centroid_update(const float* __restrict__ x, int d, int stride,
-                                  const uint32_t* __restrict__ order, const uint32_t* __restrict__ off,
-                                  float* __restrict__ cen) {
+// float(sum * (1.0 / count)) for non-empty clusters.  grid = clusters, threads over dims;
+// clusters come in sets of `per` (a set per point set, xset floats apart).  Bound: the latency
+// of one chain of dependent adds per (cluster, dim); with one member's load at a time behind
+// each add it took 100 us for 256 clusters of 256 points.
+__global__ void k_centroid_update(const float* __restrict__ x, int d, int stride, int per,
+                                  size_t xset, const uint32_t* __restrict__ order,
+                                  const uint32_t* __restrict__ off, float* __restrict__ cen) {
   const int c = blockIdx.x;
   const uint32_t b = off[c], e = off[c + 1];
   if (b == e) return;
   const double inv = 1.0 / double(e - b);
+  x += size_t(c / per) * xset;
   for (int j = threadIdx.x; j < d; j += blockDim.x) {
     double s = 0.0;
-    for (uint32_t t = b; t < e; ++t) s += double(x[size_t(order[t]) * stride + j]);
+    uint32_t t = b;
+    for (; t + 16 <= e; t += 16) {  // sixteen members' loads in flight, added in row order
+      float v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = x[size_t(order[t + i]) * stride + j];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s += double(v[i]);
+    }
+    for (; t < e; ++t) s += double(x[size_t(order[t]) * stride + j]);
     cen[size_t(c) * d + j] = float(s * inv);
   }
 }
@@ -307,6 +662,86 @@ struct KMeansInfo {
   size_t train_points = 0, empty_reseeds = 0, iterations = 0;
 };
 
+// k-means++ initialisation of `sets` point sets on the device (k_pp_dist, k_pp_pick): x + j xset
+// holds set j's n points `stride` apart, dcen receives [sets][k][d], and each set's generator is
+// advanced by the draws the reference makes.  *failed: a set needs the host's loop (no
+// generator is advanced then).
+int KMeansPPGpu(Ctx* c, const float* x, size_t xset, size_t sets, size_t n, size_t d, size_t stride,
+                size_t k, std::vector<std::mt19937_64>* rngs, float* dcen, bool* failed,
+                hipStream_t s) {
+  std::vector<std::mt19937_64> drawn = *rngs;
+  std::vector<uint32_t> first(sets);
+  std::vector<double> r(sets * std::max<size_t>(1, k - 1));
+  for (size_t j = 0; j < sets; ++j) {
+    std::uniform_int_distribution<size_t> u0(0, n - 1);
+    first[j] = uint32_t(u0(drawn[j]));
+    std::uniform_real_distribution<double> u(0.0, 1.0);
+    for (size_t q = 0; q + 1 < k; ++q) r[j * (k - 1) + q] = u(drawn[j]);
+  }
+  const size_t n4 = (n + 3) / 4 * 4;
+  DevBuf df, dr, dm, dfail;
+  VDBG_RETURN_IF_ERROR(Alloc(&df, sets * 4, s));
+  VDBG_RETURN_IF_ERROR(Alloc(&dr, r.size() * 8, s));
+  VDBG_RETURN_IF_ERROR(Alloc(&dm, sets * n4 * 4, s));
+  VDBG_RETURN_IF_ERROR(Alloc(&dfail, sets * 4, s));
+  VDBG_HIP(hipMemcpyAsync(df.p, first.data(), sets * 4, hipMemcpyHostToDevice, s));
+  VDBG_HIP(hipMemcpyAsync(dr.p, r.data(), r.size() * 8, hipMemcpyHostToDevice, s));
+  VDBG_RETURN_IF_ERROR(Fill32(dfail.p, 0, sets, s));
+  VDBG_RETURN_IF_ERROR(Fill32(dm.p, 0, sets * n4, s));  // (the padding after each set's points)
+  PpArgs a{x, xset, uint32_t(n), uint32_t(n4), int(d), int(stride), int(k), 1,
+           SimdL2(d, stride) ? 1 : 0, c->kset, df.get<uint32_t>(), dr.get<double>(),
+           dm.get<float>(), dcen, dfail.get<int>()};
+  const bool group = a.simd && c->kset == kKsetAvx512;
+  const dim3 grid(unsigned(group ? (n + 63) / 64 : (n + 255) / 256), unsigned(sets));
+  {
+    ProfScope ps(c, "kmeanspp", s);
+    for (size_t q = 1; q < std::max<size_t>(k, 2); ++q) {
+      a.q = int(q);
+      if (a.simd) k_pp_dist<0><<<grid, 256, 0, s>>>(a);
+      else if (d == 4) k_pp_dist<4><<<grid, 256, 0, s>>>(a);
+      else if (d == 8) k_pp_dist<8><<<grid, 256, 0, s>>>(a);
+      else if (d == 12) k_pp_dist<12><<<grid, 256, 0, s>>>(a);
+      else k_pp_dist<0><<<grid, 256, 0, s>>>(a);
+      if (q < k) k_pp_pick<<<dim3(unsigned(sets)), kPpThreads, 0, s>>>(a);
+    }
+    VDBG_HIP(hipGetLastError());
+  }
+  std::vector<int> fail(sets);
+  VDBG_HIP(hipMemcpyAsync(fail.data(), dfail.p, sets * 4, hipMemcpyDeviceToHost, s));
+  VDBG_HIP(hipStreamSynchronize(s));
+  *failed = std::any_of(fail.begin(), fail.end(), [](int f) { return f != 0; });
+  if (!*failed) *rngs = std::move(drawn);
+  return kOk;
+}
+// The device pass takes two launches a pick, the host's loop about 10 ns a point and pick; one
+// block's marks cover kPpMarks tiles at most.
+bool KMeansPPOnGpu(size_t n) { return n >= 4096 && n <= size_t(kPpTile) * (kPpMarks / 2); }
+
+// The empty clusters of one iteration (kmeans.cc:159-172): the largest split in two with a
+// symmetric perturbation.  cen: k x d on the host.
+void SplitLargest(float* cen, size_t k, size_t d, const uint32_t* cnt, std::mt19937_64& rng,
+                  size_t* reseeds) {
+  constexpr float kEps = 1.0f / 1024.0f;
+  std::vector<size_t> counts(cnt, cnt + k);
+  for (size_t q = 0; q < k; ++q) {
+    if (counts[q] != 0) continue;
+    const size_t big =
+        static_cast<size_t>(std::max_element(counts.begin(), counts.end()) - counts.begin());
+    std::uniform_real_distribution<float> noise(-1.f, 1.f);
+    for (size_t j = 0; j < d; ++j) {
+      const float v = cen[big * d + j];
+      const float delta = kEps * (std::fabs(v) + 1e-3f) * noise(rng);
+      cen[q * d + j] = v + delta;
+      cen[big * d + j] = v - delta;
+    }
+    counts[q] = counts[big] / 2;
+    counts[big] -= counts[q];
+    ++*reseeds;
+  }
+}
+
+unsigned UpdateThreads(size_t d) { return unsigned(std::min<size_t>(256, (d + 63) / 64 * 64)); }
+
 // KMeans (kmeans.cc:57-174) over n device rows of d floats at `stride`.
 int KMeansGpu(Ctx* c, const float* data, size_t n, size_t d, size_t stride, size_t k,
               const KMeansOpts& o, std::vector<float>* centroids, KMeansInfo* info, hipStream_t s) {
@@ -361,7 +796,19 @@ int KMeansGpu(Ctx* c, const float* data, size_t n, size_t d, size_t stride, size
   // Initialisation.
   float* cen = centroids->data();
   const bool use_pp = o.kmeanspp && static_cast<double>(k) * static_cast<double>(m) <= 2.0e7;
-  if (use_pp) {
+  bool host_pp = use_pp;
+  if (use_pp && KMeansPPOnGpu(m)) {
+    DevBuf dc;
+    VDBG_RETURN_IF_ERROR(Alloc(&dc, k * d * sizeof(float), s));
+    std::vector<std::mt19937_64> rngs{rng};
+    VDBG_RETURN_IF_ERROR(KMeansPPGpu(c, x, 0, 1, m, d, xs, k, &rngs, dc.get<float>(), &host_pp, s));
+    if (!host_pp) {
+      rng = rngs[0];
+      VDBG_HIP(hipMemcpyAsync(cen, dc.p, k * d * sizeof(float), hipMemcpyDeviceToHost, s));
+      VDBG_HIP(hipStreamSynchronize(s));
+    }
+  }
+  if (host_pp) {
     std::vector<float> xh(m * xs);
     VDBG_HIP(hipMemcpyAsync(xh.data(), x, m * xs * sizeof(float), hipMemcpyDeviceToHost, s));
     VDBG_HIP(hipStreamSynchronize(s));
@@ -390,7 +837,7 @@ int KMeansGpu(Ctx* c, const float* data, size_t n, size_t d, size_t stride, size
       }
       std::memcpy(cen + q * d, xh.data() + pick * xs, d * sizeof(float));
     }
-  } else {
+  } else if (!use_pp) {
     std::vector<size_t> idx(m);
     std::iota(idx.begin(), idx.end(), 0);
     std::vector<uint32_t> rows(k);
@@ -411,14 +858,13 @@ int KMeansGpu(Ctx* c, const float* data, size_t n, size_t d, size_t stride, size
   }
 
   // Lloyd iterations.
-  DevBuf dcen, assign, dist, keys_out, vals_in, vals_out, counts, off, tmp;
+  DevBuf dcen, assign, dist, keys_out, vals_in, vals_out, off, tmp;
   VDBG_RETURN_IF_ERROR(Alloc(&dcen, k * d * sizeof(float), s));
   VDBG_RETURN_IF_ERROR(Alloc(&assign, m * 4, s));
   VDBG_RETURN_IF_ERROR(Alloc(&dist, m * 4, s));
   VDBG_RETURN_IF_ERROR(Alloc(&keys_out, m * 4, s));
   VDBG_RETURN_IF_ERROR(Alloc(&vals_in, m * 4, s));
   VDBG_RETURN_IF_ERROR(Alloc(&vals_out, m * 4, s));
-  VDBG_RETURN_IF_ERROR(Alloc(&counts, k * 4, s));
   VDBG_RETURN_IF_ERROR(Alloc(&off, (k + 1) * 4, s));
   int end_bit = 1;
   while ((size_t(1) << end_bit) < k) ++end_bit;
@@ -427,56 +873,114 @@ int KMeansGpu(Ctx* c, const float* data, size_t n, size_t d, size_t stride, size
                                               keys_out.get<uint32_t>(), vals_in.get<uint32_t>(),
                                               vals_out.get<uint32_t>(), int(m), 0, end_bit, s));
   VDBG_RETURN_IF_ERROR(Alloc(&tmp, tmp_bytes, s));
-  k_iota<<<dim3(unsigned((m + 255) / 256)), 256, 0, s>>>(vals_in.get<uint32_t>(), uint32_t(m));
+  k_iota<<<dim3(unsigned((m + 255) / 256)), 256, 0, s>>>(vals_in.get<uint32_t>(), uint32_t(m),
+                                                         uint32_t(m));
   VDBG_HIP(hipGetLastError());
   std::vector<uint32_t> cnt(k), offh(k + 1);
-  std::vector<float> disth(m);
   st.train_points = m;
-  constexpr float kEps = 1.0f / 1024.0f;
+  VDBG_HIP(hipMemcpyAsync(dcen.p, cen, k * d * sizeof(float), hipMemcpyHostToDevice, s));
   for (size_t it = 0; it < o.iters; ++it) {
-    VDBG_HIP(hipMemcpyAsync(dcen.p, cen, k * d * sizeof(float), hipMemcpyHostToDevice, s));
     VDBG_RETURN_IF_ERROR(AssignNearestGpu(c, x, m, d, xs, dcen.get<float>(), k,
                                           assign.get<uint32_t>(), dist.get<float>(), s));
-    VDBG_HIP(hipMemsetAsync(counts.p, 0, k * 4, s));
-    k_histogram<<<dim3(unsigned((m + 255) / 256)), 256, 0, s>>>(assign.get<uint32_t>(), uint32_t(m),
-                                                                counts.get<uint32_t>());
-    VDBG_HIP(hipGetLastError());
     VDBG_HIP(hipcub::DeviceRadixSort::SortPairs(tmp.p, tmp_bytes, assign.get<uint32_t>(),
                                                 keys_out.get<uint32_t>(), vals_in.get<uint32_t>(),
                                                 vals_out.get<uint32_t>(), int(m), 0, end_bit, s));
-    VDBG_HIP(hipMemcpyAsync(cnt.data(), counts.p, k * 4, hipMemcpyDeviceToHost, s));
-    VDBG_HIP(hipMemcpyAsync(disth.data(), dist.p, m * 4, hipMemcpyDeviceToHost, s));
-    VDBG_HIP(hipStreamSynchronize(s));
-    st.inertia = 0;
-    for (size_t i = 0; i < m; ++i) st.inertia += disth[i];
-    offh[0] = 0;
-    for (size_t q = 0; q < k; ++q) offh[q + 1] = offh[q] + cnt[q];
-    VDBG_HIP(hipMemcpyAsync(off.p, offh.data(), (k + 1) * 4, hipMemcpyHostToDevice, s));
-    k_centroid_update<<<dim3(unsigned(k)), unsigned(std::min<size_t>(256, (d + 63) / 64 * 64)), 0, s>>>(
-        x, int(d), int(xs), vals_out.get<uint32_t>(), off.get<uint32_t>(), dcen.get<float>());
+    k_offsets<<<dim3(unsigned(k / 256 + 1)), 256, 0, s>>>(keys_out.get<uint32_t>(), uint32_t(m),
+                                                          uint32_t(k), off.get<uint32_t>());
+    k_centroid_update<<<dim3(unsigned(k)), UpdateThreads(d), 0, s>>>(
+        x, int(d), int(xs), int(k), 0, vals_out.get<uint32_t>(), off.get<uint32_t>(),
+        dcen.get<float>());
     VDBG_HIP(hipGetLastError());
+    VDBG_HIP(hipMemcpyAsync(offh.data(), off.p, (k + 1) * 4, hipMemcpyDeviceToHost, s));
     VDBG_HIP(hipMemcpyAsync(cen, dcen.p, k * d * sizeof(float), hipMemcpyDeviceToHost, s));
     VDBG_HIP(hipStreamSynchronize(s));
-    // Empty clusters: split the largest in two with a symmetric perturbation (:159-172).
-    std::vector<size_t> counts_sz(cnt.begin(), cnt.end());
+    size_t empty = 0;
     for (size_t q = 0; q < k; ++q) {
-      if (counts_sz[q] != 0) continue;
-      const size_t big = static_cast<size_t>(
-          std::max_element(counts_sz.begin(), counts_sz.end()) - counts_sz.begin());
-      std::uniform_real_distribution<float> noise(-1.f, 1.f);
-      for (size_t j = 0; j < d; ++j) {
-        const float v = cen[big * d + j];
-        const float delta = kEps * (std::fabs(v) + 1e-3f) * noise(rng);
-        cen[q * d + j] = v + delta;
-        cen[big * d + j] = v - delta;
-      }
-      counts_sz[q] = counts_sz[big] / 2;
-      counts_sz[big] -= counts_sz[q];
-      ++st.empty_reseeds;
+      cnt[q] = offh[q + 1] - offh[q];
+      empty += cnt[q] == 0 ? 1 : 0;
+    }
+    if (empty > 0) {
+      SplitLargest(cen, k, d, cnt.data(), rng, &st.empty_reseeds);
+      VDBG_HIP(hipMemcpyAsync(dcen.p, cen, k * d * sizeof(float), hipMemcpyHostToDevice, s));
     }
     st.iterations = it + 1;
   }
+  if (info != nullptr && o.iters > 0) {  // the last assignment's distances, summed in row order
+    std::vector<float> disth(m);
+    VDBG_HIP(hipMemcpyAsync(disth.data(), dist.p, m * 4, hipMemcpyDeviceToHost, s));
+    VDBG_HIP(hipStreamSynchronize(s));
+    for (size_t i = 0; i < m; ++i) st.inertia += disth[i];
+  }
   if (info) *info = st;
+  VDBG_HIP(hipStreamSynchronize(s));  // (copies from this call's host arrays have completed)
+  return kOk;
+}
+
+// Lloyd iterations of m sub-quantizers at once (PqTrainGpu): x [m][n][d] training sub-vectors,
+// dcen [m][256][d] initial centroids, both on the device, distances in L2SqAny order.  One
+// assignment, one stable sort by (set, cluster), one update and one small copy back an
+// iteration, where a set at a time took the same launches and two waits each.
+int LloydSets(Ctx* c, const float* x, size_t m, size_t n, size_t d, float* dcen, size_t iters,
+              std::vector<std::mt19937_64>* rngs, hipStream_t s) {
+  constexpr size_t k = 256;
+  const size_t total = m * n;
+  DevBuf key, skey, vals, order, off, tmp;
+  VDBG_RETURN_IF_ERROR(Alloc(&key, total * 4, s));
+  VDBG_RETURN_IF_ERROR(Alloc(&skey, total * 4, s));
+  VDBG_RETURN_IF_ERROR(Alloc(&vals, total * 4, s));
+  VDBG_RETURN_IF_ERROR(Alloc(&order, total * 4, s));
+  VDBG_RETURN_IF_ERROR(Alloc(&off, (m * k + 1) * 4, s));
+  int end_bit = 8;
+  while ((size_t(1) << end_bit) < m * k) ++end_bit;
+  size_t tmp_bytes = 0;
+  VDBG_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, key.get<uint32_t>(),
+                                              skey.get<uint32_t>(), vals.get<uint32_t>(),
+                                              order.get<uint32_t>(), int(total), 0, end_bit, s));
+  VDBG_RETURN_IF_ERROR(Alloc(&tmp, tmp_bytes, s));
+  k_iota<<<dim3(unsigned((total + 255) / 256)), 256, 0, s>>>(vals.get<uint32_t>(), uint32_t(total),
+                                                             uint32_t(n));
+  const dim3 grid(unsigned((n + 255) / 256), unsigned(m));
+  const size_t lds = k * d * sizeof(float);
+  std::vector<uint32_t> offh(m * k + 1), cnt(k);
+  std::vector<float> cen;
+  for (size_t it = 0; it < iters; ++it) {
+    {
+      ProfScope ps(c, "assign_any", s);
+      uint32_t* kp = key.get<uint32_t>();
+#define VDBG_SETS(DD) k_assign_sets<DD><<<grid, 256, lds, s>>>(x, uint32_t(n), int(d), dcen, int(k), kp)
+      switch (d) {
+        case 4: VDBG_SETS(4); break;
+        case 8: VDBG_SETS(8); break;
+        case 12: VDBG_SETS(12); break;
+        case 24: VDBG_SETS(24); break;
+        default: VDBG_SETS(0); break;
+      }
+#undef VDBG_SETS
+    }
+    VDBG_HIP(hipcub::DeviceRadixSort::SortPairs(tmp.p, tmp_bytes, key.get<uint32_t>(),
+                                                skey.get<uint32_t>(), vals.get<uint32_t>(),
+                                                order.get<uint32_t>(), int(total), 0, end_bit, s));
+    k_offsets<<<dim3(unsigned(m * k / 256 + 1)), 256, 0, s>>>(
+        skey.get<uint32_t>(), uint32_t(total), uint32_t(m * k), off.get<uint32_t>());
+    k_centroid_update<<<dim3(unsigned(m * k)), UpdateThreads(d), 0, s>>>(
+        x, int(d), int(d), int(k), n * d, order.get<uint32_t>(), off.get<uint32_t>(), dcen);
+    VDBG_HIP(hipGetLastError());
+    VDBG_HIP(hipMemcpyAsync(offh.data(), off.p, offh.size() * 4, hipMemcpyDeviceToHost, s));
+    VDBG_HIP(hipStreamSynchronize(s));
+    bool empty = false;
+    for (size_t q = 0; q < m * k; ++q) empty |= offh[q + 1] == offh[q];
+    if (!empty) continue;
+    cen.resize(m * k * d);
+    VDBG_HIP(hipMemcpyAsync(cen.data(), dcen, cen.size() * 4, hipMemcpyDeviceToHost, s));
+    VDBG_HIP(hipStreamSynchronize(s));
+    for (size_t j = 0; j < m; ++j) {
+      for (size_t q = 0; q < k; ++q) cnt[q] = offh[j * k + q + 1] - offh[j * k + q];
+      size_t reseeds = 0;
+      SplitLargest(cen.data() + j * k * d, k, d, cnt.data(), (*rngs)[j], &reseeds);
+    }
+    VDBG_HIP(hipMemcpyAsync(dcen, cen.data(), cen.size() * 4, hipMemcpyHostToDevice, s));
+    VDBG_HIP(hipStreamSynchronize(s));
+  }
   return kOk;
 }
 
@@ -494,8 +998,37 @@ int PqTrainGpu(Ctx* c, const float* data, size_t n, size_t stride, size_t dim, s
   for (size_t i = 0, taken = 0; i < n && taken < cap; i += step, ++taken) rows.push_back(uint32_t(i));
   DevBuf dr, sub;
   VDBG_RETURN_IF_ERROR(Alloc(&dr, rows.size() * 4, s));
-  VDBG_RETURN_IF_ERROR(Alloc(&sub, rows.size() * dsub * sizeof(float), s));
   VDBG_HIP(hipMemcpyAsync(dr.p, rows.data(), rows.size() * 4, hipMemcpyHostToDevice, s));
+  // All m sub-quantizers at once: narrow sub-vectors of enough points to initialise on the
+  // device, whose training sets fit 1 GiB and whose (set, row) pairs a 32-bit sort takes.
+  const size_t np = rows.size();
+  if (opts.kmeanspp && KMeansPPOnGpu(np) && 256.0 * double(np) <= 2.0e7 && dsub <= 64 &&
+      !SimdL2(dsub, dsub) && np * dim * 4 <= (size_t(1) << 30) && m * np < (size_t(1) << 31) &&
+      m <= 65535) {
+    VDBG_RETURN_IF_ERROR(Alloc(&sub, m * np * dsub * sizeof(float), s));
+    for (size_t j = 0; j < m; ++j)
+      k_gather_rows<<<dim3(unsigned((np * dsub + 255) / 256)), 256, 0, s>>>(
+          data, int(stride), dr.get<uint32_t>(), uint32_t(np), int(dsub), int(j * dsub),
+          sub.get<float>() + j * np * dsub);
+    VDBG_HIP(hipGetLastError());
+    std::vector<std::mt19937_64> rngs;
+    for (size_t j = 0; j < m; ++j) rngs.emplace_back(opts.seed + j * 7919);
+    DevBuf dcen;
+    VDBG_RETURN_IF_ERROR(Alloc(&dcen, centroids->size() * sizeof(float), s));
+    bool failed = false;
+    VDBG_RETURN_IF_ERROR(KMeansPPGpu(c, sub.get<float>(), np * dsub, m, np, dsub, dsub, 256, &rngs,
+                                     dcen.get<float>(), &failed, s));
+    if (!failed) {
+      VDBG_RETURN_IF_ERROR(LloydSets(c, sub.get<float>(), m, np, dsub, dcen.get<float>(),
+                                     opts.iters, &rngs, s));
+      VDBG_HIP(hipMemcpyAsync(centroids->data(), dcen.p, centroids->size() * sizeof(float),
+                              hipMemcpyDeviceToHost, s));
+      VDBG_HIP(hipStreamSynchronize(s));
+      return kOk;
+    }
+  } else {
+    VDBG_RETURN_IF_ERROR(Alloc(&sub, rows.size() * dsub * sizeof(float), s));
+  }
   std::vector<float> cen;
   for (size_t j = 0; j < m; ++j) {
     k_gather_rows<<<dim3(unsigned((rows.size() * dsub + 255) / 256)), 256, 0, s>>>(
@@ -585,7 +1118,8 @@ int IvfBuildGpu(Ctx* c, IvfIndex* x, size_t nlist_req, size_t m, uint64_t seed, 
   VDBG_RETURN_IF_ERROR(Alloc(&counts, nlist * 4, s));
   VDBG_HIP(hipMalloc(reinterpret_cast<void**>(&x->ids), n * 4));
   VDBG_HIP(hipMalloc(reinterpret_cast<void**>(&x->codes), n * m));
-  k_iota<<<dim3(unsigned((n + 255) / 256)), 256, 0, s>>>(order_in.get<uint32_t>(), uint32_t(n));
+  k_iota<<<dim3(unsigned((n + 255) / 256)), 256, 0, s>>>(order_in.get<uint32_t>(), uint32_t(n),
+                                                         uint32_t(n));
   VDBG_HIP(hipMemsetAsync(counts.p, 0, nlist * 4, s));
   k_histogram<<<dim3(unsigned((n + 255) / 256)), 256, 0, s>>>(assign.get<uint32_t>(), uint32_t(n),
                                                               counts.get<uint32_t>());
