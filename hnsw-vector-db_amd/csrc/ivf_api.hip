@@ -62,6 +62,10 @@ void FreeIvf(IvfIndex* x) {
   (void)hipFree(x->term2);
   (void)hipFree(x->rowsum);
   (void)hipFree(x->t2abs);
+  (void)hipFree(x->res16);
+  (void)hipFree(x->list_rad);
+  x->res16 = nullptr;
+  x->list_rad = nullptr;
   x->rowsum = nullptr;
   x->t2abs = nullptr;
   x->coarse_ds = nullptr;
@@ -98,6 +102,8 @@ int InstallIvf(Ctx* c, IvfIndex* x, hipStream_t s) {
     VDBG_HIP(hipMalloc(reinterpret_cast<void**>(&x->t2abs), nlist * sizeof(float)));
     VDBG_RETURN_IF_ERROR(IvfRowSums(c, x->off, int(nlist), x->codes, x->m, x->term2, x->rowsum,
                                     x->t2abs, s));
+    // (the scan by list falls back to the row-sum scan, which takes these code widths)
+    if (x->m == 4 || x->m == 8 || x->m == 16) VDBG_RETURN_IF_ERROR(IvfMakeDecoded(c, x, s));
   }
   VDBG_HIP(hipStreamSynchronize(s));
   return kOk;
@@ -216,12 +222,26 @@ static int IvfSearch(IvfIndex* x, const float* Q, size_t nq, size_t k, size_t np
   // the row-sum scan (k_ivf_scan_rs) also takes each query's per-subspace table maxima
   const bool rs = pre && c->ivf_row_sums && x->rowsum != nullptr && R <= 256 &&
                   (x->m == 4 || x->m == 8 || x->m == 16);
-  const bool want_qtab = pre || !l2;
+  // large batches contract their queries with each list's residuals (no tables), if their
+  // scratch can be had
+  bool lists = rs && allow == nullptr && IvfListsEligible(*x, nq, nprobe, R);
   void* buf = nullptr;
-  const size_t scan_bytes = R <= 256 ? IvfScanScratchBytes(nq, nprobe) : 0;
-  const size_t bytes = nq * nprobe * 8 + (want_qtab ? nq * ts * 4 : 0) + (rs ? nq * x->m * 4 : 0) +
-                       nq * R * 8 + scan_bytes + 4096 + 256;
-  VDBG_HIP(hipMallocAsync(&buf, bytes, s));
+  size_t scan_bytes = 0;
+  auto alloc = [&]() {
+    scan_bytes = lists      ? IvfListsScratch(*x, nq, nprobe)
+                 : R <= 256 ? IvfScanScratchBytes(nq, nprobe)
+                            : 0;
+    const size_t tables = lists ? 0 : (pre || !l2 ? nq * ts * 4 : 0) + (rs ? nq * x->m * 4 : 0);
+    return ScratchAlloc(c, &buf, nq * nprobe * 8 + tables + nq * R * 8 + scan_bytes + 4096 + 256, s);
+  };
+  hipError_t e = alloc();
+  if (e != hipSuccess && lists) {
+    (void)hipGetLastError();
+    lists = false;
+    e = alloc();
+  }
+  VDBG_HIP(e);
+  const bool want_qtab = (pre || !l2) && !lists;
   char* p = static_cast<char*>(buf);
   auto take = [&](size_t b) {
     char* r = p;
@@ -231,7 +251,7 @@ static int IvfSearch(IvfIndex* x, const float* Q, size_t nq, size_t k, size_t np
   uint32_t* probe = reinterpret_cast<uint32_t*>(take(nq * nprobe * 4));
   float* probe_d = reinterpret_cast<float*>(take(nq * nprobe * 4));
   float* qtab = want_qtab ? reinterpret_cast<float*>(take(nq * ts * 4)) : nullptr;
-  float* qmax = rs ? reinterpret_cast<float*>(take(nq * x->m * 4)) : nullptr;
+  float* qmax = rs && !lists ? reinterpret_cast<float*>(take(nq * x->m * 4)) : nullptr;
   uint32_t* ti = R == k ? out_ids : reinterpret_cast<uint32_t*>(take(nq * R * 4));
   float* td = R == k ? out_d : reinterpret_cast<float*>(take(nq * R * 4));
   // the scan's own scratch, allocated here with the rest (no allocation between the coarse
@@ -240,7 +260,7 @@ static int IvfSearch(IvfIndex* x, const float* Q, size_t nq, size_t k, size_t np
   // the tables depend on the queries alone: queued first, they keep the GPU busy while the
   // host plans and queues the coarse probe
   int rc = kOk;
-  if (rs)
+  if (rs && !lists)
     rc = IvfQtabRs(c, Q, x->pd, int(nq), x->cen, x->m, x->dsub, qtab, qmax, s);
   else if (qtab != nullptr)
     rc = IvfQtab(c, Q, x->pd, int(nq), x->cen, x->m, x->dsub, pre ? 1 : 0, qtab, s);
@@ -255,7 +275,9 @@ static int IvfSearch(IvfIndex* x, const float* Q, size_t nq, size_t k, size_t np
       a.t2abs = x->t2abs;
       a.qmax = qmax;
     }
-    rc = R <= 256 ? IvfScan(c, a, s, scan_scratch) : IvfScanDeep(c, a, s);
+    rc = lists      ? IvfScanLists(c, *x, a, s, scan_scratch)
+         : R <= 256 ? IvfScan(c, a, s, scan_scratch)
+                    : IvfScanDeep(c, a, s);
   }
   if (rc == kOk && depth > 0) {
     rc = Rerank(c, x->ds->rows, x->pd, x->metric, Q, nq, ti, R, k, out_ids, out_d, s,

@@ -681,8 +681,9 @@ __global__ __launch_bounds__(256) void k_ivf_qtab_rs(const float* __restrict__ Q
 // Rows not skipped (NaN included) are staged and scored exactly, as the reference scores them,
 // and those below the wave's R-th key enter its top-R; the filter is tested on those alone,
 // which skips nothing the reference would keep.  The four waves' tops merge at the end.
-template <int E, int M, int CH>
-__global__ __launch_bounds__(kRsWaves * 64, 6) void k_ivf_scan_rs(IvfScanArgs a, IvfFastArgs f) {
+// SELF: the block makes the query's table itself (k_ivf_qtab_rs's operations).
+template <int E, int M, int CH, bool SELF>
+__device__ __forceinline__ void ivf_scan_rs_query(const IvfScanArgs& a, const uint32_t q) {
   constexpr int TS = M * kKsub;
   constexpr int W = (M + 3) / 4;
   constexpr int NT = kRsWaves * kWave;
@@ -697,20 +698,30 @@ __global__ __launch_bounds__(kRsWaves * 64, 6) void k_ivf_scan_rs(IvfScanArgs a,
   __shared__ uint32_t st_row[kRsWaves][2 * kWave];
   __shared__ uint32_t st_slot[kRsWaves][2 * kWave];
 
-  const int b = blockIdx.x;
-  const int item = (b & 7) * f.per_xcd + (b >> 3);
-  if (item >= f.items) return;  // uniform over the block
-  const uint32_t q = f.qorder ? f.qorder[item] : uint32_t(item);
   const int tid = threadIdx.x, wave = tid >> 6, lane = lane_id();
   float* qt = smem;
-  {
-    const float4* g = reinterpret_cast<const float4*>(a.qtab + size_t(q) * TS);
-    for (int e = tid; e < TS / 4; e += NT) reinterpret_cast<float4*>(qt)[e] = g[e];
-  }
   if (tid == 0) tau_blk = __builtin_inff();
   float bq = 0.f;
+  if constexpr (SELF) {
+    __shared__ float wmax[M][kRsWaves];
+    for (int j = 0; j < M; ++j) {  // thread c: entry [j][c]
+      const float x = -dot_any(a.Q + size_t(q) * a.pd + size_t(j) * a.dsub,
+                               a.cen + (size_t(j) * kKsub + tid) * a.dsub, a.dsub) * 2.f;
+      qt[j * kKsub + tid] = x;
+      float mx = fabsf(x);
 #pragma unroll
-  for (int j = 0; j < M; ++j) bq += a.qmax[size_t(q) * M + j];
+      for (int o = kWave / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+      if (lane == 0) wmax[j][wave] = mx;
+    }
+    __syncthreads();
+    for (int j = 0; j < M; ++j)
+      bq += fmaxf(fmaxf(wmax[j][0], wmax[j][1]), fmaxf(wmax[j][2], wmax[j][3]));
+  } else {
+    const float4* g = reinterpret_cast<const float4*>(a.qtab + size_t(q) * TS);
+    for (int e = tid; e < TS / 4; e += NT) reinterpret_cast<float4*>(qt)[e] = g[e];
+#pragma unroll
+    for (int j = 0; j < M; ++j) bq += a.qmax[size_t(q) * M + j];
+  }
   bq *= 1.f + 0x1p-16f;
   __syncthreads();
 
@@ -946,6 +957,26 @@ __global__ __launch_bounds__(kRsWaves * 64, 6) void k_ivf_scan_rs(IvfScanArgs a,
   }
 }
 
+template <int E, int M, int CH>
+__global__ __launch_bounds__(kRsWaves * 64, 6) void k_ivf_scan_rs(IvfScanArgs a, IvfFastArgs f) {
+  const int b = blockIdx.x;
+  const int item = (b & 7) * f.per_xcd + (b >> 3);
+  if (item >= f.items) return;  // uniform over the block
+  ivf_scan_rs_query<E, M, CH, false>(a, f.qorder ? f.qorder[item] : uint32_t(item));
+}
+
+// The queries list[0, *count), on a bounded grid whose blocks stride over them (queued behind
+// the scan by list, which lists few or none).
+template <int E, int M>
+__global__ __launch_bounds__(kRsWaves * 64, 4) void k_ivf_scan_listed(
+    IvfScanArgs a, const uint32_t* __restrict__ list, const uint32_t* __restrict__ count) {
+  const uint32_t n = min(*count, uint32_t(a.nq));
+  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+    ivf_scan_rs_query<E, M, 2, true>(a, list[i]);
+    __syncthreads();  // the block's shared arrays are free again
+  }
+}
+
 // ProductQuantizer::encode (pq.cc:43-57) of the residual x - coarse[assign] (ivf_pq.cc:
 // 128-139): per subspace the first centroid with the smallest L2SqAny.  One thread per
 // (row, subspace).
@@ -1074,6 +1105,30 @@ static int launch_rs_m(int e, hipStream_t s, const IvfScanArgs& a, const IvfFast
     case 4: k_ivf_scan_rs<4, M, CH><<<g, blk, 0, s>>>(a, f); break;
     default: return SetError(kNotSupported, "IVF-PQ: max(rerank, k) > 256 on the GPU path");
   }
+  return kOk;
+}
+
+template <int M>
+static void launch_listed(int e, hipStream_t s, const IvfScanArgs& a, const uint32_t* list,
+                          const uint32_t* count) {
+  const dim3 g(unsigned(std::min(a.nq, 512))), blk(kRsWaves * 64);
+  if (e == 1) k_ivf_scan_listed<1, M><<<g, blk, 0, s>>>(a, list, count);
+  else if (e == 2) k_ivf_scan_listed<2, M><<<g, blk, 0, s>>>(a, list, count);
+  else k_ivf_scan_listed<4, M><<<g, blk, 0, s>>>(a, list, count);
+}
+
+int IvfScanListed(Ctx* c, const IvfScanArgs& a, const uint32_t* list, const uint32_t* count,
+                  hipStream_t s) {
+  int e = 1;
+  while (kWave * e < a.R) e <<= 1;
+  ProfScope ps(c, "ivf_rescan", s);
+  switch (a.m) {
+    case 4: launch_listed<4>(e, s, a, list, count); break;
+    case 8: launch_listed<8>(e, s, a, list, count); break;
+    case 16: launch_listed<16>(e, s, a, list, count); break;
+    default: return SetError(kInternal, "ivf lists: m");
+  }
+  VDBG_HIP(hipGetLastError());
   return kOk;
 }
 

@@ -227,6 +227,32 @@ int StageOut(Ctx* c, const uint8_t* const* src, const size_t* bytes, void* const
   return kOk;
 }
 
+hipError_t ScratchAlloc(Ctx* c, void** p, size_t bytes, hipStream_t s) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+  if (cap == hipStreamCaptureStatusNone) {
+    if (c->pool == nullptr) {
+      hipMemPoolProps props{};
+      props.allocType = hipMemAllocationTypePinned;
+      props.location.type = hipMemLocationTypeDevice;
+      props.location.id = c->device;
+      uint64_t keep = kScratchPoolKeep;
+      if (hipMemPoolCreate(&c->pool, &props) != hipSuccess) {
+        (void)hipGetLastError();
+        c->pool = nullptr;
+      } else if (hipMemPoolSetAttribute(c->pool, hipMemPoolAttrReleaseThreshold, &keep) !=
+                 hipSuccess) {
+        (void)hipGetLastError();
+      }
+    }
+    if (c->pool != nullptr) {
+      if (hipMallocFromPoolAsync(p, bytes, c->pool, s) == hipSuccess) return hipSuccess;
+      (void)hipGetLastError();  // the default pool may still hold it
+    }
+  }
+  return hipMallocAsync(p, bytes, s);
+}
+
 int Workspace::reserve(size_t bytes) {
   if (bytes <= cap) return kOk;
   if (fixed)
@@ -722,6 +748,7 @@ int vdbg_ctx_destroy(vdbg_ctx* ctx) {
   if (c.stage_d) (void)hipFree(c.stage_d);
   if (c.fb_dev) (void)hipFree(c.fb_dev);
   if (c.host_flag) (void)hipHostFree(c.host_flag);
+  if (c.pool) (void)hipMemPoolDestroy(c.pool);
   (void)hipStreamDestroy(c.stream);
   delete ctx;
   return kOk;

@@ -109,6 +109,9 @@ struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::recursive_mutex mu;
+  // stream-ordered scratch of large calls (ScratchAlloc): up to kScratchPoolKeep bytes stay
+  // mapped between calls, all of them go back with the context
+  hipMemPool_t pool = nullptr;
   Workspace ws;   // per-call scratch
   Workspace ws2;  // scratch of the exact re-scan that runs while ws is live
   Workspace wsc;  // scratch of the filtered scan's row compaction (kept across calls)
@@ -292,6 +295,16 @@ struct IvfIndex {
   float* term2 = nullptr;            // nlist x m x 256, or null
   float* rowsum = nullptr;           // n: sum_j term2[l][j][code_j] per CSR row (with term2)
   float* t2abs = nullptr;            // nlist: sum_j max_c |term2[l][j][c]| (with term2)
+  // the decoded residuals r of the CSR rows as fp16(r 2^res_exp) (2 pd bytes a row), which
+  // large batches contract with their queries list by list (ivf_lists.hip); null where that
+  // path does not apply or memory is short; each list's largest |r|.  Beside them what bounds
+  // its error: the largest component and norm of a residual, sqrt(sum_j max_c |C_j[c]|^2), the
+  // largest coarse norm and t2abs.
+  uint16_t* res16 = nullptr;
+  float* list_rad = nullptr;
+  int res_exp = 0;
+  float res_max = 0.f;
+  double res_norm = 0.0, cen_norm = 0.0, coarse_norm = 0.0, t2_max = 0.0;
   std::vector<float> coarse_h, cen_h;
   std::vector<uint32_t> off_h;
 };
@@ -407,8 +420,22 @@ int ScoreScan(Ctx* c, const ScanSource& src, const float* Q, size_t nq, size_t k
 // Sets up the allocation-free flat search's scratch on `device` (its address there), once per
 // device; called by vdbg_ctx_create with the device current (noalloc.hip).
 int InitNoAllocScratch(int device);
+// Stream-ordered scratch from the context's pool, freed with hipFreeAsync.  The device's
+// default pool gives its memory back at every synchronization, so each call of a large batch
+// mapped its scratch anew (10,000 IVF-PQ queries, 165 MB: ~330 us between two calls).
+constexpr size_t kScratchPoolKeep = size_t(512) << 20;
+hipError_t ScratchAlloc(Ctx* c, void** p, size_t bytes, hipStream_t s);
 // Fills n 32-bit words with v on stream s (a kernel, so a captured graph holds no memset).
 int Fill32(void* p, uint32_t v, size_t n, hipStream_t s);
+// The IVF-PQ scan by list (ivf_lists.hip): the decoded residuals of an index, the batches it
+// takes, its scratch, the scan; and k_ivf_scan_rs for the queries a device list names (count in
+// device memory), their tables made in the scan.
+int IvfMakeDecoded(Ctx* c, IvfIndex* x, hipStream_t s);
+bool IvfListsEligible(const IvfIndex& x, size_t nq, size_t nprobe, size_t R);
+size_t IvfListsScratch(const IvfIndex& x, size_t nq, size_t nprobe);
+int IvfScanLists(Ctx* c, const IvfIndex& x, const IvfScanArgs& a, hipStream_t s, void* scratch);
+int IvfScanListed(Ctx* c, const IvfScanArgs& a, const uint32_t* list, const uint32_t* count,
+                  hipStream_t s);
 // Exact fp32 distances of `depth` candidate rows per query, the k smallest.
 // rows (nullable): the dataset's scan source, whose int8 copy of integer rows serves
 // exact-integer queries.
