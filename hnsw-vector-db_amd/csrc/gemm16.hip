@@ -195,8 +195,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm16(GemmArgs a) {
       }
     }
     st.n = a.rn[base + min(uint32_t(tid & 63), valid - 1)];  // (the store applies validity)
-    if constexpr (MODE == 0)  // a scan without a filter reads one all-ones word (mask 0)
-      st.aw = a.aw[((base >> 5) + (uint32_t(tid & 63) >> 5)) & a.aw_mask];
+    // (a scan without a filter reads one all-ones word, mask 0)
+    st.aw = a.aw[((base >> 5) + (uint32_t(tid & 63) >> 5)) & a.aw_mask];
   };
   auto store_stage = [&](const Stage& st, int sidx) {
     const int tile = sidx / NKC, kc = sidx - tile * NKC;
@@ -209,8 +209,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm16(GemmArgs a) {
     }
     if (kc == 0 && tid < kGemmRows) {
       const uint32_t valid = min(uint32_t(kGemmRows), r_end - (r_begin + uint32_t(tile) * kGemmRows));
-      // rows past r_end, and in MODE 0 rows the filter excludes, start from NaN
-      const bool ok = uint32_t(tid) < valid && (MODE != 0 || ((st.aw >> (tid & 31)) & 1u));
+      // rows past r_end and rows the filter excludes start from NaN
+      const bool ok = uint32_t(tid) < valid && ((st.aw >> (tid & 31)) & 1u);
       xns[tile % 3][tid] = ok ? (METRIC == 0 ? st.n : 0.f) : __builtin_nanf("");
     }
   };
@@ -335,22 +335,14 @@ __global__ __launch_bounds__(256, 2) void k_gemm16(GemmArgs a) {
           }
         }
     } else if (wave_live) {
-      // fminf skips the NaN values of rows past r_end
+      // fminf skips the NaN values of rows past r_end or outside the filter
 #pragma unroll
       for (int qb = 0; qb < NQB; ++qb)
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk) {
           float m = __builtin_inff();
-          if (a.allow == nullptr) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) m = fminf(m, value(qb, blk, r));
-          } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const uint32_t row = lane_base + (blk * 32 + 8 * (r >> 2) + (r & 3));
-              if (row < r_end && row_allowed(a.allow, a.rid[row])) m = fminf(m, value(qb, blk, r));
-            }
-          }
+          for (int r = 0; r < 16; ++r) m = fminf(m, value(qb, blk, r));
           if (q[qb] < a.nq) {
             const uint32_t grp = ((base >> 5) + blk) * 2 + h;
             if (grp < uint32_t(a.ngroups)) a.gm[size_t(q[qb]) * a.ngroups + grp] = m;

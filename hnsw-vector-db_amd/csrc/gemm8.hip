@@ -191,8 +191,7 @@ __global__ __launch_bounds__(256, OCC) void k_gemm8(GemmArgs a) {
                  : 0;
     else
       st.n = a.rn8[base + min(uint32_t(tid & 63), valid - 1)];
-    if constexpr (MODE == 0)
-      st.aw = a.aw[((base >> 5) + (uint32_t(tid & 63) >> 5)) & a.aw_mask];
+    st.aw = a.aw[((base >> 5) + (uint32_t(tid & 63) >> 5)) & a.aw_mask];
   };
   auto store_stage = [&](const Stage& st, int sidx) {
     const int tile = sidx / NKC, kc = sidx - tile * NKC;
@@ -206,7 +205,7 @@ __global__ __launch_bounds__(256, OCC) void k_gemm8(GemmArgs a) {
     }
     if (kc == 0 && tid < kGemmRows) {
       const uint32_t valid = min(uint32_t(kGemmRows), r_end - (r_begin + uint32_t(tile) * kGemmRows));
-      const bool ok = uint32_t(tid) < valid && (MODE != 0 || ((st.aw >> (tid & 31)) & 1u));
+      const bool ok = uint32_t(tid) < valid && ((st.aw >> (tid & 31)) & 1u);
       xns[tile % 3][tid] = ok ? st.n : kDead;
     }
   };
@@ -326,16 +325,8 @@ __global__ __launch_bounds__(256, OCC) void k_gemm8(GemmArgs a) {
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk) {
           int m = kDead;
-          if (a.allow == nullptr) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) m = max(m, acc[qb][blk][r]);
-          } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const uint32_t row = lane_base + (blk * 32 + 8 * (r >> 2) + (r & 3));
-              if (row < r_end && row_allowed(a.allow, a.rid[row])) m = max(m, acc[qb][blk][r]);
-            }
-          }
+          for (int r = 0; r < 16; ++r) m = max(m, acc[qb][blk][r]);
           if constexpr (MODE == 2) {
             // insert into the descending list: t' = clamp(m, top[t + 1], top[t]) from the
             // bottom up, each step reading the entry above before it changes

@@ -872,6 +872,10 @@ struct ScanInit {
   uint32_t* ones;        // nullable, [1] all ones
   int* e8;               // nullable, [2] 0
   uint32_t* fb_zero;     // nullable: the context's count of device-gated re-scans, 0
+  const uint64_t* allow; // the filter by sample position: bit p of bits is row sid[p]'s
+  const uint32_t* sid;
+  uint32_t S;
+  uint64_t* bits;        // nullable, [ceil(S / 64)]
 };
 __global__ void k_scan_init(ScanInit a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -883,6 +887,10 @@ __global__ void k_scan_init(ScanInit a) {
     if (a.e8 != nullptr) a.e8[i] = 0;
   }
   if (i == 0 && a.ones != nullptr) a.ones[0] = 0xffffffffu;
+  if (a.bits != nullptr && uint32_t(i & ~63) < a.S) {  // (wave-uniform)
+    const uint64_t b = __ballot(uint32_t(i) < a.S && row_allowed(a.allow, a.sid[min(uint32_t(i), a.S - 1)]));
+    if (lane_id() == 0) a.bits[i >> 6] = b;
+  }
 }
 
 // SQ8 on the int8 GEMM (gemm8.hip, SQ = 1): the B operand of every query of the batch scaled
@@ -3673,7 +3681,7 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
   // counts then candidates, the candidates 256-byte aligned
   auto cand_total = [&]() {
     return std::max({cand_bytes(p32), try16 ? cand_bytes(p16) : 0,
-                     try8any ? cand_bytes(p8) : 0}) + 256;
+                     try8any ? cand_bytes(p8) : 0, (size_t(S) + 63) / 64 * sizeof(uint64_t)}) + 256;
   };
   size_t cand_need = cand_total();
   const int Esel = pow2_e(kk + 16);
@@ -3696,7 +3704,8 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
       (try16 ? (split ? 2 : 1) * nq * pd * sizeof(uint16_t) + nq * sizeof(float) : 0) +
       (try8 ? nq * pd + nq * sizeof(int) : 0) +
       (try8op ? 2 * nq * pd + nq * (sizeof(int) + sizeof(float)) : 0) +
-      (deep.on ? nq * (deep.stride * sizeof(uint64_t) + sizeof(uint32_t)) : 0) + 28 * 256;
+      (deep.on ? nq * (deep.stride * sizeof(uint64_t) + sizeof(uint32_t)) : 0) +
+      28 * 256;
   // A workspace that cannot grow caps the candidate buffers instead: fewer, longer row
   // chunks (fewer blocks, so a less filled GPU) until they fit in what the rest leaves.
   // The sample pass and everything else are planned as before.
@@ -3732,12 +3741,20 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
   uint32_t* mb8 = try8op ? reinterpret_cast<uint32_t*>(e8 + 1) : nullptr;
   // the no-filter word of the fp16 and int8 GEMMs
   uint32_t* ones = try16 || try8any ? w.take<uint32_t>(1) : nullptr;
+  // the filter by sample position, which the fp16 and int8 sample passes read as the main pass
+  // reads the filter itself (a lookup per value through Sid took them 37 us instead of 9 at
+  // 65,536 of 118,385 x 112 rows)
+  // (kept where the candidates go: the main pass writes those after the sample pass has ended)
+  uint64_t* sbits = allow != nullptr && (try16 || try8any)
+                        ? reinterpret_cast<uint64_t*>(cand_base) : nullptr;
   int* fit8q = gated ? w.take<int>(nq) : nullptr;  // per query: inside the int8 bounds
   uint64_t* dkeys = deep.on ? w.take<uint64_t>(nq * deep.stride) : nullptr;
   uint32_t* dtotal = deep.on ? w.take<uint32_t>(nq) : nullptr;
   {
-    const ScanInit si{ovf, int(nq), fb_count, all16, ones, try8op ? e8 : nullptr, fb_zero};
-    k_scan_init<<<dim3(unsigned((std::max<size_t>(nq, 2) + 255) / 256)), 256, 0, s>>>(si);
+    const ScanInit si{ovf, int(nq), fb_count, all16, ones, try8op ? e8 : nullptr, fb_zero,
+                      allow, src->Sid, S, sbits};
+    const size_t n = std::max<size_t>({nq, 2, sbits != nullptr ? S : 0});
+    k_scan_init<<<dim3(unsigned((n + 255) / 256)), 256, 0, s>>>(si);
     VDBG_HIP(hipGetLastError());
   }
 
@@ -3796,6 +3813,8 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
   sg.rid = src->Sid;
   sg.Qb = B;
   sg.allow = allow;
+  sg.aw = sbits != nullptr ? reinterpret_cast<const uint32_t*>(sbits) : ones;
+  sg.aw_mask = sbits != nullptr ? ~0u : 0u;
   sg.gm = gm;
   sg.ngroups = ngroups;
   const bool top8 = use8 && P.qb == 2 && compact8;
