@@ -3333,9 +3333,14 @@ static bool RowScanF16(const Ctx* c, const ScanSource& src) {
 // Up to 8 queries; a source the ranking GEMM serves goes there from 3 on (its cost does not
 // grow with a few queries: 200,000 x 384 rows, 1 / 2 / 3 queries take 64 / 72 / 81 us here and
 // 79 / 80 / 80 us there, 20,000 x 100 rows 35 / 39 / 45 and 47 / 47 / 48, 50,000 x 848 rows,
-// which no GEMM kernel serves, 107 us for 2 queries against 205 scored exactly).
+// which no GEMM kernel serves, 107 us for 2 queries against 205 scored exactly).  Fewer than
+// 1,024 rows have no GEMM either; few enough of them are scored exactly in less than this path's
+// fixed cost (1 query, this / exact: 256 x 96 33 / 19 us, 1,023 x 96 33 / 32, 256 x 384 35 / 26,
+// 512 x 384 35 / 39, 512 x 839 43 / 49; 4 queries: 512 x 384 47 / 39, 800 x 384 46 / 58).
 static bool RowScanBeatsGemm(const ScanSource& src, size_t nq) {
-  return nq <= 2 || !GemmSupported(src.pd) || src.N < 1024;
+  if (src.N < 1024)
+    return uint64_t(src.N) * (256 + src.pd) >= 320000 + 80000 * uint64_t(nq - 1);
+  return nq <= 2 || !GemmSupported(src.pd);
 }
 
 bool RowScanEligible(const Ctx* c, const ScanSource& src, size_t nq, size_t kk) {
