@@ -260,16 +260,16 @@ struct GroupArgs {
 };
 
 template <bool SCATTER>
-__global__ __launch_bounds__(256) void k_lists_group(GroupArgs a) {
+__global__ __launch_bounds__(1024) void k_lists_group(GroupArgs a) {
   extern __shared__ uint32_t cnt[];
   uint32_t* hist = a.hist + size_t(blockIdx.x) * a.nlist;
-  for (uint32_t l = threadIdx.x; l < a.nlist; l += 256)
+  for (uint32_t l = threadIdx.x; l < a.nlist; l += 1024)
     cnt[l] = SCATTER ? a.ent_off[l] + hist[l] : 0u;
   __syncthreads();
   const int per = (a.nq + kHistBlocks - 1) / kHistBlocks;
   const int q0 = blockIdx.x * per, q1 = min(a.nq, q0 + per);
   const int n = max(0, q1 - q0) * a.np;
-  for (int t = threadIdx.x; t < n; t += 256) {
+  for (int t = threadIdx.x; t < n; t += 1024) {
     const int qi = t / a.np, p = t - qi * a.np, q = q0 + qi;
     const uint32_t e = uint32_t(q) * uint32_t(a.nprobe) + uint32_t(p);
     const uint32_t l = a.probe[e];
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(256) void k_lists_group(GroupArgs a) {
   }
   if (SCATTER) return;
   __syncthreads();
-  for (uint32_t l = threadIdx.x; l < a.nlist; l += 256) hist[l] = cnt[l];
+  for (uint32_t l = threadIdx.x; l < a.nlist; l += 1024) hist[l] = cnt[l];
 }
 
 // Each list's counts of the blocks become the blocks' first places in the list.
@@ -783,7 +783,7 @@ __device__ __forceinline__ void pick_query(const PickArgs& a, int q, uint32_t to
 
 // One wave per query.
 template <int E>
-__global__ __launch_bounds__(256, 4) void k_ivf_pick(PickArgs a) {
+__global__ __launch_bounds__(256, 6) void k_ivf_pick(PickArgs a) {
   __shared__ uint32_t st_row[4][kCap];
   __shared__ uint8_t st_p[4][kCap];
   __shared__ __attribute__((aligned(16))) float qv[4][128];
@@ -843,10 +843,10 @@ static int launch_lists(int pd, hipStream_t s, const ListArgs& a) {
 
 static int GroupPairs(hipStream_t s, const GroupArgs& g) {
   const unsigned lds = g.nlist * 4;
-  k_lists_group<false><<<dim3(kHistBlocks), 256, lds, s>>>(g);
+  k_lists_group<false><<<dim3(kHistBlocks), 1024, lds, s>>>(g);
   k_lists_columns<<<dim3((g.nlist + 31) / 32), 256, 0, s>>>(g);
   k_lists_scan<<<1, 1024, 0, s>>>(g);
-  k_lists_group<true><<<dim3(kHistBlocks), 256, lds, s>>>(g);
+  k_lists_group<true><<<dim3(kHistBlocks), 1024, lds, s>>>(g);
   VDBG_HIP(hipGetLastError());
   return kOk;
 }
