@@ -21,6 +21,9 @@
 //                  top-k), exact re-scoring in the reference's AVX-512 order, sort by
 //                  (dist, id), and a certificate that no unselected row can enter the top
 //                  kk; failures and overflows are re-scanned exactly (k_exact_scan).
+//   k_deep_score   answers deeper than one wavefront's list (kk > 240): the exact (dist, id) key
+//                  of every admitted candidate, sorted by one block a query (topk_large.hip).
+//   k_row_scan     1 to 8 queries: one pass over the rows and a merge instead of the above.
 //   k_rerank       (SQ8) exact fp32 distances of the top-R codes' rows, top k.
 //
 // Distances returned are always the reference's exact AVX-512-order values.
