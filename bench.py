@@ -56,7 +56,7 @@ def log(*a):
 
 PROFILES = {"flat": "flat_gemm8_sift_like_1m_x128_k10_b10000.md",
             "sq8": "sq8_gemm8_sift_like_1m_x128_d100_b10000.md",
-            "ivfpq": "ivf_scan_sift_like_1m_nlist4096_m16_nprobe64.md"}
+            "ivfpq": "ivf_lists_sift_like_1m_nlist4096_m16_nprobe64.md"}
 
 
 def profiled_traffic(path):
@@ -403,20 +403,22 @@ def run_pqflat(args, ctx, torch, ref, ds, base, queries, threads, cpu_model):
                          stream=stream)
 
     steps = max(1, min(args.steps, 5))
-    el, prof, _ = timed(ctx, torch, step, steps, 1, ["pq_tables", "exact_scan", "merge",
-                                                     "rerank"])
+    el, prof, _ = timed(ctx, torch, step, steps, 1,
+                        ["pq_tables", "query_prep", "sample_gemm", "kth", "pq_gemm", "select",
+                         "exact_scan", "merge", "rerank"])
     gi = ids.cpu().numpy().view(np.uint32).copy()
     gd = dd.cpu().numpy().copy()
-    sc_ms = prof["exact_scan"][0] / max(1, prof["exact_scan"][1])
-    code_bytes = nq * N * m
+    sc_ms = prof["pq_gemm"][0] / max(1, prof["pq_gemm"][1])
+    flop = 2.0 * nq * N * dim
     r = {"qps": nq * steps / el, "ms_per_step": el * 1e3 / steps, "batch": nq, "m": m,
-         "build_s": round(build_s, 2), "kernel": "k_exact_scan over PQ codes (ADC, wave top-k per row split)",
-         "kernel_ms": sc_ms, "bound": "hbm", "algorithmic_bytes_per_launch": code_bytes,
-         "achieved": code_bytes / (sc_ms * 1e-3) / 1e9 if sc_ms > 0 else None, "unit": "GB/s",
-         "peak": HBM_PEAK_GBS,
+         "build_s": round(build_s, 2),
+         "kernel": "k_gemm16<128,L2,2 query blocks,threshold> over the decoded rows",
+         "kernel_ms": sc_ms, "bound": "mfma",
+         "achieved": flop / (sc_ms * 1e-3) / 1e12 if sc_ms > 0 else None, "unit": "TFLOP/s",
+         "peak": FP16_MFMA_PEAK_TFLOPS,
+         "mfma_inputs": "f16 high halves of the decoded rows and the queries",
          "kernel_ms_per_step": {kk: v[0] / steps for kk, v in prof.items()},
-         "note": "the 16 MB of codes stay in L2 / MALL across queries: 'achieved' counts the "
-                 "codes each query reads (n m bytes), not HBM traffic"}
+         "note": "the GEMM admits candidates; their codes are scored by ADC in the select"}
     log(f"pqflat: {r['qps']:.0f} q/s, scan {sc_ms:.3f} ms per {nq} queries")
     if ref is not None:
         blob = pq.save()
@@ -874,22 +876,22 @@ def main():
 
         el, prof, _ = timed(ctx, torch, step, args.steps, args.warmup,
                             ["query_prep", "sample_gemm", "kth", "flat_gemm", "select",
-                             "exact_scan", "merge", "ivf_qtab", "ivf_scan", "rerank"])
+                             "exact_scan", "merge", "ivf_qtab", "ivf_seed", "ivf_scan",
+                             "ivf_pick", "ivf_rescan", "rerank"])
         gi, gd = gpu_out()
         s_ms = prof["ivf_scan"][0] / max(1, prof["ivf_scan"][1])
-        # algorithmic bytes of the list scan: the codes and ids of every scanned row (m + 4
-        # bytes each).  The row-sum scan reads each row's code and its 4-byte term-2 sum (ids
-        # only for the rows it scores exactly); the per-list term-2 tables the reference reads
-        # (m x 256 floats per probed list, ivf_pq.cc:197-217) are not streamed.
-        alg_bytes = scanned * (m + 4)
+        # The scan by list reads the probed lists' decoded residuals (fp16) and term-2 sums
+        # once per batch: with 10,000 queries all lists, so every row's 2 dim + 4 bytes.  The
+        # scan by query beside it reads each probed row's code and sum per query (m + 4 bytes).
+        alg_bytes = N * (2 * dim + 4)
+        query_bytes = scanned * (m + 4)
         gbs = alg_bytes / (s_ms * 1e-3) / 1e9
         r = {"qps": nq * args.steps / el, "ms_per_step": el * 1e3 / args.steps,
-             "kernel": "k_ivf_scan_rs", "kernel_ms": s_ms, "achieved": gbs, "unit": "GB/s",
+             "kernel": "k_ivf_lists<128> (with the grouping of the probes by list)",
+             "kernel_ms": s_ms, "achieved": gbs, "unit": "GB/s",
              "peak": HBM_PEAK_GBS, "bound": "hbm",
-             "algorithmic_bytes": "codes + ids of the scanned rows",
+             "algorithmic_bytes": "decoded residuals and term-2 sums of the lists, once",
              "algorithmic_bytes_per_launch": alg_bytes,
-             "stream_bytes_per_launch": scanned * (m + 4),
-             "stream_note": "codes + per-row term-2 sums (m + 4 bytes per scanned row)",
              "codes_scanned_per_query": scanned / nq,
              "kernel_ms_per_step": {kk: v[0] / args.steps for kk, v in prof.items()},
              "nlist": nlist, "m": m, "nprobe": nprobe, "rerank": rerank,
@@ -905,7 +907,7 @@ def main():
         t_ms = prof_t["ivf_scan"][0] / max(1, prof_t["ivf_scan"][1])
         r["table_scan"] = {
             "qps": nq * args.steps / el_t, "kernel": "k_ivf_scan_fast", "kernel_ms": t_ms,
-            "achieved": alg_bytes / (t_ms * 1e-3) / 1e9,
+            "achieved": query_bytes / (t_ms * 1e-3) / 1e9,
             "term2_bytes_per_launch": nq * nprobe * m * 256 * 4,
             "same_results": bool(np.array_equal(gi_t, gi) and
                                  np.array_equal(gd_t.view(np.uint32), gd.view(np.uint32)))}
@@ -949,7 +951,6 @@ def main():
                     sweep[f"nprobe{npb}_rerank{rr}"] = {
                         "qps": round(nq * args.steps / els, 1),
                         "scan_ms": round(sms, 4),
-                        "scan_GBps": round(sc * (m + 4) / (sms * 1e-3) / 1e9, 1),
                         "codes_scanned_per_query": round(sc / nq, 1)}
                     log(f"ivfpq nprobe {npb} rerank {rr}: {nq * args.steps / els:.0f} q/s")
             r["sweep"] = sweep
