@@ -179,9 +179,14 @@ int StageOut(Ctx* c, const uint8_t* const* src, const size_t* bytes, void* const
   if (nout < 1 || nout > 4) return SetError(kInternal, "StageOut: 1 to 4 regions");
   // the results land at the start of the pinned block (the inputs there have been read: the
   // copy-in kernel ran before everything queued after it)
+  size_t off = 0, total16 = 0;
+  for (int r = 0; r < nout; ++r) off += StageRound(bytes[r]);
+  // (reserved by StageIn already; a block grown here replaces stage_h, so no address is taken
+  // from it before)
+  VDBG_RETURN_IF_ERROR(StageReserve(c, off, 0, s));
   StageOutArgs a{};
   a.n = nout;
-  size_t off = 0, total16 = 0;
+  off = 0;
   for (int r = 0; r < nout; ++r) {
     a.src[r] = reinterpret_cast<const uint4*>(src[r]);
     a.dst[r] = reinterpret_cast<uint4*>(c->stage_h_dev + off);
@@ -189,7 +194,6 @@ int StageOut(Ctx* c, const uint8_t* const* src, const size_t* bytes, void* const
     total16 += a.n16[r];
     off += StageRound(bytes[r]);
   }
-  VDBG_RETURN_IF_ERROR(StageReserve(c, off, 0, s));  // (reserved by StageIn already)
   a.counter = reinterpret_cast<uint32_t*>(c->stage_d);
   std::lock_guard<std::mutex> g(c->flag_mu);
   a.flag = c->host_flag_dev;

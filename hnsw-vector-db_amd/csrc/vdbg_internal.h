@@ -621,8 +621,10 @@ inline int StageRegions(Ctx* c, const float* queries, size_t qb, const void* ext
   const void* src[2] = {queries, extra};
   const size_t bytes[2] = {qb, eb};
   uint8_t* base = nullptr;
+  uint32_t uncertified[4] = {};  // (sent out behind the results)
   VDBG_RETURN_IF_ERROR(StageIn(c, src, bytes, extra ? 2 : 1,
-                               2 * StageRound(ob) + StageRound(cb), s, &base));
+                               2 * StageRound(ob) + StageRound(cb) + StageRound(sizeof(uncertified)),
+                               s, &base));
   const size_t in_end = StageSpan(qb) + (extra ? StageSpan(eb) : 0);
   const float* dq = reinterpret_cast<const float*>(base);
   const void* dx = extra ? static_cast<const void*>(base + StageSpan(qb)) : nullptr;
@@ -637,7 +639,6 @@ inline int StageRegions(Ctx* c, const float* queries, size_t qb, const void* ext
   void* odst[4] = {out_ids, out_dists, dist_comps};
   int nout = dist_comps ? 3 : 2;
   if (nq <= kOptQueries && c->gate_fallbacks) {
-    uint32_t uncertified[4] = {};
     {
       OptCount armed(c);
       VDBG_RETURN_IF_ERROR(fn(dq, dx, di, dd, ddc, s));
