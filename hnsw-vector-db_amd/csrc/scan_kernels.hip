@@ -2461,14 +2461,24 @@ struct RowScanArgs {
   uint32_t* fb_zero;      // nullable: zeroed by block 0
 };
 
+// LDS of k_row_scan, at most the 64 KB a launch may ask for without an attribute: NQ queries
+// staged and, per wave and query, two runs of 64 keys and rows.  (5 queries: NQ 8, the widest
+// rows 816 values, 61 KB.)
+constexpr size_t RowScanStaticLds(int nq) {
+  return size_t(kTinyWaves) * nq * 2 * kWave * 8 + kRowTile / 64 * 8 + kRowTile * 2;
+}
+static_assert(RowScanStaticLds(8) + 8 * (kRowMaxQ / 5) * sizeof(float) <= 65536 &&
+                  RowScanStaticLds(4) + 4 * (kRowMaxQ / 3) * sizeof(float) <= 65536 &&
+                  RowScanStaticLds(2) + kRowMaxQ * sizeof(float) <= 65536,
+              "k_row_scan's LDS");
+
 template <int NQ, bool F16>
 __global__ __launch_bounds__(256) void k_row_scan(RowScanArgs a) {
   constexpr int W = kTinyWaves, R = 4;
   constexpr int U = F16 ? 4 : 2;  // 64-dim runs loaded at a time
+  // the staged keys; a wave's final list takes the first run of its own (lane by lane)
   __shared__ float sd[W][NQ][2 * kWave];
   __shared__ uint32_t si[W][NQ][2 * kWave];
-  __shared__ float md[W][NQ][kWave];
-  __shared__ uint32_t mi[W][NQ][kWave];
   __shared__ uint64_t s_word[kRowTile / 64];
   __shared__ uint16_t s_row[kRowTile];
   extern __shared__ float s_q[];  // [NQ][pd]
@@ -2622,8 +2632,8 @@ __global__ __launch_bounds__(256) void k_row_scan(RowScanArgs a) {
       const bool have = lane < staged[q];
       top[q].insert(have ? sd[wave][q][lane] : __builtin_inff(), have ? si[wave][q][lane] : kNoId);
     }
-    md[wave][q][lane] = top[q].k.d[0];
-    mi[wave][q][lane] = top[q].k.id[0];
+    sd[wave][q][lane] = top[q].k.d[0];
+    si[wave][q][lane] = top[q].k.id[0];
   }
   __syncthreads();
   // the four lists of query q merge in wave q % 4
@@ -2632,7 +2642,7 @@ __global__ __launch_bounds__(256) void k_row_scan(RowScanArgs a) {
     if (q >= a.nq) break;
     if ((q & (W - 1)) != wave) continue;
     for (int w = 1; w < W; ++w)
-      top[q].insert(md[(wave + w) & (W - 1)][q][lane], mi[(wave + w) & (W - 1)][q][lane]);
+      top[q].insert(sd[(wave + w) & (W - 1)][q][lane], si[(wave + w) & (W - 1)][q][lane]);
     const size_t o = size_t(q) * a.nchunks + blockIdx.x;
     if (lane < a.kp) a.part[o * a.kp + lane] = make_uint2(__float_as_uint(top[q].k.d[0]), top[q].k.id[0]);
     const float kth = __shfl(top[q].k.d[0], rl);

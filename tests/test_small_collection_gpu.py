@@ -110,3 +110,19 @@ def test_small_collection_device_results(ctx, oracle):
     assert np.array_equal(dc, want[2]) and plans == want[3]
     for ds in handles:
         ds.close()
+
+
+# the largest LDS of each query count (5 queries stage 8 x 816 floats), and one query too many
+# for the widest rows (6 x 704 floats are past what the kernel stages)
+@pytest.mark.parametrize("dim,counts", [(512, (5, 8)), (768, (5,)), (816, (5,)), (704, (5, 6)),
+                                        (1360, (3,)), (2048, (2,))])
+def test_small_collection_wide_rows(ctx, oracle, dim, counts):
+    segs, handles = build(ctx, [1500, 40, 2100], dim, "cosine", "unit", 700)
+    for i, sg in enumerate(segs):
+        sg["filter"] = mask(sg["base"].shape[0], 0.4, 80 + i)
+    for nq in counts:
+        print(f"small collection dim={dim} nq={nq}", flush=True)
+        raw = (datagen.clustered_unit(nq, dim, 83, 79, 40, 0.5) * 3).astype(np.float32)
+        run(ctx, oracle, segs, handles, dim, "cosine", raw, 10)
+    for ds in handles:
+        ds.close()
