@@ -296,6 +296,7 @@ int SmallCollection(Ctx* c, const std::vector<RowSet>& sets,
   }
   MergeArgs a{int(nq), int(n), int(k), hits_d, hits_r, nullptr, nullptr, oi, od};
   a.ext_parts = extp;
+  a.status = status;  // (a refused query leaves the caller's device results as they are)
   VDBG_RETURN_IF_ERROR(MergeParts(c, a, s));
   std::vector<int> st(nq);
   std::vector<uint64_t> ids(device_io ? 0 : slice);

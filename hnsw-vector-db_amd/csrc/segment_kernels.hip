@@ -467,6 +467,8 @@ __global__ __launch_bounds__(256) void k_merge(MergeArgs a) {
   const int wave = threadIdx.x >> 6, lane = lane_id();
   const int q = blockIdx.x * 4 + wave;
   if (q >= a.nq) return;
+  if (a.status != nullptr && __ballot(lane < a.nq && a.status[min(lane, a.nq - 1)] != 0) != 0)
+    return;
   const int total = a.nparts * a.k;
   const int ko = a.kout > 0 ? a.kout : a.k;  // results written per query
   WaveKeys<E> r;
@@ -681,6 +683,8 @@ static int MergePartsLarge(Ctx* c, const MergeArgs& a, hipStream_t s) {
 int MergeParts(Ctx* c, const MergeArgs& a, hipStream_t s) {
   if (a.nq == 0 || a.k == 0) return kOk;
   const int total = a.nparts * a.k;
+  if (a.status != nullptr && (a.nq > kWave || total > 16 * kWave))
+    return SetError(kInternal, "merge: a status of too large a batch");
   if (total > 16 * kWave) return MergePartsLarge(c, a, s);
   int e = 1;
   while (kWave * e < total) e <<= 1;

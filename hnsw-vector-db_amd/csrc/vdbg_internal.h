@@ -490,6 +490,9 @@ struct MergeArgs {
   float* out_d;
   const uint64_t* const* ext_parts = nullptr;  // or row r of part p at ext_parts[p][r]
   int kout = 0;  // results per query written to out_ext / out_d ([nq][kout]); 0: k
+  // nullable, [nq <= 64] (of hits that one wavefront's sort takes): nothing is written when the
+  // preparation refused a query of the batch
+  const int* status = nullptr;
 };
 int MergeParts(Ctx* c, const MergeArgs& a, hipStream_t s);
 // PrepareQuery + NormalizeVector for nq raw queries into padded rows; waits for the result

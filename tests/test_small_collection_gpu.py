@@ -126,3 +126,23 @@ def test_small_collection_wide_rows(ctx, oracle, dim, counts):
         run(ctx, oracle, segs, handles, dim, "cosine", raw, 10)
     for ds in handles:
         ds.close()
+
+
+@pytest.mark.parametrize("bad", [np.nan, 0.0])
+def test_small_collection_refused_query_writes_nothing(ctx, bad):
+    """A NaN or, under cosine, a zero query: the error, and the device results as they were."""
+    import torch
+    segs, handles = build(ctx, [3000, 2000], 96, "cosine", "unit", 900)
+    raw = datagen.clustered_unit(3, 96, 91, 79, 40, 0.5)
+    raw[1, :] = bad
+    q = torch.from_numpy(raw).cuda()
+    ids = torch.full((3, 10), 77, dtype=torch.int64, device="cuda")
+    d = torch.full((3, 10), 5.0, dtype=torch.float32, device="cuda")
+    with pytest.raises(vdbg.VdbgError) as e:
+        vdbg.collection_search_device(ctx, [(ds, None, None, None) for ds in handles], 96,
+                                      "cosine", q.data_ptr(), 3, 10, ids.data_ptr(), d.data_ptr())
+    assert e.value.code == 1
+    torch.cuda.synchronize()
+    assert bool((ids == 77).all()) and bool((d == 5.0).all())
+    for ds in handles:
+        ds.close()
