@@ -3503,6 +3503,7 @@ struct DeepPlan {
   uint32_t stride;  // keys kept per query
   size_t max_nq;    // queries per pass (1 GiB of keys and candidates)
 };
+constexpr size_t kDeepAllBytes = size_t(256) << 20;  // a place for every row of the batch
 static DeepPlan PlanDeep(const Ctx* c, const ScanSource& src, size_t nq, size_t kk) {
   DeepPlan p{};
   const uint32_t S = std::min(SampleWant(c, src, nq, kk), src.Smax);
@@ -3674,6 +3675,11 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
     p.caph = 32;
     while (p.caph < 3.0 * expect_seg + 32) p.caph <<= 1;
     p.nseg = 2 * p.nchunks;
+    // Rows stored by cluster put many of a deep answer into one segment.  One place per row of
+    // the half chunk, where that takes little, holds whatever the threshold admits.
+    const int all = int(p.chunk_rows / 2);
+    if (deep.on && (all <= p.caph || nq * size_t(p.nseg) * all * sizeof(uint2) <= kDeepAllBytes))
+      p.caph = all;
     return p;
   };
   // Rows with an fp16 copy may rank on the fp16 GEMM: integer-valued flat rows exactly
@@ -3961,18 +3967,12 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
     SortKeysArgs sk{dkeys, deep.stride, int(kk), out_ids, out_d, dtotal, T, shift, ebx, fb_list,
                     fb_count, c->test_fallbacks >= 1 ? 1 : 0};
     VDBG_RETURN_IF_ERROR(SortKeysTopK(c, sk, int(nq), s));
-    // uncertified queries (rare) have every row scored and sorted, one by one
+    // uncertified queries (rare, but for rows stored by cluster in batches too large for a place
+    // per row) have every row scored and sorted, side by side
     uint32_t nfb = 0;
     VDBG_RETURN_IF_ERROR(ReadWords(c, fb_count, 1, s, &nfb));
-    if (nfb == 0) return kOk;
-    std::vector<uint32_t> list(nfb);
-    VDBG_HIP(hipMemcpyAsync(list.data(), fb_list, nfb * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    VDBG_HIP(hipStreamSynchronize(s));
     c->last_fallbacks += nfb;
-    for (const uint32_t q : list)
-      VDBG_RETURN_IF_ERROR(ExactScanAll(c, *src, SQ + size_t(q) * ScorePd(*src), 1, kk, allow,
-                                        out_ids + size_t(q) * kk, out_d + size_t(q) * kk, s));
-    return kOk;
+    return ExactScanAllListed(c, *src, SQ, nq, fb_list, nfb, kk, allow, out_ids, out_d, s);
   }
   SelectArgs se{};
   se.Q = SQ;

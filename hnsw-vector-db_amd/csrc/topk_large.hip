@@ -203,6 +203,50 @@ int ExactScanAll(Ctx* c, const ScanSource& src, const float* Q, size_t nq, size_
                    nq, kk, allow, out_ids, out_d, s);
 }
 
+// The listed queries' rows of w floats, gathered.
+__global__ void k_gather_queries(const float* __restrict__ Q, int w,
+                                 const uint32_t* __restrict__ list, float* __restrict__ y) {
+  const float* src = Q + size_t(list[blockIdx.x]) * w;
+  float* dst = y + size_t(blockIdx.x) * w;
+  for (int i = threadIdx.x; i < w; i += blockDim.x) dst[i] = src[i];
+}
+// Their results, back to their places.
+__global__ void k_scatter_results(const uint32_t* __restrict__ ids, const float* __restrict__ d,
+                                  size_t kk, const uint32_t* __restrict__ list,
+                                  uint32_t* __restrict__ out_ids, float* __restrict__ out_d) {
+  const size_t from = size_t(blockIdx.x) * kk, to = size_t(list[blockIdx.x]) * kk;
+  for (size_t i = threadIdx.x; i < kk; i += blockDim.x) {
+    out_ids[to + i] = ids[from + i];
+    out_d[to + i] = d[from + i];
+  }
+}
+
+int ExactScanAllListed(Ctx* c, const ScanSource& src, const float* Q, size_t nq,
+                       const uint32_t* list, size_t n, size_t kk, const uint64_t* allow,
+                       uint32_t* out_ids, float* out_d, hipStream_t s) {
+  if (n == 0 || kk == 0) return kOk;
+  if (n == nq) return ExactScanAll(c, src, Q, nq, kk, allow, out_ids, out_d, s);
+  // parts of at most 64 MiB of gathered queries and as many of results
+  const size_t w = size_t(ScorePd(src));
+  const size_t part = std::min(n, std::max<size_t>(1, (size_t(64) << 20) / (4 * (w + 2 * kk))));
+  char* buf = nullptr;
+  VDBG_HIP(hipMallocAsync(reinterpret_cast<void**>(&buf), part * (w + 2 * kk) * 4, s));
+  float* q = reinterpret_cast<float*>(buf);
+  uint32_t* ids = reinterpret_cast<uint32_t*>(q + part * w);
+  float* d = reinterpret_cast<float*>(ids + part * kk);
+  int rc = kOk;
+  for (size_t i = 0; i < n && rc == kOk; i += part) {
+    const size_t m = std::min(part, n - i);
+    k_gather_queries<<<dim3(unsigned(m)), 256, 0, s>>>(Q, int(w), list + i, q);
+    rc = ExactScanAll(c, src, q, m, kk, allow, ids, d, s);
+    if (rc != kOk) break;
+    k_scatter_results<<<dim3(unsigned(m)), 256, 0, s>>>(ids, d, kk, list + i, out_ids, out_d);
+    if (hipGetLastError() != hipSuccess) rc = SetError(kInternal, "listed scan");
+  }
+  (void)hipFreeAsync(buf, s);
+  return rc;
+}
+
 // Rerank (src/index/index.cc:89-95) for depths beyond the wave kernel: exact distances of
 // the depth candidates per query, sorted, the first k.
 __global__ void k_rerank_keys(const float* __restrict__ X, const float* __restrict__ Q, int pd,

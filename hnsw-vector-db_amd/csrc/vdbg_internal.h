@@ -449,6 +449,10 @@ int Sq8Encode(Ctx* c, const Dataset* ds, const float* vmin_dev, const float* sca
 // per query, segmented sort.
 int ExactScanAll(Ctx* c, const ScanSource& src, const float* Q, size_t nq, size_t kk,
                  const uint64_t* allow, uint32_t* out_ids, float* out_d, hipStream_t s);
+// The same for the queries list[0, n) of nq (distinct, device memory), results in their places.
+int ExactScanAllListed(Ctx* c, const ScanSource& src, const float* Q, size_t nq,
+                       const uint32_t* list, size_t n, size_t kk, const uint64_t* allow,
+                       uint32_t* out_ids, float* out_d, hipStream_t s);
 // Rerank for depths beyond 256 candidates per query.
 int RerankLarge(Ctx* c, const float* X, int pd, int metric, const float* Q, size_t nq,
                 const uint32_t* cand, size_t depth, size_t k, uint32_t* out_ids, float* out_d,

@@ -94,3 +94,35 @@ def test_deep_sq8(ctx, oracle, n, depth):
     check(*sq.search(qs, 10, depth), oi, od)
     sq.close()
     ds.close()
+
+
+# A deep answer's rows lie together.  61 queries: the candidates' segments hold every row of
+# their half chunks, so no answer is re-scanned; 900: the segments are sized for rows in any order,
+# and the queries that overflow them are scored over every row in one batch.
+@pytest.mark.parametrize("nq", [61, 900])
+@pytest.mark.parametrize("kind", ["flat", "sq8"])
+def test_deep_rows_stored_by_cluster(ctx, oracle, nq, kind):
+    n, dim, k, per = 118385, 112, 1000, 1500
+    print(f"deep, rows by cluster, {kind} nq={nq}", flush=True)
+    rng = np.random.default_rng(95)
+    centers = rng.random((n // per + 1, dim), dtype=np.float32)
+    base = np.repeat(centers, per, axis=0)[:n]
+    base += 0.2 * rng.standard_normal((n, dim), dtype=np.float32)
+    qs = centers[rng.integers(0, n // per, nq)]
+    qs = (qs + 0.2 * rng.standard_normal((nq, dim), dtype=np.float32)).astype(np.float32)
+    qs[: nq // 2] = rng.random((nq // 2, dim), dtype=np.float32)  # (no cluster of their own)
+    at = np.r_[0:8, nq - 8 : nq]
+    ds = vdbg.Dataset(ctx, base, dim)
+    if kind == "flat":
+        gi, gd = ds.flat_search(qs, k)
+        again = ctx.last_fallbacks()
+        od, oi = oracle.flat_search(base, qs[at], k)
+    else:
+        sq = vdbg.Sq8Index(ds)
+        gi, gd = sq.search(qs, 10, k)
+        again = ctx.last_fallbacks()
+        od, oi = oracle.sq8_search(base, sq.codes(), sq.vmin, sq.scale, qs[at], 10, k)
+        sq.close()
+    check(gi[at], gd[at], oi, od)
+    assert again == 0 if nq == 61 else 0 < again < nq
+    ds.close()
