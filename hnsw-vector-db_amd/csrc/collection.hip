@@ -234,13 +234,13 @@ int CombinedScan(Ctx* c, const vdbg_segment* segs, size_t nseg, const std::vecto
 // masks and external id tables staged in one copy and the results, the queries' status and the
 // count of uncertified answers in another: six launches and one host wait, where the segments
 // scanned one by one took 112 launches (one query, eight segments of 500,000 x 384 rows in
-// all, 10% allowed: 712 -> 118 us).  *done stays false, with nothing returned, when an
-// answer was not certified: the caller then searches the segments one by one.
+// all, 10% allowed: 712 -> 118 us).  Segments with answers that were not certified are re-scanned
+// behind that, in the chunks that can hold such an answer's rows, and the parts merged again.
 int SmallCollection(Ctx* c, const std::vector<RowSet>& sets,
                     const std::vector<const uint64_t*>& allow_h,
                     const std::vector<const uint64_t*>& ext, size_t dim, size_t pd, int metric,
                     const float* queries, size_t nq, size_t k, uint64_t* out_ids,
-                    float* out_dists, bool device_io, hipStream_t s, bool* done) {
+                    float* out_dists, bool device_io, hipStream_t s) {
   const size_t n = sets.size(), slice = nq * k;
   // inputs: the external id tables, the raw queries (from the host), the sets' masks
   std::vector<const void*> src{ext.data()};
@@ -286,13 +286,13 @@ int SmallCollection(Ctx* c, const std::vector<RowSet>& sets,
   VDBG_RETURN_IF_ERROR(LaunchPrepare(c, raw, nq, dim, pd, metric, q, status, s));
   c->last_fallbacks = 0;
   c->last_gemm_gate = nullptr;
+  WsUse wuse(&c->ws, s);
+  VDBG_RETURN_IF_ERROR(wuse.status());
+  RowScanLists lists;
   {
     OptCount armed(c);
-    WsUse wuse(&c->ws, s);
-    VDBG_RETURN_IF_ERROR(wuse.status());
-    uint32_t *fl = nullptr, *fc = nullptr;
     VDBG_RETURN_IF_ERROR(RowScan(c, dev.data(), int(n), q, nq, k, hits_r, hits_d, s, c->ws,
-                                 c->fb_dev, &fl, &fc));
+                                 c->fb_dev, &lists));
   }
   MergeArgs a{int(nq), int(n), int(k), hits_d, hits_r, nullptr, nullptr, oi, od};
   a.ext_parts = extp;
@@ -301,17 +301,27 @@ int SmallCollection(Ctx* c, const std::vector<RowSet>& sets,
   std::vector<int> st(nq);
   std::vector<uint64_t> ids(device_io ? 0 : slice);
   std::vector<float> dists(device_io ? 0 : slice);
-  uint32_t uncertified[4] = {};
+  uint32_t uncertified[kRowSets] = {};
   const uint8_t* osrc[4] = {reinterpret_cast<uint8_t*>(status), c->stage_d + kStageOptWord,
                             reinterpret_cast<uint8_t*>(oi), reinterpret_cast<uint8_t*>(od)};
   const size_t obytes[4] = {nq * 4, sizeof(uncertified), slice * 8, slice * 4};
   void* const odst[4] = {st.data(), uncertified, ids.data(), dists.data()};
   VDBG_RETURN_IF_ERROR(StageOut(c, osrc, obytes, odst, device_io ? 2 : 4, s));
   VDBG_RETURN_IF_ERROR(PrepareStatusError(st.data(), nq));
-  if (uncertified[0] != 0) return kOk;
+  bool again = false;
+  for (size_t i = 0; i < n; ++i) {
+    if (uncertified[i] == 0) continue;
+    const OptRescan r{dev[i].src,           q,       k, dev[i].allow, hits_r + i * slice,
+                      hits_d + i * slice, &c->ws2, lists.list + i * nq, lists.prune[i]};
+    VDBG_RETURN_IF_ERROR(RunOptRescan(c, r, uncertified[i], s));
+    again = true;
+  }
+  if (again) {
+    VDBG_RETURN_IF_ERROR(MergeParts(c, a, s));
+    if (!device_io) VDBG_RETURN_IF_ERROR(StageOut(c, osrc + 2, obytes + 2, odst + 2, 2, s));
+  }
   std::copy(ids.begin(), ids.end(), out_ids);
   std::copy(dists.begin(), dists.end(), out_dists);
-  *done = true;
   return kOk;
 }
 
@@ -492,15 +502,12 @@ int CollectionSearch(vdbg_ctx* ctx, const vdbg_segment* segs, size_t nseg, size_
       ext.push_back(g.rows->d.ext_ids);
     }
     if (ok && !sets.empty()) {
-      bool done = false;
       VDBG_RETURN_IF_ERROR(SmallCollection(c, sets, allow_h, ext, dim, pd, metric, queries, nq, k,
-                                           out_ids, out_dists, device_io, s, &done));
-      if (done) {
-        count_scans();
-        if (seg_plans != nullptr)
-          for (size_t p = 0; p < nseg; ++p) seg_plans[p] = plan[p].plan;
-        return kOk;
-      }
+                                           out_ids, out_dists, device_io, s));
+      count_scans();
+      if (seg_plans != nullptr)
+        for (size_t p = 0; p < nseg; ++p) seg_plans[p] = plan[p].plan;
+      return kOk;
     }
   }
 

@@ -1666,6 +1666,7 @@ struct ScanArgs {
   uint2* part;            // [slot][split][64*E]
   uint32_t* part_counts;  // [slot][split]
   const uint32_t* nslots_dev;  // nullable: slots at or past *nslots_dev are not scanned
+  ScanPrune prune;        // keys null: every split is scanned
 };
 
 // Grid of a gated exact re-scan pass (two blocks per CU of a 256-CU part).
@@ -1689,16 +1690,59 @@ __device__ __forceinline__ void exact_scan_item(const ScanArgs& a, const Scorer&
   const uint32_t r1 = min(a.N, r0 + a.split_rows);
   WaveTopK<E> top;
   top.init();
-  for (uint32_t base = r0 + wave * kWave; base < r1; base += 4 * kWave) {
-    const uint32_t r = base + lane;
-    float d = __builtin_inff();
-    uint32_t id = kNoId;
-    if (r < r1 && row_allowed(a.allow, r)) {
-      d = sc(qv, r);
-      id = r;
+  bool listed = false;
+  if (a.prune.keys != nullptr) {
+    // The split is a chunk of the scan whose answer was not certified.  A key above the k-th
+    // distance found by more than its error (the merge's certificate) keeps its row out of the
+    // answer: the chunk is left out when its smallest key does, and only its listed rows below
+    // that are scored when its bound does.
+    const ScanPrune& p = a.prune;
+    const size_t at = size_t(q) * p.stride + split;
+    const uint2* keys = p.keys + at * p.kp;
+    const float eb = p.eb[q], shift = p.shift[q], Qd = p.Qd != nullptr ? float(p.Qd[q]) : 0.f;
+    const bool fits = p.fits != nullptr ? p.fits[q] != 0 : eb < __builtin_inff();
+    const float dk = p.dist[size_t(q) * p.k + p.k - 1];
+    auto behind = [&](float v) { return fits && dk < (v - Qd + shift) - eb; };
+    const uint2 f = keys[0];
+    if (behind(f.y == kNoId ? __builtin_inff() : __uint_as_float(f.x))) {  // (block-uniform)
+      if (threadIdx.x == 0) a.part_counts[size_t(slot) * a.nsplit + split] = 0;
+      return;
     }
-    top.insert(d, id);
+    listed = behind(p.bound[at]);
+    if (listed && wave == 0) {
+      uint32_t id = kNoId;
+      if (lane < p.kp && !behind(__uint_as_float(keys[lane].x))) id = keys[lane].y;
+      float d = __builtin_inff();
+      bool grouped = false;
+      if constexpr (std::is_same<Scorer, FlatScorer>::value) {
+        if (sc.kset == kKsetAvx512) {  // eight lanes a row
+          grouped = true;
+          const int n = __popcll(__ballot(id != kNoId));  // (the list's first: it is sorted)
+          group_pass(id, 0, n, d, [&](const auto& ids, auto& dd) {
+            constexpr int R = sizeof(dd) / sizeof(float);
+            const float* xs[R];
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+              xs[i] = sc.X + size_t(sc.map != nullptr ? sc.map[ids[i]] : ids[i]) * sc.pd;
+            metric_exact_g8n<R>(sc.metric, qv, xs, sc.pd, dd);
+          });
+        }
+      }
+      if (!grouped && id != kNoId) d = sc(qv, id);
+      top.insert(id != kNoId ? d : __builtin_inff(), id);
+    }
   }
+  if (!listed)
+    for (uint32_t base = r0 + wave * kWave; base < r1; base += 4 * kWave) {
+      const uint32_t r = base + lane;
+      float d = __builtin_inff();
+      uint32_t id = kNoId;
+      if (r < r1 && row_allowed(a.allow, r)) {
+        d = sc(qv, r);
+        id = r;
+      }
+      top.insert(d, id);
+    }
   if (wave > 0) {
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -2054,14 +2098,19 @@ struct ExactPlan {
   uint32_t split_rows;
   size_t need;
 };
-static ExactPlan PlanExact(uint32_t N, int nslots, size_t k) {
+static ExactPlan PlanExact(uint32_t N, int nslots, size_t k, const ScanPrune* prune = nullptr) {
   ExactPlan p{};
-  int nsplit = int(std::min<size_t>((2048 + nslots - 1) / nslots,
-                                    std::max<size_t>(1, (N + 1023) / 1024)));
-  nsplit = std::max(1, std::min(nsplit, kMaxSeg));
-  p.split_rows = (N + nsplit - 1) / nsplit;
-  p.split_rows = (p.split_rows + 63) / 64 * 64;
-  p.nsplit = int((N + p.split_rows - 1) / p.split_rows);
+  if (prune != nullptr) {
+    p.split_rows = prune->split_rows;
+    p.nsplit = prune->nsplit;
+  } else {
+    int nsplit = int(std::min<size_t>((2048 + nslots - 1) / nslots,
+                                      std::max<size_t>(1, (N + 1023) / 1024)));
+    nsplit = std::max(1, std::min(nsplit, kMaxSeg));
+    p.split_rows = (N + nsplit - 1) / nsplit;
+    p.split_rows = (p.split_rows + 63) / 64 * 64;
+    p.nsplit = int((N + p.split_rows - 1) / p.split_rows);
+  }
   const int cap = kWave * pow2_e(k);
   p.need = size_t(nslots) * p.nsplit * cap * sizeof(uint2) +
            size_t(nslots) * p.nsplit * sizeof(uint32_t) + 4096;
@@ -2072,10 +2121,12 @@ template <class Scorer>
 static int ExactScanT(Ctx* c, Workspace& w, const ScanSource& src, const Scorer& sc,
                       const float* Q, const uint32_t* qlist, int nslots, size_t k,
                       const uint64_t* allow, uint32_t* out_ids, float* out_d, hipStream_t s,
-                      const uint32_t* nslots_dev = nullptr, uint32_t* fb_acc = nullptr) {
+                      const uint32_t* nslots_dev = nullptr, uint32_t* fb_acc = nullptr,
+                      const ScanPrune* prune = nullptr) {
   const int E = pow2_e(k);
   const uint32_t N = src.N;
-  const ExactPlan ep = PlanExact(N, nslots, k);
+  const ExactPlan ep = PlanExact(N, nslots, k, prune);
+  if (ep.nsplit > kMaxSeg) return SetError(kInternal, "exact scan: too many row splits");
   const int nsplit = ep.nsplit;
   const uint32_t split_rows = ep.split_rows;
   const int cap = kWave * E;
@@ -2087,7 +2138,8 @@ static int ExactScanT(Ctx* c, Workspace& w, const ScanSource& src, const Scorer&
   uint2* part = w.take<uint2>(size_t(nslots) * nsplit * cap);
   uint32_t* pc = w.take<uint32_t>(size_t(nslots) * nsplit);
   const int spd = ScorePd(src);
-  ScanArgs sa{Q, allow, spd, N, qlist, nslots, split_rows, nsplit, part, pc, nslots_dev};
+  ScanArgs sa{Q, allow, spd, N, qlist, nslots, split_rows, nsplit, part, pc, nslots_dev,
+              prune != nullptr ? *prune : ScanPrune{}};
   {
     ProfScope ps(c, "exact_scan", s);
     VDBG_DISPATCH_ES(E, launch_scan, Scorer, s, sa, sc);
@@ -2119,12 +2171,13 @@ static int ExactScanT(Ctx* c, Workspace& w, const ScanSource& src, const Scorer&
 static int ExactScan(Ctx* c, Workspace& w, const ScanSource& src, const float* Q,
                      const uint32_t* qlist, int nslots, size_t k, const uint64_t* allow,
                      uint32_t* out_ids, float* out_d, hipStream_t s,
-                     const uint32_t* nslots_dev = nullptr, uint32_t* fb_acc = nullptr) {
+                     const uint32_t* nslots_dev = nullptr, uint32_t* fb_acc = nullptr,
+                     const ScanPrune* prune = nullptr) {
   if (nslots == 0) return kOk;
   if (pow2_e(k) > 4) return SetError(kNotSupported, "k > 256 is not supported on the GPU path");
   if (src.kind == 0)
     return ExactScanT(c, w, src, FlatOf(src, c->kset), Q, qlist, nslots, k, allow, out_ids, out_d,
-                      s, nslots_dev, fb_acc);
+                      s, nslots_dev, fb_acc, prune);
   if (src.kind == 2)
     return ExactScanT(c, w, src, PqScorer{src.C, src.pq_m}, Q, qlist, nslots, k, allow, out_ids,
                       out_d, s, nslots_dev, fb_acc);
@@ -2258,7 +2311,7 @@ struct TinyArgs {
   uint32_t N, chunk_rows;
   uint2* part;            // [q][chunk][kp] (key bits, row)
   float* bound;           // [q][chunk] the chunk's kp-th key, +inf when not full
-  uint32_t* fb_count;     // [2] zeroed by the scan's block 0; [1] counts finished merges
+  uint32_t* fb_count;     // [1] zeroed by the scan's block 0
   int nchunks;            // the scan's blocks
   uint32_t* fb_zero;      // nullable: the call's device fallback count, zeroed by block 0
 };
@@ -2277,7 +2330,7 @@ __global__ __launch_bounds__(kTinyWaves * 64) void k_tiny_scan(TinyArgs a) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = lane_id();
   constexpr int vpr = VPR;             // 16-byte vectors per row (pd / 16)
   int4* tile = tile_all + size_t(wave) * kWave * (vpr + 1);
-  if (blockIdx.x == 0 && tid < 2) a.fb_count[tid] = 0;
+  if (blockIdx.x == 0 && tid == 0) *a.fb_count = 0;
   if (blockIdx.x == 0 && tid == 0 && a.fb_zero != nullptr) *a.fb_zero = 0;
   const int pw = a.pd / 4;
   for (int e = tid; e < NQ * pw; e += kTinyWaves * 64) {
@@ -2457,7 +2510,7 @@ struct RowScanArgs {
   uint2* part;            // [q][chunk][kp] (key bits, row)
   float* bound;           // [q][chunk]
   int nchunks;
-  uint32_t* fb_count;     // [2] zeroed by block 0
+  uint32_t* fb_count;     // [nsets] zeroed by block 0
   uint32_t* fb_zero;      // nullable: zeroed by block 0
 };
 
@@ -2484,7 +2537,7 @@ __global__ __launch_bounds__(256) void k_row_scan(RowScanArgs a) {
   extern __shared__ float s_q[];  // [NQ][pd]
   const int tid = threadIdx.x, wave = tid >> 6, lane = lane_id();
   const int g = lane >> 3, j = lane & 7;
-  if (blockIdx.x == 0 && tid < 2) a.fb_count[tid] = 0;
+  if (blockIdx.x == 0 && tid < a.nsets) a.fb_count[tid] = 0;
   if (blockIdx.x == 0 && tid == 0 && a.fb_zero != nullptr) *a.fb_zero = 0;
   int p = 0;
   while (p + 1 < a.nsets && int(blockIdx.x) >= a.set[p + 1].chunk0) ++p;
@@ -2939,8 +2992,8 @@ struct TinyMergeArgs {
   int nchunks, kp, k;     // nchunks: of all sets
   uint32_t* out_ids;      // [set][q][k]
   float* out_d;
-  uint32_t* fb_list;      // set * nq + q of every uncertified answer (null: only counted)
-  uint32_t* fb_count;
+  uint32_t* fb_list;      // [set][nq] the queries without a certified answer,
+  uint32_t* fb_count;     // [set] and their number
   int force_fallback;
 };
 
@@ -3175,8 +3228,8 @@ __global__ __launch_bounds__(kMergeWaves * 64 + 64) void k_tiny_merge(TinyMergeA
     a.out_d[slot * a.k + lane] = r.d[0];
   }
   if (lane == 0 && !certified) {
-    const uint32_t at = atomicAdd(a.fb_count, 1u);
-    if (a.fb_list != nullptr) a.fb_list[at] = uint32_t(slot);
+    const int set = I8 ? 0 : blockIdx.y;
+    a.fb_list[size_t(set) * pa.nq + atomicAdd(a.fb_count + set, 1u)] = uint32_t(q);
   }
 }
 
@@ -3232,24 +3285,36 @@ static void launch_small(hipStream_t s, int blocks, const TinyArgs& a) {
   }
 }
 
-// The exact re-scan of a small batch's uncertified queries: queued for every query and gated on
-// the device count, or sized from a host read of it.
+// The exact re-scan of a small batch's uncertified queries, over the chunks that can still hold
+// one of their rows (ScanPrune): queued for every query and gated on the device count, or sized
+// from a host read of it.  Rows repeated 100 times fail every certificate; scoring every row for
+// them took a search of 1M x 128 integer rows 510 us (1 query) and 2,560 us (32), the chunks
+// alone take it 108 and 151, and 200,000 x 384 float rows, one query, 318 and 110.
 static int SmallFallback(Ctx* c, const ScanSource& src, const float* Q, size_t nq, size_t kk,
                          const uint64_t* allow, uint32_t* out_ids, float* out_d, hipStream_t s,
                          Workspace& W2, const uint32_t* fb_list, const uint32_t* fb_count,
-                         bool gated) {
-  // a host call reads the count with its results and runs again when it is not zero
-  if (c->opt_count != nullptr) return kOk;
+                         bool gated, const ScanPrune& prune) {
+  if (c->opt_count != nullptr) {  // a host call reads the count with its results
+    c->opt_rescan = {&src, Q, kk, allow, out_ids, out_d, &W2, fb_list, prune};
+    return kOk;
+  }
   if (gated) {
     VDBG_RETURN_IF_ERROR(ExactScan(c, W2, src, Q, fb_list, int(nq), kk, allow, out_ids, out_d, s,
-                                   fb_count, c->fb_dev));
+                                   fb_count, c->fb_dev, &prune));
     c->fb_dev_used = true;
     return kOk;
   }
   uint32_t nfb = 0;
   VDBG_RETURN_IF_ERROR(ReadWords(c, fb_count, 1, s, &nfb));
   c->last_fallbacks += nfb;
-  return ExactScan(c, W2, src, Q, fb_list, int(nfb), kk, allow, out_ids, out_d, s);
+  return ExactScan(c, W2, src, Q, fb_list, int(nfb), kk, allow, out_ids, out_d, s, nullptr, nullptr,
+                   &prune);
+}
+
+int RunOptRescan(Ctx* c, const OptRescan& r, uint32_t n, hipStream_t s) {
+  c->last_fallbacks += n;
+  return ExactScan(c, *r.ws, *r.src, r.Q, r.list, int(n), r.kk, r.allow, r.out_ids, r.out_d, s,
+                   nullptr, nullptr, &r.prune);
 }
 
 static int TinyScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
@@ -3295,7 +3360,7 @@ static int TinyScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t k
   int* fit8q = W.take<int>(nq);
   int8_t* Q8 = W.take<int8_t>(nq * size_t(pd));
   uint32_t* fb_list = W.take<uint32_t>(nq);
-  uint32_t* fb_count = W.take<uint32_t>(2);
+  uint32_t* fb_count = W.take<uint32_t>(1);
   c->last_gemm_bits = 8;
   PrepArgs pa{Q, nullptr, int(nq), pd, src->kind, src->metric, src->stats, src->rmag,
               src->vmin, src->scale, shift, eb, exact, nullptr, nullptr, nullptr,
@@ -3320,7 +3385,7 @@ static int TinyScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t k
   ma.k = int(kk);
   ma.out_ids = out_ids;
   ma.out_d = out_d;
-  ma.fb_list = c->opt_count != nullptr ? nullptr : fb_list;
+  ma.fb_list = fb_list;
   ma.fb_count = c->opt_count != nullptr ? c->opt_count : fb_count;
   ma.force_fallback = c->test_fallbacks;
   {
@@ -3328,7 +3393,10 @@ static int TinyScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t k
     k_tiny_merge<true><<<dim3(unsigned(nq)), kMergeWaves * 64 + 64, 0, s>>>(ma);
     VDBG_HIP(hipGetLastError());
   }
-  return SmallFallback(c, *src, Q, nq, kk, allow, out_ids, out_d, s, W2, fb_list, fb_count, gated);
+  const ScanPrune prune{part, bound, size_t(nchunks), kp, nchunks, small ? chunk * kSmallWaves : chunk,
+                        shift, eb, Qd, fit8q, out_d, int(kk)};
+  return SmallFallback(c, *src, Q, nq, kk, allow, out_ids, out_d, s, W2, fb_list, fb_count, gated,
+                       prune);
 }
 
 template <int NQ>
@@ -3374,7 +3442,7 @@ bool SmallBatch(const Ctx* c, const ScanSource& src, size_t nq, size_t kk) {
 
 int RowScan(Ctx* c, const RowSet* sets, int nsets, const float* Q, size_t nq, size_t kk,
             uint32_t* out_ids, float* out_d, hipStream_t s, Workspace& W, uint32_t* fb_zero,
-            uint32_t** fb_list, uint32_t** fb_count) {
+            RowScanLists* out) {
   if (nsets < 1 || nsets > kRowSets) return SetError(kInternal, "row scan: 1..16 row sets");
   const ScanSource& s0 = *sets[0].src;
   const int pd = s0.pd;
@@ -3424,8 +3492,8 @@ int RowScan(Ctx* c, const RowSet* sets, int nsets, const float* Q, size_t nq, si
   float* Qf = W.take<float>(slots);
   uint16_t* Q16 = W.take<uint16_t>(slots * 2 * pd);
   int* all16 = W.take<int>(2);
-  *fb_list = W.take<uint32_t>(slots);
-  *fb_count = W.take<uint32_t>(2);
+  uint32_t* fb_list = W.take<uint32_t>(slots);
+  uint32_t* fb_count = W.take<uint32_t>(kRowSets);
   ra.nsets = nsets;
   ra.Q = Q;
   ra.nq = int(nq);
@@ -3433,7 +3501,7 @@ int RowScan(Ctx* c, const RowSet* sets, int nsets, const float* Q, size_t nq, si
   ra.metric = s0.metric == 0 ? 0 : 1;
   ra.kp = kp;
   ra.nchunks = chunks;
-  ra.fb_count = *fb_count;
+  ra.fb_count = fb_count;
   ra.fb_zero = fb_zero;
   c->last_gemm_bits = f16 ? 16 : 32;
   {
@@ -3464,14 +3532,20 @@ int RowScan(Ctx* c, const RowSet* sets, int nsets, const float* Q, size_t nq, si
   ma.k = int(kk);
   ma.out_ids = out_ids;
   ma.out_d = out_d;
-  ma.fb_list = c->opt_count != nullptr ? nullptr : *fb_list;
-  ma.fb_count = c->opt_count != nullptr ? c->opt_count : *fb_count;
+  ma.fb_list = fb_list;
+  ma.fb_count = c->opt_count != nullptr ? c->opt_count : fb_count;
   ma.force_fallback = c->test_fallbacks;
   {
     ProfScope ps(c, "select", s);
     k_tiny_merge<false><<<dim3(unsigned(nq), unsigned(nsets)), kMergeWaves * 64 + 64, 0, s>>>(ma);
     VDBG_HIP(hipGetLastError());
   }
+  out->list = fb_list;
+  out->count = fb_count;
+  for (int i = 0; i < nsets; ++i)
+    out->prune[i] = {ra.part + size_t(ma.set[i].chunk0) * kp, ra.bound + ma.set[i].chunk0,
+                     size_t(chunks), kp, ma.set[i].nchunks, ra.set[i].chunk_rows, shift + i * nq, eb + i * nq, nullptr,
+                     nullptr, out_d + i * nq * kk, int(kk)};
   return kOk;
 }
 
@@ -3542,10 +3616,10 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
     WsUse wuse(&W, s);
     VDBG_RETURN_IF_ERROR(wuse.status());
     const RowSet set{src, allow};
-    uint32_t *fb_list = nullptr, *fb_count = nullptr;
-    VDBG_RETURN_IF_ERROR(RowScan(c, &set, 1, Q, nq, kk, out_ids, out_d, s, W, zero, &fb_list,
-                                 &fb_count));
-    return SmallFallback(c, *src, Q, nq, kk, allow, out_ids, out_d, s, W2, fb_list, fb_count, gated);
+    RowScanLists lists;
+    VDBG_RETURN_IF_ERROR(RowScan(c, &set, 1, Q, nq, kk, out_ids, out_d, s, W, zero, &lists));
+    return SmallFallback(c, *src, Q, nq, kk, allow, out_ids, out_d, s, W2, lists.list, lists.count,
+                         gated, lists.prune[0]);
   }
   // the GEMM path clears the device count in its init kernel (no launch of its own)
   const bool main_path = !tiny && nq > 0 && kk > 0 && kk <= 240 && src->N >= 1024 &&

@@ -286,9 +286,14 @@ int CompactScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
   cs.Sbuf = nullptr;
   // only as many sample rows as this one scan uses
   int rc = GatherSample(c, &cs, s, sample, SampleWant(c, cs, nq, kk));
-  if (rc == kOk)
+  if (rc == kOk) {
+    // (a re-scan behind the results would name compacted rows: it is queued, ahead of the map)
+    uint32_t* armed = c->opt_count;
+    if (armed != nullptr) c->opt_count = nullptr;  // (never set while lanes run)
     rc = RunScan(c, &cs, Q, nq, kk, nullptr, out_ids, out_d, s,
                  lane != nullptr ? &lane->ws : nullptr, lane != nullptr ? &lane->ws2 : nullptr);
+    if (armed != nullptr) c->opt_count = armed;
+  }
   if (rc == kOk) {
     k_map_ids<<<dim3(unsigned((nq * kk + 255) / 256)), 256, 0, s>>>(out_ids, nq * kk, ids);
     if (hipGetLastError() != hipSuccess) rc = SetError(kInternal, "map ids launch");

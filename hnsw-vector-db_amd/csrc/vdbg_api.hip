@@ -71,10 +71,10 @@ int WaitWords(Ctx* c, uint32_t seq, const uint32_t* dev, int n, hipStream_t s) {
 // ------------------------------------------------------------ host staging
 
 // Inputs: the device reads the mapped pinned block (16-byte vectors, grid-strided); the call's
-// count of uncertified answers (Ctx::opt_count) starts at zero.
+// counts of uncertified answers (Ctx::opt_count) start at zero.
 __global__ void k_stage_in(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t n16,
                            uint32_t* __restrict__ zero) {
-  if (blockIdx.x == 0 && threadIdx.x < 4) zero[threadIdx.x] = 0;
+  if (blockIdx.x == 0 && threadIdx.x < kRowSets) zero[threadIdx.x] = 0;
   const size_t step = size_t(gridDim.x) * blockDim.x;
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n16; i += step)
     dst[i] = src[i];

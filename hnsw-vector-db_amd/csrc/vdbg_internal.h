@@ -105,6 +105,37 @@ struct ProfEntry {
 
 struct ScanScratch;  // below
 
+struct ScanSource;
+constexpr int kRowSets = 16;  // row sets of one RowScan
+// The key lists of a small batch's scan (k_tiny_scan, k_small_scan, k_row_scan), which tell the
+// exact re-scan of its uncertified answers the chunks it may leave out, and those whose listed
+// rows are all it has to score.
+struct ScanPrune {
+  const uint2* keys = nullptr;  // [q][chunk][kp] (key bits, row), smallest first
+  const float* bound = nullptr; // [q][chunk]: no row left out of a list has a smaller key
+  size_t stride = 0;            // chunks of one q (of every row set)
+  int kp = 0, nsplit = 0;       // this set's chunks, of split_rows rows each
+  uint32_t split_rows = 0;
+  const float* shift = nullptr; // [q] distance = key - Qd + shift, within eb
+  const float* eb = nullptr;
+  const int* Qd = nullptr;      // nullable
+  const int* fits = nullptr;    // [q] eb holds (null: where it is finite)
+  const float* dist = nullptr;  // [q][k] the merge's answers
+  int k = 0;
+};
+
+struct OptRescan {
+  const ScanSource* src = nullptr;
+  const float* Q = nullptr;
+  size_t kk = 0;
+  const uint64_t* allow = nullptr;
+  uint32_t* out_ids = nullptr;
+  float* out_d = nullptr;
+  Workspace* ws = nullptr;
+  const uint32_t* list = nullptr;
+  ScanPrune prune;
+};
+
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -131,11 +162,12 @@ struct Ctx {
   std::vector<uint8_t*> stage_h_retired;
   uint8_t* stage_d = nullptr;
   size_t stage_d_cap = 0;
-  // set while a host call runs a small batch (StageRegions): its merges only count uncertified
-  // answers here (a word of the device block, zeroed by the copy-in kernel), no re-scan is
-  // queued, and the host, which reads the word with the results, runs the call again without
-  // it when it is not zero
+  // set while a host call runs a small batch (StageRegions, SmallCollection): its merges count
+  // uncertified answers here (kRowSets words of the device block, zeroed by the copy-in kernel),
+  // no re-scan is queued, and the host, which reads the words with the results, re-scans what
+  // they name; opt_rescan is what a flat search's re-scan takes
   uint32_t* opt_count = nullptr;
+  OptRescan opt_rescan;
   std::mutex flag_mu;  // one readback through host_flag at a time (scan lanes may run on
                        // worker threads of one call)
   std::mutex prof_mu;  // guards pending / free_events against those threads
@@ -397,9 +429,13 @@ int RunScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t kk,
             const uint64_t* allow, uint32_t* out_ids, float* out_d, hipStream_t s,
             Workspace* ws = nullptr, Workspace* ws2 = nullptr);
 // At most 8 queries, kk <= 48, over up to kRowSets row sets at once (k_row_scan and its merge):
-// out [set][nq][kk]; *fb_list / *fb_count (in W) receive the uncertified answers, set * nq + q
-// each, which the caller re-scans.  Sets share pd, metric and the form their rows are read in.
-constexpr int kRowSets = 16;
+// out [set][nq][kk]; *lists (arrays in W) names the uncertified answers, which the caller
+// re-scans.  Sets share pd, metric and the form their rows are read in.
+struct RowScanLists {
+  uint32_t* list;             // [set][nq] queries
+  uint32_t* count;            // [set] (Ctx::opt_count in its place while that is set)
+  ScanPrune prune[kRowSets];
+};
 struct RowSet {
   const ScanSource* src;
   const uint64_t* allow;  // nullable, device words
@@ -412,7 +448,7 @@ bool RowScanLike(const Ctx* c, const ScanSource& a, const ScanSource& b);
 bool SmallBatch(const Ctx* c, const ScanSource& src, size_t nq, size_t kk);
 int RowScan(Ctx* c, const RowSet* sets, int nsets, const float* Q, size_t nq, size_t kk,
             uint32_t* out_ids, float* out_d, hipStream_t s, Workspace& W, uint32_t* fb_zero,
-            uint32_t** fb_list, uint32_t** fb_count);
+            RowScanLists* lists);
 // Top-kk by the source's exact score without a ranking GEMM: every allowed row scored, wave
 // top-k per row split then a merge (kk <= 240), or a segmented sort (kk up to 10,000).
 int ScoreScan(Ctx* c, const ScanSource& src, const float* Q, size_t nq, size_t kk,
@@ -591,12 +627,16 @@ inline int ScorePd(const ScanSource& src) { return src.kind == 2 ? src.pq_m * 25
 constexpr size_t kStageAlign = 256;
 constexpr size_t kStageOptWord = 128;  // Ctx::opt_count's place in the device block's header
 // Host calls of at most this many queries go without queued re-scans (the two gated launches
-// cost a lone query 9 of its 82 us; one uncertified query of the batch costs it a second run).
+// cost a lone query 9 of its 82 us); uncertified queries of a flat search are re-scanned behind
+// the first read of the results, those of an IVF-PQ search's coarse probe cost it a second run.
 constexpr size_t kOptQueries = 32;
+// The exact re-scan of r's n listed queries, queued on s.
+int RunOptRescan(Ctx* c, const OptRescan& r, uint32_t n, hipStream_t s);
 // Arms Ctx::opt_count for one host call's queued work.
 struct OptCount {
   Ctx* c;
   explicit OptCount(Ctx* ctx) : c(ctx) {
+    c->opt_rescan = OptRescan{};
     c->opt_count = reinterpret_cast<uint32_t*>(c->stage_d + kStageOptWord);
   }
   ~OptCount() { c->opt_count = nullptr; }
@@ -655,6 +695,10 @@ inline int StageRegions(Ctx* c, const float* queries, size_t qb, const void* ext
     odst[nout] = uncertified;
     VDBG_RETURN_IF_ERROR(StageOut(c, osrc, obytes, odst, nout + 1, s));
     if (uncertified[0] == 0) return kOk;
+    if (c->opt_rescan.out_ids == di) {  // the scan's answers are the call's
+      VDBG_RETURN_IF_ERROR(RunOptRescan(c, c->opt_rescan, uncertified[0], s));
+      return StageOut(c, osrc, obytes, odst, nout, s);
+    }
   }
   VDBG_RETURN_IF_ERROR(fn(dq, dx, di, dd, ddc, s));
   return StageOut(c, osrc, obytes, odst, nout, s);

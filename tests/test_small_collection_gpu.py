@@ -1,8 +1,8 @@
 """Collection searches of at most 8 queries over flat segments (every segment scored in one
 launch under its mask) against the oracle's composition of the per-segment searches: segments
 of one row to several chunks, empty ones and empty filters, ids held by two segments, the
-largest number of segments and one more, and the segment-by-segment search behind an
-uncertified answer."""
+largest number of segments and one more, and the re-scan of the segments behind uncertified
+answers."""
 import numpy as np
 import pytest
 
@@ -74,7 +74,7 @@ def test_small_collection(ctx, oracle, sizes, dim, metric, data):
             raw = datagen.clustered_unit(nq, dim, int(rng.integers(1000)), 79, 40, 0.5) * 3
             raw = raw.astype(np.float32)
         run(ctx, oracle, segs, handles, dim, metric, raw, k)
-        try:  # no answer certified: the segments one by one
+        try:  # no answer certified: every segment re-scanned
             ctx.set_test_fallbacks(1)
             run(ctx, oracle, segs, handles, dim, metric, raw, k)
         finally:
