@@ -197,7 +197,8 @@ void FreePqFlat(PqFlatIndex* x) {
 
 // Makes the decoded rows the ranking GEMM reads (the codes are in place).  Without them, for
 // padded dims with no GEMM kernel, segments below the GEMM path's 1,024 rows, non-finite
-// codebooks or when memory is short, searches score every code.
+// codebooks or where they would take more than a quarter of the free memory (they are 2 pd / m
+// times the codes, and later segments need room), searches score every code.
 int MakeDecoded(Ctx* c, PqFlatIndex* x, hipStream_t s) {
   const size_t n = x->ds->n, pd = x->ds->pd;
   if (n < kRankRows || !GemmSupported(pd)) return kOk;
@@ -211,6 +212,12 @@ int MakeDecoded(Ctx* c, PqFlatIndex* x, hipStream_t s) {
     int ex = 0;
     (void)std::frexp(ma, &ex);
     e = 15 - ex;
+  }
+  size_t mem_free = 0, mem_all = 0;
+  if (hipMemGetInfo(&mem_free, &mem_all) != hipSuccess ||
+      n * (pd * sizeof(uint16_t) + sizeof(float)) > mem_free / 4) {
+    (void)hipGetLastError();
+    return kOk;
   }
   uint32_t* max_norm = nullptr;
   const bool got =

@@ -73,7 +73,8 @@ const char* vdbg_last_error(void);
 /* ---------------------------------------------------------------- context */
 
 /* A device, its stream and reusable device workspace.  Replaces nothing in the reference
- * (vdb's CPU indexes need no device state); owned by the GPU Index adapters. */
+ * (vdb's CPU indexes need no device state); owned by the GPU Index adapters.  Up to 512 MiB of
+ * the scratch of large calls stay mapped between calls; all of it goes back with the context. */
 int vdbg_ctx_create(int device, vdbg_ctx** out);
 /* Fails (VDBG_INVALID_ARGUMENT, nothing released) while datasets of the context remain:
  * destroy indexes, then datasets, then the context. */
@@ -120,8 +121,10 @@ int vdbg_ctx_set_int8_float_min_work(vdbg_ctx* ctx, double work);
  * on, each row is ranked by its term-2 sum, kept per row (4 bytes per row, made when the index
  * is loaded or built), plus the query's table, and the rows near the running threshold are
  * scored exactly as the reference scores them; off, each probed list's table
- * fl(term2 + qtab) is built per query and every code scored on it.  Results are identical
- * either way.  No counterpart in the reference. */
+ * fl(term2 + qtab) is built per query and every code scored on it.  Indexes of up to 128 padded
+ * dims with 4, 8 or 16 bytes a code also keep their decoded residuals as fp16 (2 x padded dim
+ * bytes a row, where that is at most a quarter of the free memory), which large batches rank on
+ * list by list while it is on.  Results are identical either way.  No counterpart in the reference. */
 int vdbg_ctx_set_ivf_row_sums(vdbg_ctx* ctx, int enable);
 
 /* Host threads for the CPU side of a search (the HNSW walk); n <= 0 restores the default:
@@ -451,7 +454,10 @@ typedef struct vdbg_pqflat vdbg_pqflat;
 /* PqFlatIndex::build (src/index/quant/ivf_pq.cc:45-57): ProductQuantizer::train over every row
  * (pq.cc:14-41: per subspace a strided sample of at most 256 x max_points_per_centroid rows,
  * k-means seeded with seed + 7919 j) and every row encoded, on the GPU.  pq_m must divide the
- * dimension (InvalidArgument otherwise, index.cc:27-29).  vdb builds with kmeans_iters 25. */
+ * dimension (InvalidArgument otherwise, index.cc:27-29).  vdb builds with kmeans_iters 25.
+ * Built and loaded indexes also keep the rows their codes decode to, as fp16 (2 x padded dim + 4
+ * bytes a row of device memory), where searches rank on them, unless that is more than a quarter
+ * of the free memory. */
 int vdbg_pqflat_build(vdbg_dataset* ds, size_t pq_m, uint64_t seed,
                       size_t max_points_per_centroid, size_t kmeans_iters, vdbg_pqflat** out);
 /* LoadIndex of a VDBPQFL1 file (index.cc:38-87) and PqFlatIndex::load (ivf_pq.cc:89-98):

@@ -75,3 +75,35 @@ def test_duplicate_codes_and_fallbacks(ctx, oracle):
     assert np.array_equal(ids[keep], oi[keep])
     ix.close()
     ds.close()
+
+
+def test_decoded_rows_leave_memory_to_others(ctx):
+    """An index whose decoded rows would take more than a quarter of the free memory goes without
+    them: every code is scored, with the same answers."""
+    import torch
+    n, dim = 1200000, 128  # 312 MB of decoded rows
+    print(f"decoded rows n={n}", flush=True)
+    x = torch.randint(0, 200, (n, dim), generator=torch.Generator("cuda").manual_seed(3),
+                      device="cuda").float()
+    torch.cuda.synchronize()
+    ds = vdbg.Dataset.from_device(ctx, x.data_ptr(), n, dim, dim)
+    del x
+    torch.cuda.empty_cache()
+    q = np.random.default_rng(4).integers(0, 200, (40, dim)).astype(np.float32)
+    want = None
+    for left in (None, 1 << 30):
+        fill = []
+        while left is not None and torch.cuda.mem_get_info()[0] > left and len(fill) < 4:
+            over = torch.cuda.mem_get_info()[0] - left  # (large allocations are rounded)
+            fill.append(torch.empty(over, dtype=torch.uint8, device="cuda"))
+        ix = vdbg.PqFlatIndex.build(ds, 16, max_points=4, iters=1)
+        del fill
+        torch.cuda.empty_cache()
+        ids, d, dc = ix.search(q, 10)
+        assert ctx.last_gemm_bits() == (16 if left is None else 0)
+        ix.close()
+        if want is None:
+            want = ids, d, dc
+    assert np.array_equal(ids, want[0]) and np.array_equal(dc, want[2])
+    assert np.array_equal(d.view(np.uint32), want[1].view(np.uint32))
+    ds.close()
