@@ -22,13 +22,6 @@
 namespace vdbg {
 namespace {
 
-size_t CountRows(const uint64_t* w, size_t rows) {
-  size_t n = 0;
-  for (size_t i = 0; i < rows / 64; ++i) n += size_t(__builtin_popcountll(w[i]));
-  if (rows % 64) n += size_t(__builtin_popcountll(w[rows / 64] & ((uint64_t(1) << (rows % 64)) - 1)));
-  return n;
-}
-
 // A device buffer freed on the stream when the call ends.
 struct DevBuf {
   void* p = nullptr;
@@ -552,8 +545,11 @@ int CollectionSearch(vdbg_ctx* ctx, const vdbg_segment* segs, size_t nseg, size_
     const vdbg_segment& g = segs[p];
     const size_t rows = g.rows->d.n;
     if (g.pqflat != nullptr) {  // PqFlatIndex::search (ivf_pq.cc:59-79)
-      VDBG_RETURN_IF_ERROR(vdbg_pqflat_search_device(g.pqflat, q, nq, kk, P.rerank, allow, ids, dd,
-                                                     static_cast<uint64_t*>(dcb.p), s));
+      const bool own = !plan[p].allow.empty() &&  // (a post-filter searches under other words)
+                       allow == static_cast<const uint64_t*>(allow_dev.p) + allow_at[p];
+      VDBG_RETURN_IF_ERROR(PqFlatSearchDevice(g.pqflat, q, nq, kk, P.rerank, allow,
+                                              own ? plan[p].allowed : -1, ids, dd,
+                                              static_cast<uint64_t*>(dcb.p), s));
       VDBG_HIP(hipMemcpyAsync(dch.data(), dcb.p, nq * 8, hipMemcpyDeviceToHost, s));
       VDBG_HIP(hipStreamSynchronize(s));
       if (dist_comps != nullptr)

@@ -13,8 +13,10 @@
 // GEMM over the rows the codes decode to (fp16 halves, gemm16.hip SPLIT 3: the ADC is the
 // distance to the decoded row up to its rounding, which the query's bound takes in); every
 // candidate it admits is then scored by ADC from the query's table, certified against the
-// admission threshold, and re-scanned code by code when that fails.  Otherwise every code is
-// scored (row splits with a wave top-k each, then a merge; a sort beyond 240 results).
+// admission threshold, and re-scanned code by code when that fails.  Small batches over few
+// rows or under a selective filter (PqScoreFew, PqScoreFiltered), and widths without a kernel,
+// score every allowed code instead (row splits with a wave top-k each, then a merge; a sort
+// beyond 240 results).
 //
 // Bound: MFMA (2 n pd flop per query; 890 TFLOP/s at 1M x 128, 2,000 queries).  Scoring every
 // code is bound by its m table reads a row instead: the batch of 2,000 queries over 1M codes
@@ -108,9 +110,44 @@ struct Tmp {
   }
 };
 
+// Whether scoring every allowed code takes less than the ranking GEMM over every row.  Each side
+// of the lines was timed with host calls, in us.
+//
+// Few rows: below 25 rows for each of the depth the ranking's threshold admits most of them
+// (ranked / scored at depth 100, m 16 x 8 dims: 2,000 rows 118 / 81 for 1 query and 317 / 237 for
+// 2,000; 3,000 rows 96 / 82 and 209 / 272; at depth 240: 4,000 rows 440 / 423 for 2,000 queries,
+// 6,000 rows 294 / 503).  Above that small batches score while the table reads cost less than the
+// ranking's launches do beyond the scoring's (depth 10: 4,000 rows 88 / 69 for 1 query, 98 / 112
+// for 500; 12,000 rows 86 / 83 for 16, 90 / 94 for 64; depth 100: 4,000 rows 121 / 103 for 64,
+// 142 / 154 for 500, 20,000 rows 125 / 126 for 64; depth 240: 6,000 rows 135 / 146 for 1).  From 8
+// queries on the ranking takes about 12 us more at depths up to 100, none at 240.
+bool PqScoreFew(size_t rows, int m, size_t nq, size_t kk) {
+  const double n = double(rows), q = double(nq), k = double(kk);
+  if (n < 25.0 * k) return true;
+  const double reads = n * (6e-4 + q * 1e-6 * std::max(13, m));
+  return reads < 20.0 - 0.16 * k + (nq >= 8 && kk <= 100 ? 12.0 : 0.0) + (rows < 3000 ? 25.0 : 0.0);
+}
+// A selective filter (at most a sixteenth of the rows, past which the fits below fail): the scan
+// of the codes skips what it leaves out.  Both sides as fitted, within 15%.  Ranked / scored at
+// depth 100, 1M x 128, m 16: 0.2% allowed 188 / 119 for 1 query, 195 / 173 for 16, 200 / 220
+// for 32, and 2% 194 / 209 for 1; 100,000 rows: 2% 131 / 114 for 1, 144 / 133 for 16, 148 / 156
+// for 32; 200,000 x 384, m 48: 2% 190 / 169 for 8, 193 / 202 for 16.  `spent`: what the choice
+// itself costs (counting the filter's rows on the device).
+bool PqScoreFiltered(size_t rows, size_t pd, int m, size_t nq, size_t allowed, double spent) {
+  const double n = double(rows), q = double(nq), a = double(allowed);
+  if (16 * a > n) return false;
+  const double score = 85.0 + 3e-5 * n + 4.5e-3 * a +
+                       q * (0.06 + 2e-6 * n + 4e-4 * a * (16.0 + m) / 32.0);
+  const double rank = 110.0 + 6.2e-7 * n * double(pd) + 0.25 * std::min(q, 64.0) +
+                      q * (0.05 + 2e-7 * n);
+  return score + spent + 8.0 < rank;
+}
+constexpr double kCountUs = 10.0;  // CountAllowed
+
+// allowed: the rows a filter allows, where the caller knows (-1: not).
 int PqFlatSearch(PqFlatIndex* x, const float* Q, size_t nq, size_t k, int rerank,
-                 const uint64_t* allow, uint32_t* out_ids, float* out_d, uint64_t* dc,
-                 hipStream_t s) {
+                 const uint64_t* allow, int64_t allowed, uint32_t* out_ids, float* out_d,
+                 uint64_t* dc, hipStream_t s) {
   Dataset* ds = x->ds;
   Ctx* c = ds->ctx;
   const size_t n = ds->n;
@@ -126,9 +163,29 @@ int PqFlatSearch(PqFlatIndex* x, const float* Q, size_t nq, size_t k, int rerank
   const size_t depth = rerank < 0 ? std::max<size_t>(10 * k, 100) : size_t(rerank);
   const size_t kk = std::max(depth, k);
   const size_t ts = size_t(x->m) * kKsub;
-  Tmp tables;
+  // the scan keeps at most n candidates, as a TopK of any capacity over n rows does (depth
+  // may exceed vdb's largest k: max(10 k, 100) at k = 10,000)
+  const size_t keep = std::min(kk, std::max<size_t>(n, k));
+  const bool can_rank = x->src.X16 != nullptr && x->src.N == n && c->fp16_gemm && kk <= 10000;
+  bool ranked = can_rank && (kk > 240 || !PqScoreFew(n, x->m, nq, kk));
+  if (ranked && allow != nullptr && kk <= 240) {
+    if (allowed < 0 && PqScoreFiltered(n, ds->pd, x->m, nq, 0, kCountUs)) {
+      // (a captured stream cannot be read from: it ranks)
+      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+      if (cap == hipStreamCaptureStatusNone) {
+        uint32_t count = 0;
+        VDBG_RETURN_IF_ERROR(CountAllowed(c, allow, uint32_t(n), &count, s, nullptr));
+        allowed = count;
+      }
+    }
+    if (allowed >= 0) ranked = !PqScoreFiltered(n, ds->pd, x->m, nq, size_t(allowed), 0.0);
+  }
+  Tmp tables;  // the tables, and the candidates handed to the rerank
   tables.s = s;
-  VDBG_HIP(hipMallocAsync(&tables.p, nq * ts * sizeof(float), s));
+  const size_t tb = (nq * ts * sizeof(float) + 255) / 256 * 256;
+  const size_t cb = depth == 0 ? 0 : (nq * keep * 4 + 255) / 256 * 256;
+  VDBG_HIP(ScratchAlloc(c, &tables.p, tb + 2 * cb, s));
   {
     ProfScope ps(c, "pq_tables", s);
     const size_t total = nq * ts;
@@ -146,19 +203,16 @@ int PqFlatSearch(PqFlatIndex* x, const float* Q, size_t nq, size_t k, int rerank
   src.pd = int(ds->pd);
   src.metric = ds->metric;
   // the kk best by (ADC, id): the ranking GEMM over the decoded rows and the ADC of the few
-  // codes it admits, or the ADC of every code
+  // codes it admits, or the ADC of every allowed code
   auto scan = [&](size_t kk, uint32_t* ids, float* d) {
-    if (x->src.X16 != nullptr && x->src.N == n && c->fp16_gemm && kk <= 10000) {
+    if (ranked) {
       VDBG_RETURN_IF_ERROR(BuildSample(c, &x->src, s));
-      ScanSource ranked = x->src;
-      ranked.pq_tables = T;
-      return RunScan(c, &ranked, Q, nq, kk, allow, ids, d, s);
+      ScanSource rs = x->src;
+      rs.pq_tables = T;
+      return RunScan(c, &rs, Q, nq, kk, allow, ids, d, s);
     }
     return ScoreScan(c, src, T, nq, kk, allow, ids, d, s);
   };
-  // the scan keeps at most n candidates, as a TopK of any capacity over n rows does (depth
-  // may exceed vdb's largest k: max(10 k, 100) at k = 10,000)
-  const size_t keep = std::min(kk, std::max<size_t>(n, k));
   if (depth == 0) {
     VDBG_RETURN_IF_ERROR(scan(k, out_ids, out_d));
     if (dc != nullptr)
@@ -167,12 +221,9 @@ int PqFlatSearch(PqFlatIndex* x, const float* Q, size_t nq, size_t k, int rerank
     VDBG_HIP(hipGetLastError());
     return kOk;
   }
-  Tmp ci, cd;
-  ci.s = cd.s = s;
-  VDBG_HIP(hipMallocAsync(&ci.p, nq * keep * 4, s));
-  VDBG_HIP(hipMallocAsync(&cd.p, nq * keep * 4, s));
-  uint32_t* cand = static_cast<uint32_t*>(ci.p);
-  VDBG_RETURN_IF_ERROR(scan(keep, cand, static_cast<float*>(cd.p)));
+  uint32_t* cand = reinterpret_cast<uint32_t*>(static_cast<char*>(tables.p) + tb);
+  float* cand_d = reinterpret_cast<float*>(static_cast<char*>(tables.p) + tb + cb);
+  VDBG_RETURN_IF_ERROR(scan(keep, cand, cand_d));
   VDBG_RETURN_IF_ERROR(Rerank(c, ds->rows, int(ds->pd), ds->metric, Q, nq, cand, keep, k, out_ids,
                               out_d, s, &ds->src));
   if (dc != nullptr)
@@ -289,6 +340,22 @@ int InstallPqFlat(Ctx* c, PqFlatIndex* x, const uint8_t* codes_h, hipStream_t s)
 }
 
 }  // namespace
+
+int PqFlatSearchDevice(vdbg_pqflat* ix, const float* queries, size_t nq, size_t k, int rerank,
+                       const uint64_t* allow_words, int64_t allowed, uint32_t* out_ids,
+                       float* out_dists, uint64_t* dist_comps, void* stream) {
+  if (ix == nullptr) return SetError(kInvalidArgument, "null index");
+  if (nq > 0 && k > 0 && (queries == nullptr || out_ids == nullptr || out_dists == nullptr))
+    return SetError(kInvalidArgument, "null pointer");
+  if (k > 10000) return SetError(kInvalidArgument, "k must be in 1..10000");
+  Ctx* c = ix->p.ds->ctx;
+  std::lock_guard<std::recursive_mutex> g(c->mu);
+  VDBG_HIP(hipSetDevice(c->device));
+  hipStream_t s = stream ? static_cast<hipStream_t>(stream) : c->stream;
+  return PqFlatSearch(&ix->p, queries, nq, k, rerank, allow_words, allowed, out_ids, out_dists,
+                      dist_comps, s);
+}
+
 }  // namespace vdbg
 
 using namespace vdbg;
@@ -465,16 +532,8 @@ int vdbg_pqflat_codes(vdbg_pqflat* ix, uint8_t* codes_out) {
 int vdbg_pqflat_search_device(vdbg_pqflat* ix, const float* queries, size_t nq, size_t k,
                               int rerank, const uint64_t* allow_words, uint32_t* out_ids,
                               float* out_dists, uint64_t* dist_comps, void* stream) {
-  if (ix == nullptr) return SetError(kInvalidArgument, "null index");
-  if (nq > 0 && k > 0 && (queries == nullptr || out_ids == nullptr || out_dists == nullptr))
-    return SetError(kInvalidArgument, "null pointer");
-  if (k > 10000) return SetError(kInvalidArgument, "k must be in 1..10000");
-  Ctx* c = ix->p.ds->ctx;
-  std::lock_guard<std::recursive_mutex> g(c->mu);
-  VDBG_HIP(hipSetDevice(c->device));
-  hipStream_t s = stream ? static_cast<hipStream_t>(stream) : c->stream;
-  return PqFlatSearch(&ix->p, queries, nq, k, rerank, allow_words, out_ids, out_dists,
-                      dist_comps, s);
+  return PqFlatSearchDevice(ix, queries, nq, k, rerank, allow_words, -1, out_ids, out_dists,
+                            dist_comps, stream);
 }
 
 int vdbg_pqflat_search_host(vdbg_pqflat* ix, const float* queries, size_t nq, size_t k,
@@ -492,10 +551,11 @@ int vdbg_pqflat_search_host(vdbg_pqflat* ix, const float* queries, size_t nq, si
   Ctx* c = d.ctx;
   std::lock_guard<std::recursive_mutex> g(c->mu);
   VDBG_HIP(hipSetDevice(c->device));
+  const int64_t allowed = allow_words != nullptr ? int64_t(CountRows(allow_words, d.n)) : -1;
   return StageHost(c, d.n, d.pd, queries, nq, k, allow_words, out_ids, out_dists, dist_comps,
                    [&](const float* dq, const uint64_t* dm, uint32_t* di, float* dd,
                        uint64_t* ddc, hipStream_t st) {
-                     return PqFlatSearch(&ix->p, dq, nq, k, rerank, dm, di, dd, ddc, st);
+                     return PqFlatSearch(&ix->p, dq, nq, k, rerank, dm, allowed, di, dd, ddc, st);
                    });
 }
 

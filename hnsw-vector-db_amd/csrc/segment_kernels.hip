@@ -153,6 +153,35 @@ __global__ void k_map_ids(uint32_t* __restrict__ out, size_t n, const uint32_t* 
   if (t < n && out[t] != kNoId) out[t] = ids[out[t]];
 }
 
+// One block: the set bits of w among N rows, to *out and, behind `flag`'s sequence number, to the
+// host (as ReadWords publishes).
+__global__ __launch_bounds__(1024) void k_count_allowed(const uint64_t* __restrict__ w,
+                                                        uint32_t nwords, uint32_t N, uint32_t* out,
+                                                        uint32_t* flag, uint32_t seq) {
+  __shared__ uint32_t part[16];
+  uint32_t n = 0;
+#pragma unroll 4
+  for (uint32_t i = threadIdx.x; i < nwords; i += 1024) {
+    uint64_t v = w[i];
+    const uint32_t left = N - i * 64;  // (at least one row)
+    if (left < 64) v &= (1ull << left) - 1ull;
+    n += uint32_t(__popcll(v));
+  }
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) n += __shfl_xor(n, o);
+  if (lane_id() == 0) part[threadIdx.x >> 6] = n;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  n = 0;
+  for (int i = 0; i < 16; ++i) n += part[i];
+  *out = n;
+  flag[1] = n;
+  __threadfence_system();
+  __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// (2M rows: 256 KB of words)
+constexpr size_t kCountOneBlock = 32768;
+
 int CountAllowed(Ctx* c, const uint64_t* allow, uint32_t N, uint32_t* count, hipStream_t s,
                  ScanScratch* lane) {
   const size_t nwords = (size_t(N) + 63) / 64;
@@ -168,6 +197,15 @@ int CountAllowed(Ctx* c, const uint64_t* allow, uint32_t N, uint32_t* count, hip
   if (done != nullptr) VDBG_HIP(hipStreamWaitEvent(s, done, 0));
   VDBG_RETURN_IF_ERROR(w.reserve((nwords + 1) * 4 + tmp_bytes + 1024));
   uint32_t* cnt = w.take<uint32_t>(nwords + 1);
+  if (nwords <= kCountOneBlock) {  // one launch
+    std::lock_guard<std::mutex> g(c->flag_mu);
+    const uint32_t seq = NextFlagSeq(c);
+    k_count_allowed<<<1, 1024, 0, s>>>(allow, uint32_t(nwords), N, cnt, c->host_flag_dev, seq);
+    VDBG_HIP(hipGetLastError());
+    VDBG_RETURN_IF_ERROR(WaitWords(c, seq, cnt, 1, s));
+    *count = c->host_pinned[0];
+    return kOk;
+  }
   void* tmp = w.take<char>(tmp_bytes + 16);
   k_word_counts<<<dim3(unsigned((nwords + 255) / 256)), 256, 0, s>>>(allow, nwords, N, cnt);
   VDBG_HIP(hipGetLastError());

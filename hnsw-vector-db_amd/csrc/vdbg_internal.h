@@ -27,6 +27,7 @@ enum Code : int {
 
 int SetError(int code, const std::string& msg);  // records the thread's message, returns code
 int BestHostKernelSet();  // the host CPU's best distance kernel set (host_cpu.cc)
+size_t CountRows(const uint64_t* w, size_t rows);  // set bits among the first rows (host_cpu.cc)
 
 // File formats (files.cc): CRC32C of every vdb file, and Segment::Open's vectors.f32 checks
 // (src/storage/segment_reader.cc:37-55); *data is the first row, *rows the header's count.
@@ -517,6 +518,13 @@ int SortKeysTopK(Ctx* c, const SortKeysArgs& a, int nq, hipStream_t s);
 // the first K of each as (id, dist), padded with (UINT32_MAX, +inf).
 int SortSegmentsTopK(Ctx* c, uint64_t* keys, uint64_t* keys_alt, const int* off_dev, int nseg,
                      int total, int K, uint32_t* out_ids, float* out_d, hipStream_t s);
+// The rows a device filter allows, read back (lane: nullable, a collection lane's scratch).
+int CountAllowed(Ctx* c, const uint64_t* allow, uint32_t N, uint32_t* count, hipStream_t s,
+                 ScanScratch* lane);
+// vdbg_pqflat_search_device for a caller that knows the rows its filter allows (-1: not).
+int PqFlatSearchDevice(vdbg_pqflat* ix, const float* queries, size_t nq, size_t k, int rerank,
+                       const uint64_t* allow_words, int64_t allowed, uint32_t* out_ids,
+                       float* out_dists, uint64_t* dist_comps, void* stream);
 // RunScan under an optional filter; compacts the allowed rows when they are few.
 // CollectionImpl::Search's merge (segment_kernels.hip): hits of every part ordered by
 // (dist, part, row), first hit of each external id kept.

@@ -18,6 +18,7 @@ def words(bits):
     return w.view(np.uint64)
 
 
+# (batches of few rows score every code: test_ranked_few_rows has the batches that rank)
 # rows at the path's limit of 1,024 and at remainders of the 64-row tiles; padded dims of one
 # and several K chunks, with padding (100 -> 112, 20 -> 32) and without a kernel (400)
 @pytest.mark.parametrize("n,dim,m,metric", [
@@ -44,6 +45,30 @@ def test_ranked_search_matches_oracle(ctx, oracle, n, dim, m, metric):
         assert np.array_equal(ids, oi)
         assert np.array_equal(d.view(np.uint32), od.view(np.uint32))
         assert np.array_equal(dc, odc)
+    ix.close()
+    ds.close()
+
+
+# few rows rank only in batches large enough to repay it
+@pytest.mark.parametrize("n,dim,m,metric", [(1024, 64, 8, "l2"), (1025, 100, 20, "cosine"),
+                                            (4097, 20, 5, "l2")])
+def test_ranked_few_rows(ctx, oracle, n, dim, m, metric):
+    nq, k = 4500, 10
+    print(f"ranked few rows n={n} dim={dim} m={m} {metric}", flush=True)
+    pd = vdbg.padded_dim(dim)
+    rows = datagen.pad(datagen.clustered_unit(n, dim, 31, 32, 60, 0.6) * np.float32(3.0), pd)
+    q = datagen.pad(datagen.clustered_unit(nq, dim, 33, 32, 60, 0.6) * np.float32(3.0), pd)
+    ds = vdbg.Dataset(ctx, rows, dim, metric)
+    ix = vdbg.PqFlatIndex.build(ds, m, max_points=16, iters=2)
+    at = np.r_[0:20, nq - 20:nq]
+    for frac in (None, 0.4):
+        allow = None if frac is None else words(np.random.default_rng(7).random(n) < frac)
+        ids, d, dc = ix.search(q, k, 0, allow)
+        assert ctx.last_gemm_bits() == 16
+        od, oi, odc = oracle.pqflat_search(parse_pqflat(ix.save()), rows, q[at], k, 0, metric, allow,
+                                           kset=ctx.kernels)
+        assert np.array_equal(ids[at], oi) and np.array_equal(dc[at], odc)
+        assert np.array_equal(d[at].view(np.uint32), od.view(np.uint32))
     ix.close()
     ds.close()
 
@@ -106,4 +131,43 @@ def test_decoded_rows_leave_memory_to_others(ctx):
             want = ids, d, dc
     assert np.array_equal(ids, want[0]) and np.array_equal(dc, want[2])
     assert np.array_equal(d.view(np.uint32), want[1].view(np.uint32))
+    ds.close()
+
+
+@pytest.mark.parametrize("n", [20000, 70001])
+def test_routes_agree(ctx, oracle, n):
+    """Calls on both sides of the choice between ranking and scoring every allowed code: few
+    queries under a selective filter score (the filter's rows counted on the host, or on the
+    device for a device call), the rest rank; the oracle's answers either way."""
+    import torch
+    rows, q = datagen.sift_like(n, 128, 51), datagen.sift_like(200, 128, 52)
+    ds = vdbg.Dataset(ctx, rows, 128)
+    ix = vdbg.PqFlatIndex.build(ds, 16, max_points=16, iters=2)
+    pix = parse_pqflat(ix.save())
+    rng = np.random.default_rng(8)
+    seen = set()
+    for nq, frac in ((1, 0.0), (1, 0.002), (7, 0.02), (33, 0.02), (200, 0.02), (200, 0.0625),
+                     (1, 0.5), (33, None), (200, None)):
+        print(f"routes n={n} nq={nq} filter={frac}", flush=True)
+        allow = None if frac is None else words(rng.random(n) < frac)
+        od, oi, odc = oracle.pqflat_search(pix, rows, q[:nq], 10, 100, "l2", allow,
+                                           kset=ctx.kernels)
+        ids, d, dc = ix.search(q[:nq], 10, 100, allow)
+        bits = ctx.last_gemm_bits()
+        seen.add(bits)
+        assert np.array_equal(ids, oi) and np.array_equal(dc, odc)
+        assert np.array_equal(d.view(np.uint32), od.view(np.uint32))
+        dq = torch.from_numpy(q[:nq]).cuda()
+        da = None if allow is None else torch.from_numpy(allow.view(np.int64)).cuda()
+        di = torch.empty((nq, 10), dtype=torch.int32, device="cuda")
+        dd = torch.empty((nq, 10), dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        ix.search_device(dq.data_ptr(), nq, 10, 100, di.data_ptr(), dd.data_ptr(),
+                         None if da is None else da.data_ptr())
+        ctx.synchronize()
+        assert ctx.last_gemm_bits() in (bits, 16)
+        assert np.array_equal(di.cpu().numpy().view(np.uint32), oi)
+        assert np.array_equal(dd.cpu().numpy().view(np.uint32), od.view(np.uint32))
+    assert seen == {0, 16}
+    ix.close()
     ds.close()
