@@ -461,8 +461,8 @@ int CollectionSearch(vdbg_ctx* ctx, const vdbg_segment* segs, size_t nseg, size_
   }
 
   // flat scans (in-memory parts, flat segments under their index plan, the exact scan of a
-  // prefilter plan): one launch for a small batch, else the lanes; every other plan runs on s
-  // in turn
+  // prefilter plan): one launch for a small batch (of not too many rows), else the lanes; every
+  // other plan runs on s in turn
   auto on_lane = [&](size_t p) {
     const int pl = plan[p].plan;
     const vdbg_segment& g = segs[p];
@@ -482,6 +482,7 @@ int CollectionSearch(vdbg_ctx* ctx, const vdbg_segment* segs, size_t nseg, size_
     std::vector<RowSet> sets;
     std::vector<const uint64_t*> allow_h, ext;
     bool ok = true;
+    double extra = 0.0;
     for (size_t p = 0; p < nseg && ok; ++p) {
       const vdbg_segment& g = segs[p];
       if (g.host_rows == nullptr && plan[p].plan == VDBG_PLAN_EMPTY) continue;
@@ -490,11 +491,14 @@ int CollectionSearch(vdbg_ctx* ctx, const vdbg_segment* segs, size_t nseg, size_
       const ScanSource& sp = g.rows->d.src;
       ok = RowScanEligible(c, sp, nq, k) && sets.size() < size_t(kRowSets) &&
            (sets.empty() || RowScanLike(c, *sets[0].src, sp));
+      const bool filtered = !plan[p].allow.empty();
+      extra += RowScanExtraUs(c, sp, nq, k, filtered && plan[p].allowed >= 0
+                                                ? size_t(plan[p].allowed) : g.rows->d.n, filtered);
       sets.push_back(RowSet{&sp, nullptr});
       allow_h.push_back(plan[p].allow.empty() ? nullptr : plan[p].allow.data());
       ext.push_back(g.rows->d.ext_ids);
     }
-    if (ok && !sets.empty()) {
+    if (ok && !sets.empty() && extra <= kRowScanSavesUs) {
       VDBG_RETURN_IF_ERROR(SmallCollection(c, sets, allow_h, ext, dim, pd, metric, queries, nq, k,
                                            out_ids, out_dists, device_io, s));
       count_scans();

@@ -3430,6 +3430,24 @@ bool RowScanEligible(const Ctx* c, const ScanSource& src, size_t nq, size_t kk) 
          (RowScanF16(c, src) || (src.Xmap == nullptr && src.X != nullptr));
 }
 
+// Per million allowed rows k_row_scan takes 2, 17 or 48 us for up to 2, 4 or 8 queries beside its
+// bytes, which the lanes' scans do not, and 0.16 us a million values more than the int8 scans
+// where the rows have those; testing a filter takes the lanes 5 us a million rows more than it
+// does here, 31 in the int8 scan of more than two queries, and one below half the rows is cheaper
+// here at any size.  Collections, this path / the lanes in us: integer rows, 128 dims, no filter:
+// 4M rows 480 / 507 for 8 queries, 8M rows 430 / 542 for 1, 557 / 517 for 3, 793 / 521 for 8, 16M
+// rows 775 / 732 for 1; 97% allowed: 8M rows 662 / 859 for 3, 16M rows 1,645 / 1,533 for 8; 70%:
+// 16M rows 1,338 / 1,559 for 8.  Float rows, 384 dims: 4M rows 874 / 883 for 8, 8M rows 1,210 /
+// 1,487 for 4, 1,562 / 1,491 for 8.
+double RowScanExtraUs(const Ctx* c, const ScanSource& src, size_t nq, size_t kk, size_t allowed,
+                      bool filtered) {
+  if (!GemmSupported(src.pd) || 2 * allowed <= src.N) return 0.0;
+  const bool int8 = TinyEligible(c, src, nq, kk, c->ws);
+  const double row = nq <= 2 ? 2.0 : nq <= 4 ? 17.0 : 48.0;
+  const double test = !filtered ? 0.0 : int8 && nq > size_t(kTinyQ) ? 31.0 : 5.0;
+  return 1e-6 * (double(allowed) * (row + (int8 ? 0.16 : 0.0) * src.pd) - double(src.N) * test);
+}
+
 bool RowScanLike(const Ctx* c, const ScanSource& a, const ScanSource& b) {
   return a.pd == b.pd && a.metric == b.metric && RowScanF16(c, a) == RowScanF16(c, b);
 }

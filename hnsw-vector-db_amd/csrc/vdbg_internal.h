@@ -442,6 +442,10 @@ struct RowSet {
   const uint64_t* allow;  // nullable, device words
 };
 bool RowScanEligible(const Ctx* c, const ScanSource& src, size_t nq, size_t kk);
+// What RowScan takes beyond the lanes' scan of a large, mostly allowed source, in us.
+double RowScanExtraUs(const Ctx* c, const ScanSource& src, size_t nq, size_t kk, size_t allowed,
+                      bool filtered);
+constexpr double kRowScanSavesUs = 280.0;  // of launches and waits, over the lanes
 // Whether two sources can be sets of one RowScan.
 bool RowScanLike(const Ctx* c, const ScanSource& a, const ScanSource& b);
 // Whether RunScan answers the batch from one pass over the rows (k_tiny_scan, k_small_scan,

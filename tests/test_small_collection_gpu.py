@@ -146,3 +146,25 @@ def test_small_collection_refused_query_writes_nothing(ctx, bad):
     assert bool((ids == 77).all()) and bool((d == 5.0).all())
     for ds in handles:
         ds.close()
+
+
+@pytest.mark.parametrize("filt", [None, 0.4, 0.9])
+def test_few_queries_over_many_rows(ctx, oracle, filt):
+    """Sizes on both sides of the line between one launch over every segment and the lanes (5 to
+    8 queries, 6M allowed rows): the same answers."""
+    rng = np.random.default_rng(31)
+    segs, handles, at = [], [], 0
+    for n in (3500000, 3000000):
+        base = rng.random((n, 16), dtype=np.float32)
+        ds = vdbg.Dataset(ctx, base, 16, "l2")
+        ext = np.arange(at, at + n, dtype=np.uint64)
+        at += n
+        ds.set_external_ids(ext)
+        segs.append({"base": base, "ext": ext, "kind": "flat", "deleted": None,
+                     "filter": None if filt is None else mask(n, filt, at)})
+        handles.append(ds)
+    for nq in (4, 8):
+        print(f"few queries over many rows nq={nq} filter={filt}", flush=True)
+        run(ctx, oracle, segs, handles, 16, "l2", rng.random((nq, 16), dtype=np.float32), 10)
+    for ds in handles:
+        ds.close()
