@@ -652,25 +652,39 @@ struct PickArgs {
   uint32_t* fb_count;
 };
 
-// sum_j fl(term2 + qtab), the reference's four accumulators over j mod 4.  The common shape (m 16
-// of 8 dims) loads eight subspaces' entries at once.
+// sum_j fl(term2 + qtab), the reference's four accumulators over j mod 4.  M subspaces of D dims
+// compiled in (M 0: both at run time), one or two code words a turn, at most 128 floats of centroids
+// in flight (unrolled whole it spills at six waves a SIMD).  4,000 queries, 32 of 512 lists of
+// 200,000 rows, scores returned, against the run-time loop: m 16 x 4 dims 181 -> 151 us, 8 x 16
+// 166 -> 121, 8 x 8 123 -> 105, 4 x 32 141 -> 117, 4 x 8 79 -> 73.
+template <int M, int D>
 __device__ __forceinline__ float pick_score(const PickArgs& a, const float* qv,
                                             const float* __restrict__ t2,
                                             const uint8_t* __restrict__ cd) {
   float s[4] = {0.f, 0.f, 0.f, 0.f};
-  if (a.m == 16 && a.dsub == 8) {
-    const u32x4 w = *reinterpret_cast<const u32x4*>(cd);
+  if constexpr (M != 0) {
+    constexpr int W = D <= 8 && M >= 8 ? 2 : 1;  // words of four codes a turn
+    uint32_t codes[M / 4];  // (a row's codes start on a multiple of M bytes: one load)
+    __builtin_memcpy(codes, __builtin_assume_aligned(cd, M), M);
+#pragma unroll 1
+    for (int j0 = 0; j0 < M / 4; j0 += W) {
+      uint32_t w[W];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      if (j % 8 == 0) __builtin_amdgcn_sched_barrier(0);
-      const int c = int((w[j >> 2] >> (8 * (j & 3))) & 0xffu);
-      const v4f* q = reinterpret_cast<const v4f*>(qv + j * 8);
-      const float4* y = reinterpret_cast<const float4*>(a.cen + (j * kKsub + c) * 8);
-      const float4 u = y[0], v = y[1];
-      const v4f g0 = q[0], g1 = q[1];
-      const float s0 = g0[0] * u.x + g1[0] * v.x, s1 = g0[1] * u.y + g1[1] * v.y;
-      const float s2 = g0[2] * u.z + g1[2] * v.z, s3 = g0[3] * u.w + g1[3] * v.w;
-      s[j & 3] += t2[j * kKsub + c] + (-((s0 + s1) + (s2 + s3))) * 2.f;
+      for (int i = 0; i < W; ++i) {
+        w[i] = codes[i];
+#pragma unroll
+        for (int t = i; t + W < M / 4; t += W) codes[t] = codes[t + W];  // (the next turn's)
+      }
+#pragma unroll
+      for (int i = 0; i < 4 * W; ++i) {
+        const int j = 4 * j0 + i, c = int((w[i >> 2] >> (8 * (i & 3))) & 0xffu);
+        const v4f* q = reinterpret_cast<const v4f*>(qv + j * D);
+        const v4f* y = reinterpret_cast<const v4f*>(a.cen + (j * kKsub + c) * D);
+        v4f d = q[0] * y[0];  // dot_any's four accumulators
+#pragma unroll
+        for (int e = 1; e < D / 4; ++e) d += q[e] * y[e];
+        s[i & 3] += t2[j * kKsub + c] + (-((d[0] + d[1]) + (d[2] + d[3]))) * 2.f;
+      }
     }
   } else {
 #pragma unroll 1
@@ -689,7 +703,7 @@ __device__ __forceinline__ float pick_score(const PickArgs& a, const float* qv,
 }
 
 // The top R of a query's total <= 64 V candidates.
-template <int E, int V>
+template <int E, int V, int M, int D>
 __device__ __forceinline__ void pick_query(const PickArgs& a, int q, uint32_t total,
                                            uint32_t* st_row, uint8_t* st_p, float* qv) {
   const int lane = lane_id();
@@ -757,7 +771,7 @@ __device__ __forceinline__ void pick_query(const PickArgs& a, int q, uint32_t to
       const float* t2 = a.term2 + size_t(a.probe[pq]) * a.m * kKsub;
       const uint8_t* cd = a.codes + size_t(r) * a.m;
       id = a.ids[r];
-      const float sum = pick_score(a, qv + z, t2, cd);
+      const float sum = pick_score<M, D>(a, qv + z, t2, cd);
       d = a.probe_d[pq] + sum;
     }
     top.insert(d, id);
@@ -787,7 +801,7 @@ __device__ __forceinline__ void pick_query(const PickArgs& a, int q, uint32_t to
 // One wave per query.  Bound: a chain of gathers (candidates, codes, centroids and term-2
 // entries of the band's rows), hidden by waves, so the registers are held to six a SIMD: 84 us per
 // 10,000 queries of 182 candidates (94 at four).
-template <int E>
+template <int E, int M, int D>
 __global__ __launch_bounds__(256, 6) void k_ivf_pick(PickArgs a) {
   __shared__ uint32_t st_row[4][kCap];
   __shared__ uint8_t st_p[4][kCap];
@@ -800,8 +814,8 @@ __global__ __launch_bounds__(256, 6) void k_ivf_pick(PickArgs a) {
     if (lane_id() == 0) a.fb_list[atomicAdd(a.fb_count, 1u)] = uint32_t(q);
     return;
   }
-  if (total <= 4 * kWave) pick_query<E, 4>(a, q, total, st_row[wave], st_p[wave], qv[wave]);
-  else pick_query<E, kCap / kWave>(a, q, total, st_row[wave], st_p[wave], qv[wave]);
+  if (total <= 4 * kWave) pick_query<E, 4, M, D>(a, q, total, st_row[wave], st_p[wave], qv[wave]);
+  else pick_query<E, kCap / kWave, M, D>(a, q, total, st_row[wave], st_p[wave], qv[wave]);
 }
 
 // ---------------------------------------------------------------- host
@@ -844,6 +858,25 @@ static int launch_lists(int pd, hipStream_t s, const ListArgs& a) {
   }
   VDBG_HIP(hipGetLastError());
   return kOk;
+}
+
+template <int E>
+static void launch_pick(unsigned grid, hipStream_t s, const PickArgs& a) {
+#define VDBG_P(MM, DD) \
+  if (a.m == MM && a.dsub == DD) return k_ivf_pick<E, MM, DD><<<dim3(grid), 256, 0, s>>>(a)
+  VDBG_P(16, 8);
+  VDBG_P(16, 4);
+  VDBG_P(8, 16);
+  VDBG_P(8, 12);
+  VDBG_P(8, 8);
+  VDBG_P(8, 4);
+  VDBG_P(4, 32);
+  VDBG_P(4, 24);
+  VDBG_P(4, 16);
+  VDBG_P(4, 8);
+  VDBG_P(4, 4);
+#undef VDBG_P
+  k_ivf_pick<E, 0, 0><<<dim3(grid), 256, 0, s>>>(a);
 }
 
 static int GroupPairs(hipStream_t s, const GroupArgs& g) {
@@ -927,9 +960,9 @@ static int ListsOnePass(Ctx* c, const IvfIndex& x, const IvfScanArgs& a, hipStre
                 x.codes, x.off, x.ids, a.probe, a.probe_d, cand, cand_p, cnt, uint32_t(cap), ovf,
                 eb, a.count_top ? 0 : 1, a.out_ids, a.out_d, a.dc, a.dc_base, a.count_top,
                 fb_list, fb_count};
-    if (a.R <= 64) k_ivf_pick<1><<<dim3(g4), 256, 0, s>>>(pk);
-    else if (a.R <= 128) k_ivf_pick<2><<<dim3(g4), 256, 0, s>>>(pk);
-    else k_ivf_pick<4><<<dim3(g4), 256, 0, s>>>(pk);
+    if (a.R <= 64) launch_pick<1>(g4, s, pk);
+    else if (a.R <= 128) launch_pick<2>(g4, s, pk);
+    else launch_pick<4>(g4, s, pk);
     VDBG_HIP(hipGetLastError());
   }
   return IvfScanListed(c, a, fb_list, fb_count, s);

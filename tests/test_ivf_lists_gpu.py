@@ -63,6 +63,19 @@ def test_list_scan_is_the_scan_by_query(ctx, n, dim, nlist, m, nprobe, rerank, k
     _same(ctx, ix, qs, k, nprobe, rerank)
 
 
+# the compiled code widths that the sizes above leave out, scores returned and re-ranked
+@pytest.mark.parametrize("dim,m", [(64, 16), (128, 8), (96, 8), (64, 8), (128, 4), (96, 4), (32, 4)])
+def test_list_scan_code_widths(ctx, dim, m):
+    n, nlist, nprobe = 20000, 64, 8
+    nq = _fewest(n, nlist, nprobe)
+    print(f"ivf lists widths {dim} m={m} nq={nq}", flush=True)
+    base = _rows(n, dim, 4101)
+    qs = _rows(nq, dim, 4102)
+    ix = vdbg.IvfPqIndex.load(vdbg.Dataset(ctx, base, dim), synth_ivfpq(base, dim, nlist, m, seed=7))
+    _same(ctx, ix, qs, 10, nprobe, 100)
+    _same(ctx, ix, qs, 150, nprobe, 0)
+
+
 def test_list_scan_duplicates_and_unbounded_queries(ctx):
     print("ivf lists duplicated rows, huge and NaN queries", flush=True)
     uniq = (datagen.sift_like(1500, 64, 4111) - 60.0).astype(np.float32) * np.float32(0.013)
