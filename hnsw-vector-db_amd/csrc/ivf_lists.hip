@@ -42,7 +42,8 @@ constexpr int kSeeds = 256;     // seeds of a (query, list): the minima of 1 or 
 constexpr int kSeedLists = 4;   // nearest lists that give seeds
 constexpr int kCap = 1024;      // candidates of a query
 constexpr int kStage = 768;     // candidates a wave stages before they are stored
-constexpr size_t kListsQueries = 65536;  // queries of one pass (at most 0.9 GB of scratch)
+constexpr size_t kListsQueries = 65536;  // queries of one pass, at most,
+constexpr size_t kListsBytes = size_t(1) << 30;  // and its scratch per query times their number
 constexpr int kListBlocks = 768;  // persistent blocks (three a CU)
 constexpr int kHistBlocks = 256;
 constexpr int kMaxLists = 16384;  // LDS histogram words
@@ -837,11 +838,17 @@ bool IvfListsEligible(const IvfIndex& x, size_t nq, size_t nprobe, size_t R) {
 
 static size_t Al(size_t b) { return (b + 255) & ~size_t(255); }
 
-// Queries of one pass (the scratch of all stays bounded).
-static size_t ListsPass(size_t nq) { return std::min<size_t>(nq, kListsQueries); }
+// Scratch of one query, and the queries of one pass (the scratch of all stays bounded: at 128
+// padded dims 14.6 KB a query at nprobe 64, 17.7 KB at 256).
+static size_t QueryBytes(const IvfIndex& x, size_t nprobe) {
+  return size_t(x.pd) * 2 + 8 * 4 + nprobe * 16 + kCap * 9 + kSeedLists * kSeeds * 4;
+}
+static size_t ListsPass(const IvfIndex& x, size_t nq, size_t nprobe) {
+  return std::min({nq, kListsQueries, kListsBytes / QueryBytes(x, nprobe)});
+}
 
 size_t IvfListsScratch(const IvfIndex& x, size_t all, size_t nprobe) {
-  const size_t nl = size_t(x.nlist), nq = ListsPass(all), pairs = nq * nprobe;
+  const size_t nl = size_t(x.nlist), nq = ListsPass(x, all, nprobe), pairs = nq * nprobe;
   return Al(nq * size_t(x.pd) * 2) + 8 * Al(nq * 4) + Al(kHistBlocks * nl * 4) + Al(nl * 4) +
          Al((nl + 1) * 4) + Al(pairs * 16) + Al((pairs / kLq + nl + 1) * 16) + 2 * 256 +
          Al(nq * kCap * 8) + Al(nq * kCap) + Al(nq * kSeedLists * kSeeds * 4);
@@ -969,7 +976,7 @@ static int ListsOnePass(Ctx* c, const IvfIndex& x, const IvfScanArgs& a, hipStre
 }
 
 int IvfScanLists(Ctx* c, const IvfIndex& x, const IvfScanArgs& a, hipStream_t s, void* scratch) {
-  const size_t pass = ListsPass(size_t(a.nq));
+  const size_t pass = ListsPass(x, size_t(a.nq), size_t(a.nprobe));
   for (size_t q0 = 0; q0 < size_t(a.nq); q0 += pass) {
     IvfScanArgs b = a;
     b.nq = int(std::min(pass, size_t(a.nq) - q0));

@@ -3562,8 +3562,8 @@ int RowScan(Ctx* c, const RowSet* sets, int nsets, const float* Q, size_t nq, si
   out->count = fb_count;
   for (int i = 0; i < nsets; ++i)
     out->prune[i] = {ra.part + size_t(ma.set[i].chunk0) * kp, ra.bound + ma.set[i].chunk0,
-                     size_t(chunks), kp, ma.set[i].nchunks, ra.set[i].chunk_rows, shift + i * nq, eb + i * nq, nullptr,
-                     nullptr, out_d + i * nq * kk, int(kk)};
+                     size_t(chunks), kp, ma.set[i].nchunks, ra.set[i].chunk_rows, shift + i * nq,
+                     eb + i * nq, nullptr, nullptr, out_d + i * nq * kk, int(kk)};
   return kOk;
 }
 
@@ -3593,7 +3593,7 @@ struct DeepPlan {
   bool on;
   double expect;    // candidates per query
   uint32_t stride;  // keys kept per query
-  size_t max_nq;    // queries per pass (1 GiB of keys and candidates)
+  size_t max_nq;    // queries per pass (about 1 GiB of keys, candidates and group minima)
 };
 constexpr size_t kDeepAllBytes = size_t(256) << 20;  // a place for every row of the batch
 static DeepPlan PlanDeep(const Ctx* c, const ScanSource& src, size_t nq, size_t kk) {
@@ -3608,8 +3608,11 @@ static DeepPlan PlanDeep(const Ctx* c, const ScanSource& src, size_t nq, size_t 
   if (!(want <= double(kBlockSortKeys))) return p;
   p.stride = 1024;
   while (p.stride < want) p.stride <<= 1;
-  // (the candidate buffers hold about four times the expectation, in 8-byte entries)
-  p.max_nq = std::max<size_t>(64, (size_t(1) << 30) / (size_t(p.stride) * 8 * 4));
+  // In 8-byte entries a query keeps its keys and up to 12 times the expectation as candidates
+  // (segments of the next power of two above three times their share), besides 64 to 128 for each
+  // of its chunks (a pass fills the device at most once: 16.8M), and up to 4,096 group minima.
+  const double per = 8.0 * (12.0 * p.expect + p.stride) + 4.0 * 4096;
+  p.max_nq = std::max<size_t>(64, size_t(((size_t(1) << 30) - (size_t(1) << 27)) / per));
   p.on = true;
   return p;
 }

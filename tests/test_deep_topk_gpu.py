@@ -54,7 +54,7 @@ def test_deep_flat(ctx, oracle, n, dim, nq, k, metric, data, frac):
 
 
 def test_deep_batch_in_parts(ctx, oracle):
-    """More queries than one pass's scratch is planned for (2,048 at 16,384 keys a query)."""
+    """More queries than one pass's scratch is planned for (some 1,300 at 16,384 keys a query)."""
     n, dim, nq, k = 70000, 16, 2050, 5000
     base, qs = datagen.uniform_rows(n, dim, 71), datagen.uniform_rows(nq, dim, 72)
     ds = vdbg.Dataset(ctx, base, dim)

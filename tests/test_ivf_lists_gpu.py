@@ -76,6 +76,16 @@ def test_list_scan_code_widths(ctx, dim, m):
     _same(ctx, ix, qs, 150, nprobe, 0)
 
 
+@pytest.mark.parametrize("nq,nprobe", [(65600, 8), (62000, 256)])
+def test_list_scan_in_passes(ctx, nq, nprobe):
+    """More queries than a pass takes: 65,536, or fewer with many probes a query (its scratch)."""
+    n, dim, nlist = 20000, 16, 256
+    print(f"ivf lists passes nq={nq} nprobe={nprobe}", flush=True)
+    base, qs = _rows(n, dim, 4121), _rows(nq, dim, 4122)
+    ix = vdbg.IvfPqIndex.load(vdbg.Dataset(ctx, base, dim), synth_ivfpq(base, dim, nlist, 4, seed=9))
+    _same(ctx, ix, qs, 10, nprobe, 20)
+
+
 def test_list_scan_duplicates_and_unbounded_queries(ctx):
     print("ivf lists duplicated rows, huge and NaN queries", flush=True)
     uniq = (datagen.sift_like(1500, 64, 4111) - 60.0).astype(np.float32) * np.float32(0.013)
