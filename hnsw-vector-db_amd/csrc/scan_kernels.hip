@@ -3387,6 +3387,7 @@ static int TinyScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t k
   ma.out_d = out_d;
   ma.fb_list = fb_list;
   ma.fb_count = c->opt_count != nullptr ? c->opt_count : fb_count;
+  c->opt_used |= c->opt_count != nullptr;
   ma.force_fallback = c->test_fallbacks;
   {
     ProfScope ps(c, "select", s);
@@ -3552,6 +3553,7 @@ int RowScan(Ctx* c, const RowSet* sets, int nsets, const float* Q, size_t nq, si
   ma.out_d = out_d;
   ma.fb_list = fb_list;
   ma.fb_count = c->opt_count != nullptr ? c->opt_count : fb_count;
+  c->opt_used |= c->opt_count != nullptr;
   ma.force_fallback = c->test_fallbacks;
   {
     ProfScope ps(c, "select", s);

@@ -168,6 +168,7 @@ struct Ctx {
   // no re-scan is queued, and the host, which reads the words with the results, re-scans what
   // they name; opt_rescan is what a flat search's re-scan takes
   uint32_t* opt_count = nullptr;
+  bool opt_used = false;  // some scan of the call counts there
   OptRescan opt_rescan;
   std::mutex flag_mu;  // one readback through host_flag at a time (scan lanes may run on
                        // worker threads of one call)
@@ -649,6 +650,7 @@ struct OptCount {
   Ctx* c;
   explicit OptCount(Ctx* ctx) : c(ctx) {
     c->opt_rescan = OptRescan{};
+    c->opt_used = false;
     c->opt_count = reinterpret_cast<uint32_t*>(c->stage_d + kStageOptWord);
   }
   ~OptCount() { c->opt_count = nullptr; }
@@ -702,6 +704,7 @@ inline int StageRegions(Ctx* c, const float* queries, size_t qb, const void* ext
       OptCount armed(c);
       VDBG_RETURN_IF_ERROR(fn(dq, dx, di, dd, ddc, s));
     }
+    if (!c->opt_used) return StageOut(c, osrc, obytes, odst, nout, s);
     osrc[nout] = c->stage_d + kStageOptWord;
     obytes[nout] = sizeof(uncertified);
     odst[nout] = uncertified;
