@@ -94,6 +94,8 @@ def points(kind, n, d, seed):
     return few[rng.integers(0, 3, n)]
 
 
+# (below some 10,000 points of few dims one set is initialised on the host: the sub-quantizers below
+# have the device's sets of that size)
 # around the tile of 4,096 points; widths with a compiled kernel, without one, and padded ones
 # (the kernel sets' distance) up to 128
 @pytest.mark.parametrize("n,d,k,kind", [
@@ -111,7 +113,8 @@ def test_kmeanspp_picks(ctx, n, d, k, kind):
 
 @pytest.mark.parametrize("n,dim,m,kind", [
     (4096, 32, 8, "uniform"), (5003, 96, 8, "wide"), (6000, 40, 8, "int"), (20000, 128, 16, "int"),
-    (4500, 64, 4, "int"), (5000, 60, 3, "uniform"), (4100, 16, 4, "few"), (3000, 32, 8, "uniform")])
+    (4500, 64, 4, "int"), (5000, 60, 3, "uniform"), (4097, 64, 16, "wide"), (8191, 64, 8, "wide"),
+    (8193, 72, 6, "grid"), (4100, 64, 8, "grid"), (12289, 48, 16, "wide"), (4099, 96, 8, "few"), (4100, 16, 4, "few"), (3000, 32, 8, "uniform")])
 def test_sub_quantizers_and_codes(ctx, oracle, n, dim, m, kind):
     """The codebook of a build equals m separate k-means runs (iterations, splits of empty
     clusters and generators included), its codes the oracle's encoder's."""
