@@ -889,7 +889,7 @@ def main():
         r = {"qps": nq * args.steps / el, "ms_per_step": el * 1e3 / args.steps,
              "kernel": "k_ivf_lists<128> (with the grouping of the probes by list)",
              "kernel_ms": s_ms, "achieved": gbs, "unit": "GB/s",
-             "peak": HBM_PEAK_GBS, "bound": "hbm",
+             "peak": HBM_PEAK_GBS, "bound": "latency",  # (waves wait between work items)
              "algorithmic_bytes": "decoded residuals and term-2 sums of the lists, once",
              "algorithmic_bytes_per_launch": alg_bytes,
              "codes_scanned_per_query": scanned / nq,

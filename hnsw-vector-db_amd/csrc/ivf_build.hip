@@ -716,12 +716,13 @@ int KMeansPPGpu(Ctx* c, const float* x, size_t xset, size_t sets, size_t n, size
 // Where the device pass is the faster one.  It takes two launches a pick for all sets, 28 us and
 // 0.6 ns a point; the host's loop, a set at a time, 2.9 ns a point or 0.24 a dim where that is
 // more, 1.1 a dim in the kernel sets' order (a whole call of 64 picks, host / device in ms:
-// 4,096 x 8 1.2 / 2.4, 12,288 x 8 2.7 / 3.0, 16,384 x 8 3.4 / 3.2, 65,536 x 8 13.4 / 5.3, 4,096 x 24
-// 2.0 / 2.5, 8,192 x 24 3.7 / 2.9, 4,096 x 32 9.8 / 2.7).  One block's marks cover kPpMarks tiles
-// at most.
+// 4,096 x 8 1.2 / 2.4, 12,288 x 8 2.7 / 3.0, 16,384 x 8 3.4 / 3.2, 65,536 x 8 13.4 / 5.3, 4,096 x
+// 24 2.0 / 2.5, 8,192 x 24 3.7 / 2.9, 4,096 x 32 9.8 / 2.7).  One block's marks cover kPpMarks
+// tiles at most.
 bool KMeansPPOnGpu(size_t n, size_t d, size_t stride, size_t sets) {
   if (n < 4096 || n > size_t(kPpTile) * (kPpMarks / 2)) return false;
-  const double host = SimdL2(d, stride) ? 1.1e-3 * double(d) : std::max(2.9e-3, 0.24e-3 * double(d));
+  const double host =
+      SimdL2(d, stride) ? 1.1e-3 * double(d) : std::max(2.9e-3, 0.24e-3 * double(d));
   return host * double(n) * double(sets) > 28.0 + 0.6e-3 * double(n);
 }
 
@@ -1010,7 +1011,8 @@ int PqTrainGpu(Ctx* c, const float* data, size_t n, size_t stride, size_t dim, s
   // All m sub-quantizers at once: narrow sub-vectors of enough points to initialise on the
   // device, whose training sets fit 1 GiB and whose (set, row) pairs a 32-bit sort takes.
   const size_t np = rows.size();
-  if (opts.kmeanspp && KMeansPPOnGpu(np, dsub, dsub, m) && 256.0 * double(np) <= 2.0e7 && dsub <= 64 &&
+  if (opts.kmeanspp && KMeansPPOnGpu(np, dsub, dsub, m) && 256.0 * double(np) <= 2.0e7 &&
+      dsub <= 64 &&
       !SimdL2(dsub, dsub) && np * dim * 4 <= (size_t(1) << 30) && m * np < (size_t(1) << 31) &&
       m <= 65535) {
     VDBG_RETURN_IF_ERROR(Alloc(&sub, m * np * dsub * sizeof(float), s));

@@ -654,8 +654,8 @@ struct PickArgs {
 };
 
 // sum_j fl(term2 + qtab), the reference's four accumulators over j mod 4.  M subspaces of D dims
-// compiled in (M 0: both at run time), one or two code words a turn, at most 128 floats of centroids
-// in flight (unrolled whole it spills at six waves a SIMD).  4,000 queries, 32 of 512 lists of
+// compiled in (M 0: both at run time), one or two code words a turn, at most 128 floats of
+// centroids in flight (unrolled whole it spills at six waves a SIMD).  4,000 queries, 32 of 512 lists of
 // 200,000 rows, scores returned, against the run-time loop: m 16 x 4 dims 181 -> 151 us, 8 x 16
 // 166 -> 121, 8 x 8 123 -> 105, 4 x 32 141 -> 117, 4 x 8 79 -> 73.
 template <int M, int D>

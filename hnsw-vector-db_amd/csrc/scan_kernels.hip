@@ -2291,8 +2291,7 @@ int ScoreScan(Ctx* c, const ScanSource& src, const float* Q, size_t nq, size_t k
 // distance lies strictly below every unscored row's lower bound: the (n1+1)-th key, and each
 // full chunk's kp-th key (a row outside a chunk's list has a key at least that), taken back
 // to distances by -Qd + shift - eb.  Queries that are outside the int8 bounds or fail the
-// certificate go to the exact re-scan.  The last block publishes the fallback count to the
-// host (as ReadWords does), so the call makes no other launch.
+// certificate go to the exact re-scan (SmallFallback).
 
 constexpr int kTinyQ = 2;       // queries
 constexpr int kTinyK = 48;      // k (kp = k + 16 <= 64 keys per chunk)
@@ -3394,8 +3393,8 @@ static int TinyScan(Ctx* c, ScanSource* src, const float* Q, size_t nq, size_t k
     k_tiny_merge<true><<<dim3(unsigned(nq)), kMergeWaves * 64 + 64, 0, s>>>(ma);
     VDBG_HIP(hipGetLastError());
   }
-  const ScanPrune prune{part, bound, size_t(nchunks), kp, nchunks, small ? chunk * kSmallWaves : chunk,
-                        shift, eb, Qd, fit8q, out_d, int(kk)};
+  const ScanPrune prune{part,  bound, size_t(nchunks), kp,    nchunks,
+                        small ? chunk * kSmallWaves : chunk, shift, eb, Qd, fit8q, out_d, int(kk)};
   return SmallFallback(c, *src, Q, nq, kk, allow, out_ids, out_d, s, W2, fb_list, fb_count, gated,
                        prune);
 }

@@ -684,7 +684,8 @@ inline int StageRegions(Ctx* c, const float* queries, size_t qb, const void* ext
   uint8_t* base = nullptr;
   uint32_t uncertified[4] = {};  // (sent out behind the results)
   VDBG_RETURN_IF_ERROR(StageIn(c, src, bytes, extra ? 2 : 1,
-                               2 * StageRound(ob) + StageRound(cb) + StageRound(sizeof(uncertified)),
+                               2 * StageRound(ob) + StageRound(cb) +
+                                   StageRound(sizeof(uncertified)),
                                s, &base));
   const size_t in_end = StageSpan(qb) + (extra ? StageSpan(eb) : 0);
   const float* dq = reinterpret_cast<const float*>(base);

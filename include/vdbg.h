@@ -124,7 +124,8 @@ int vdbg_ctx_set_int8_float_min_work(vdbg_ctx* ctx, double work);
  * fl(term2 + qtab) is built per query and every code scored on it.  Indexes of up to 128 padded
  * dims with 4, 8 or 16 bytes a code also keep their decoded residuals as fp16 (2 x padded dim
  * bytes a row, where that is at most a quarter of the free memory), which large batches rank on
- * list by list while it is on.  Results are identical either way.  No counterpart in the reference. */
+ * list by list while it is on.  Results are identical either way.  No counterpart in the
+ * reference. */
 int vdbg_ctx_set_ivf_row_sums(vdbg_ctx* ctx, int enable);
 
 /* Host threads for the CPU side of a search (the HNSW walk); n <= 0 restores the default:
