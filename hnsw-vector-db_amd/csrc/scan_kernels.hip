@@ -1666,7 +1666,7 @@ struct ScanArgs {
   uint2* part;            // [slot][split][64*E]
   uint32_t* part_counts;  // [slot][split]
   const uint32_t* nslots_dev;  // nullable: slots at or past *nslots_dev are not scanned
-  ScanPrune prune;        // keys null: every split is scanned
+  ScanPrune prune;        // of a PRUNE pass
 };
 
 // Grid of a gated exact re-scan pass (two blocks per CU of a 256-CU part).
@@ -1678,7 +1678,9 @@ constexpr size_t kGatedScanBlocks = 512;
 // but run for the few the pass before listed) and the blocks stride over the items the
 // device count allows, so a pass with nothing to do costs a small grid, not one block per
 // item.
-template <int E, class Scorer>
+// PRUNE: the splits are the chunks of the scan whose answers were not certified (a variant of its
+// own: the test's registers would cost the plain scan two of its seven waves a SIMD).
+template <int E, class Scorer, bool PRUNE>
 __device__ __forceinline__ void exact_scan_item(const ScanArgs& a, const Scorer& sc, int slot,
                                                 int split, float (*md)[kWave * E],
                                                 uint32_t (*mi)[kWave * E]) {
@@ -1691,11 +1693,10 @@ __device__ __forceinline__ void exact_scan_item(const ScanArgs& a, const Scorer&
   WaveTopK<E> top;
   top.init();
   bool listed = false;
-  if (a.prune.keys != nullptr) {
-    // The split is a chunk of the scan whose answer was not certified.  A key above the k-th
-    // distance found by more than its error (the merge's certificate) keeps its row out of the
-    // answer: the chunk is left out when its smallest key does, and only its listed rows below
-    // that are scored when its bound does.
+  if constexpr (PRUNE) {
+    // A key above the k-th distance found by more than its error (the merge's certificate) keeps
+    // its row out of the answer: the chunk is left out when its smallest key does, and only its
+    // listed rows below that are scored when its bound does.
     const ScanPrune& p = a.prune;
     const size_t at = size_t(q) * p.stride + split;
     const uint2* keys = p.keys + at * p.kp;
@@ -1766,18 +1767,18 @@ __device__ __forceinline__ void exact_scan_item(const ScanArgs& a, const Scorer&
   if (lane == 0) a.part_counts[ps] = valid;
 }
 
-template <int E, class Scorer, bool GATED>
+template <int E, class Scorer, bool GATED, bool PRUNE = false>
 __global__ __launch_bounds__(256) void k_exact_scan(ScanArgs a, Scorer sc) {
   __shared__ float md[3][kWave * E];
   __shared__ uint32_t mi[3][kWave * E];
   if constexpr (!GATED) {  // one item per block: (slot, split) = (blockIdx.x, blockIdx.y)
-    exact_scan_item<E, Scorer>(a, sc, int(blockIdx.x), int(blockIdx.y), md, mi);
+    exact_scan_item<E, Scorer, PRUNE>(a, sc, int(blockIdx.x), int(blockIdx.y), md, mi);
   } else {
     const uint32_t nslots = min(*a.nslots_dev, uint32_t(a.nslots));
     const uint32_t items = nslots * uint32_t(a.nsplit);
     for (uint32_t item = blockIdx.x; item < items; item += gridDim.x) {
-      exact_scan_item<E, Scorer>(a, sc, int(item / uint32_t(a.nsplit)),
-                                 int(item % uint32_t(a.nsplit)), md, mi);
+      exact_scan_item<E, Scorer, PRUNE>(a, sc, int(item / uint32_t(a.nsplit)),
+                                        int(item % uint32_t(a.nsplit)), md, mi);
       __syncthreads();  // wave 0 has read md / mi before the next item writes them
     }
   }
@@ -1987,14 +1988,14 @@ static void launch_select(hipStream_t s, const SelectArgs& a, const Scorer& sc) 
   else
     k_select<E, Scorer, 1><<<dim3((a.nslots + 3) / 4), 256, 0, s>>>(a, sc);
 }
-template <int E, class Scorer>
+template <int E, class Scorer, bool PRUNE = false>
 static void launch_scan(hipStream_t s, const ScanArgs& a, const Scorer& sc) {
   if (a.nslots_dev == nullptr) {
-    k_exact_scan<E, Scorer, false><<<dim3(a.nslots, a.nsplit), 256, 0, s>>>(a, sc);
+    k_exact_scan<E, Scorer, false, PRUNE><<<dim3(a.nslots, a.nsplit), 256, 0, s>>>(a, sc);
   } else {  // a gated pass: a bounded grid striding over the items the device count allows
     const size_t items = size_t(a.nslots) * size_t(a.nsplit);
     const unsigned blocks = unsigned(std::max<size_t>(1, std::min<size_t>(items, kGatedScanBlocks)));
-    k_exact_scan<E, Scorer, true><<<dim3(blocks), 256, 0, s>>>(a, sc);
+    k_exact_scan<E, Scorer, true, PRUNE><<<dim3(blocks), 256, 0, s>>>(a, sc);
   }
 }
 template <int V>
@@ -2142,7 +2143,16 @@ static int ExactScanT(Ctx* c, Workspace& w, const ScanSource& src, const Scorer&
               prune != nullptr ? *prune : ScanPrune{}};
   {
     ProfScope ps(c, "exact_scan", s);
-    VDBG_DISPATCH_ES(E, launch_scan, Scorer, s, sa, sc);
+    if constexpr (std::is_same<Scorer, FlatScorer>::value) {
+      if (prune != nullptr) {  // (k <= kTinyK: one wavefront's list)
+        if (E != 1) return SetError(kInternal, "exact scan: pruned beyond k 64");
+        launch_scan<1, FlatScorer, true>(s, sa, sc);
+      } else {
+        VDBG_DISPATCH_ES(E, launch_scan, Scorer, s, sa, sc);
+      }
+    } else {
+      VDBG_DISPATCH_ES(E, launch_scan, Scorer, s, sa, sc);
+    }
     VDBG_HIP(hipGetLastError());
   }
   SelectArgs se{};

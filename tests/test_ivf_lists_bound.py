@@ -129,8 +129,8 @@ class Case:
         prod = half(q, sc, flush).astype(D) * half(r, e, flush).astype(D)
         order = ("in turn", "pairs", "blocks", "shuffled")[seed % 4]
         dot = sums(prod, order, rng)
-        v = (np.ldexp(D(-2), -sc - e) * dot.astype(D) + rowsum.astype(D)).astype(F)
-        self.value = (offset + v).astype(F)
+        self.v = (np.ldexp(D(-2), -sc - e) * dot.astype(D) + rowsum.astype(D)).astype(F)
+        self.value = (offset + self.v).astype(F)
 
 
 SHAPES = [(16, 8), (4, 32), (8, 2), (16, 3)]
@@ -165,9 +165,9 @@ def test_bounds_and_threshold():
             # any R rows' R-th smallest value bounds the rest: all rows (the tightest), the first
             for a in (np.sort(c.value)[R - 1], np.sort(c.value[:500])[R - 1]):
                 T = F(a + F(2) * c.eb)
-                # (the kernel compares value - offset with T - offset, widened as here)
+                # (the kernel compares v, value without the offset, with T - offset, widened so)
                 Td = F(F(T - c.offset) + F(2.0 ** -20) * F(abs(T) + abs(c.offset)))
-                assert ((c.value[top] - c.offset).astype(F) <= Td).all()
+                assert (c.v[top] <= Td).all()
             short += int((c.value[top] > np.sort(c.value)[R - 1]).any())
     assert short > 0  # the data needs the margin: without it rows of the top R are lost
 
