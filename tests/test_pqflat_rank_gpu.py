@@ -120,7 +120,11 @@ def test_decoded_rows_leave_memory_to_others(ctx):
         fill = []
         while left is not None and torch.cuda.mem_get_info()[0] > left and len(fill) < 4:
             over = torch.cuda.mem_get_info()[0] - left  # (large allocations are rounded)
-            fill.append(torch.empty(over, dtype=torch.uint8, device="cuda"))
+            try:
+                fill.append(torch.empty(over, dtype=torch.uint8, device="cuda"))
+            except torch.cuda.OutOfMemoryError:
+                ds.close()
+                pytest.skip("the free memory cannot be taken in one piece")
         ix = vdbg.PqFlatIndex.build(ds, 16, max_points=4, iters=1)
         del fill
         torch.cuda.empty_cache()
